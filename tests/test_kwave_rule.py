@@ -1,0 +1,83 @@
+"""The rule that puts a launch on the tiles whose K the waves share
+(kernels::kwave_plan_shape and launch_bytes_wanted, through the hostsim
+library): over seeded shapes of every form a plan's ranges cover K in multiples
+of 32, its tile is one the form has, no chain of a sum is longer than the ranges
+of the split rule nor than 1024 (up to the tile's fold granularity), a launch
+given exactly the partials its plan wants takes the same plan and one byte less
+another that fits, and the partials of any launch fit the allocation-free
+entry's 128 MiB."""
+import ctypes
+
+import numpy as np
+
+import xvram_amd as xv
+
+ANY = (1 << 64) - 1
+RUN = (64, 48, 32, 32, 128, 0)
+
+
+def fns():
+    dll = xv.load(hostsim=True).dll
+    i64, pint = ctypes.c_int64, ctypes.POINTER(ctypes.c_int)
+    dll.xvram_hostsim_kwave_plan.argtypes = [i64] * 3 + [ctypes.c_int, ctypes.c_uint64] + [pint] * 3
+    dll.xvram_hostsim_split_shape.argtypes = [i64] * 3 + [ctypes.c_int] * 2 + [ctypes.c_uint64, pint, pint]
+    dll.xvram_hostsim_launch_bytes_wanted.argtypes = [ctypes.c_int] * 5 + [i64] * 2
+    dll.xvram_hostsim_launch_bytes_wanted.restype = ctypes.c_uint64
+    return dll
+
+
+def test_plan_properties():
+    dll = fns()
+
+    def plan(m, n, k, nt, ws=ANY):
+        s, d, f = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+        t = dll.xvram_hostsim_kwave_plan(m, n, k, nt, ws, ctypes.byref(s), ctypes.byref(d), ctypes.byref(f))
+        return t, s.value, d.value, f.value
+
+    rng = np.random.default_rng(41)
+    tiles, split = set(), 0
+    for _ in range(4000):
+        m, n = (int(2 ** v) for v in rng.uniform(0, 13, 2))
+        k = int(2 ** rng.uniform(0, 16))
+        nt = int(rng.integers(0, 2))
+        tile, s, depth, fold = plan(m, n, k, nt)
+        fits = k >= 8 and -(-m // 256) * -(-n // 256) < 256
+        old = ctypes.c_int(), ctypes.c_int()
+        olds = dll.xvram_hostsim_split_shape(m, n, k, nt, 1, ANY, ctypes.byref(old[0]), ctypes.byref(old[1]))
+        if tile < 0:
+            ring = olds > 1 and not old[1].value and old[0].value >= 4096
+            assert not fits or ring
+            continue
+        tiles.add((tile, nt))
+        assert fits and (tile != 5 or nt)
+        assert (s == 1 and depth == k) or (depth % 32 == 0 and (s - 1) * depth < k <= s * depth)
+        chain = min(old[0].value if olds > 1 else k, 1024)
+        if (depth + 3) // 4 > chain:
+            assert fold % RUN[tile] == 0 and RUN[tile] <= fold <= max(chain, RUN[tile])
+        partial = (m + 3) // 4 * 4 * n * 4
+        if s > 1:
+            split += 1
+            assert s * partial <= 64 << 20
+            assert plan(m, n, k, nt, s * partial) == (tile, s, depth, fold)
+            less = plan(m, n, k, nt, s * partial - 1)
+            assert less[1] == 1 or less[1] * partial < s * partial
+        assert plan(m, n, k, nt, 0)[1] == 1
+    assert tiles >= {(t, nt) for t in range(5) for nt in (0, 1)} | {(5, 1)} and split > 500
+
+
+def test_partials_fit_the_scratch():
+    dll = fns()
+    rng = np.random.default_rng(43)
+    split = 0
+    for _ in range(8000):
+        scale = int(rng.choice([512, 4096, 16384]))
+        m, n = (int(v) for v in rng.integers(1, scale + 1, 2))
+        k = int(rng.integers(1, 3 * scale))
+        if rng.random() < 0.5:
+            m, n = 256 * max(1, m // 256), 256 * max(1, n // 256)
+        ak, bn = (int(v) for v in rng.integers(0, 2, 2))
+        lda, ldb = ((k if ak else m) + 3) // 4 * 4, ((n if bn else k) + 3) // 4 * 4
+        wanted = dll.xvram_hostsim_launch_bytes_wanted(m, n, k, ak, bn, lda, ldb)
+        split += wanted > 0
+        assert wanted <= 128 << 20, (m, n, k, ak, bn)
+    assert split > 300

@@ -611,6 +611,36 @@ extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_bytes_w
   return xvram::kernels::split_k_bytes_wanted(l);
 }
 
+// The same as the GPU's launch_sgemm runs the launch
+// (kernels::launch_bytes_wanted).
+extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_launch_bytes_wanted(
+    int m, int n, int k, int a_kcontig, int b_ncontig, int64_t lda, int64_t ldb) {
+  xvram::kernels::SgemmLaunch l;
+  l.m = m;
+  l.n = n;
+  l.k = k;
+  l.a_kcontig = a_kcontig != 0;
+  l.b_ncontig = b_ncontig != 0;
+  l.lda = lda;
+  l.ldb = ldb;
+  l.ldc = m;
+  return xvram::kernels::launch_bytes_wanted(l);
+}
+
+// The tiles whose K the waves share (kernels::kwave_plan_shape): returns the
+// tile's index (-1: the launch runs elsewhere), *splits K ranges of *depth and
+// *fold k values between folds.
+extern "C" __attribute__((visibility("default"))) int xvram_hostsim_kwave_plan(
+    int64_t m, int64_t n, int64_t k, int nt, uint64_t workspace_bytes, int* splits, int* depth,
+    int* fold) {
+  const xvram::kernels::KwavePlan p =
+      xvram::kernels::kwave_plan_shape(m, n, k, nt != 0, workspace_bytes);
+  if (splits != nullptr) *splits = p.splits;
+  if (depth != nullptr) *depth = p.depth;
+  if (fold != nullptr) *fold = p.fold;
+  return p.tile;
+}
+
 // Launches that ran as an interior and edge strips since the last reset.
 extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_edge_split_launches() {
   using namespace xvram;

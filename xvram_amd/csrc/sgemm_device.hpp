@@ -1,6 +1,7 @@
 // sgemm_device.hpp — device-side pieces shared by the tile kernels
-// (sgemm_mfma.hip: 256 x 128 tiles, two workgroups per CU; sgemm_wide.hip:
-// two kernels of 256 x 256 tiles, one workgroup per CU). Compiled only by hipcc.
+// (sgemm_kwave.hip: tiles of 32 x 32 to 128 x 64 whose K the waves share;
+// sgemm_mfma.hip: 256 x 128 tiles, two workgroups per CU; sgemm_wide.hip:
+// kernels of 256 x 256 tiles, one workgroup per CU). Compiled only by hipcc.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -51,6 +52,30 @@ __device__ __forceinline__ float4 load4(const float* __restrict__ line, int firs
     if (left < 2) v.y = 0.f;
   }
   return v;
+}
+
+// Raw buffer descriptor (no stride, 32-bit data format word) over `bytes`
+// bytes from `base`; reads at or past `bytes` return zeros.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t panel_rsrc(const float* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, (int)bytes,
+                                           0x00020000);
+}
+
+// One wave-wide direct load: lane l's 16 bytes at rsrc.base + soff + voff land
+// at LDS byte address lds_base + kOff + 16*l (lds_base wave-uniform). Counted
+// by vmcnt only: the caller waits on vmcnt before the data is read (and, when
+// other waves read it, before the barrier that publishes it).
+template <int kOff>
+__device__ __forceinline__ void load_lds16(uint32_t lds_base, uint32_t voff,
+                                           __amdgpu_buffer_rsrc_t rsrc, uint32_t soff) {
+  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :: "s"(lds_base), "v"(voff), "s"(rsrc), "s"(soff), "i"(kOff)
+               : "memory", "m0", "scc");
+}
+
+__device__ __forceinline__ uint32_t lds_byte_addr(const float* p) {
+  return __builtin_amdgcn_readfirstlane(
+      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p);
 }
 
 // Linear workgroup id -> (tile_m, tile_n): undo the round-robin XCD dispatch
@@ -211,6 +236,42 @@ __device__ __forceinline__ void store_c_interior(const Params& p, const float16_
         *reinterpret_cast<float4*>(cline + row_of(v)) = r;
       }
     }
+  }
+}
+
+// C(row .. row+3, col) from the sums of four consecutive rows (row a multiple
+// of 4 below m): alpha, beta, biases and ReLU in store_c_tile's arithmetic and
+// order; only rows inside C are touched.
+__device__ __forceinline__ void store_quad(const Params& p, const float4& sum, int row, int col) {
+  float* cp = p.c + (int64_t)col * p.ldc + row;
+  const bool extra = p.bias_row != nullptr || p.bias_col != nullptr || p.relu != 0;
+  const float bias_c = p.bias_col != nullptr ? p.bias_col[col] : 0.f;
+  const auto finish = [&](float v, int r) {
+    if (p.bias_row != nullptr) v += p.bias_row[r];
+    v += bias_c;
+    return (p.relu != 0 && v < 0.f) ? 0.f : v;
+  };
+  if (row + 4 <= p.m) {
+    float r[4] = {p.alpha * sum.x, p.alpha * sum.y, p.alpha * sum.z, p.alpha * sum.w};
+    if (p.beta != 0.f) {
+      const float4 old = *reinterpret_cast<const float4*>(cp);
+      r[0] = p.alpha * sum.x + p.beta * old.x;
+      r[1] = p.alpha * sum.y + p.beta * old.y;
+      r[2] = p.alpha * sum.z + p.beta * old.z;
+      r[3] = p.alpha * sum.w + p.beta * old.w;
+    }
+    if (extra) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) r[t] = finish(r[t], row + t);
+    }
+    *reinterpret_cast<float4*>(cp) = make_float4(r[0], r[1], r[2], r[3]);
+    return;
+  }
+  const float v[4] = {sum.x, sum.y, sum.z, sum.w};
+  for (int t = 0; t < 4 && row + t < p.m; ++t) {
+    const float val = p.alpha * v[t];
+    const float out = p.beta != 0.f ? val + p.beta * cp[t] : val;
+    cp[t] = extra ? finish(out, row + t) : out;
   }
 }
 

@@ -62,11 +62,14 @@ int scratch_address(hipStream_t stream, void** out) {
 int direct_sgemm_no_alloc(const kernels::SgemmLaunch& launch, void* stream) {
   kernels::SgemmLaunch l = launch;
   l.padded = true;
-  const uint64_t wanted = kernels::split_k_bytes_wanted(l);
+  const uint64_t wanted = kernels::launch_bytes_wanted(l);
+  // Looked up on the first call on a GPU whether or not it splits: the array
+  // becomes resident with its code object then, and no later call takes memory.
+  void* p = nullptr;
+  const int found = scratch_address(static_cast<hipStream_t>(stream), &p);
   if (wanted > 0 && (l.workspace == nullptr || l.workspace_bytes < wanted)) {
     if (wanted > kScratchBytes) return kScratchTooSmall;
-    void* p = nullptr;
-    if (const int rc = scratch_address(static_cast<hipStream_t>(stream), &p)) return rc;
+    if (found != 0) return found;
     l.workspace = static_cast<float*>(p);
     l.workspace_bytes = kScratchBytes;
   }
@@ -80,7 +83,7 @@ int direct_sgemm(const kernels::SgemmLaunch& launch, void* stream) {
   // The split this launch wants with room for all of its partials; the
   // caller's workspace serves when it holds them, else a stream-ordered one
   // (the same split either way, so the same result).
-  const uint64_t wanted = kernels::split_k_bytes_wanted(l);
+  const uint64_t wanted = kernels::launch_bytes_wanted(l);
   void* own = nullptr;
   if (wanted > 0 && (l.workspace == nullptr || l.workspace_bytes < wanted)) {
     if (const hipError_t e = hipMallocAsync(&own, wanted, s); e != hipSuccess) {

@@ -21,6 +21,12 @@
 // spanning less than 2^31 bytes from its base (two_panel_valid below);
 // anything else returns hipErrorInvalidValue.
 //
+// Fewer than 256 tiles of 256 x 256: smaller tiles whose K the waves of a
+// workgroup share (kwave_plan_shape below), K split over workgroups too where
+// that is faster and a workspace is set. What follows is for the launches that
+// rule leaves: panels of 2^31 bytes and more (256 x 128 kernel) and deep
+// interior ranges (ring kernels).
+//
 // Split K (optional, workspace set): a launch that would leave CUs idle may
 // cut its K into ranges (split_k_plan below), one workgroup per tile and
 // range; each stores the raw partial sums of its range to the workspace
@@ -202,6 +208,122 @@ inline SplitK split_k_plan(const SgemmLaunch& l) {
 // C), not the MFMA tiles: a K remainder's last 1-7 rows, or any such launch.
 constexpr int kThinK = 8;
 
+// Tiles whose K the waves share (sgemm_kwave.hip). A one-panel launch of K >= 8
+// with fewer than kComputeUnits tiles of 256 x 256 runs on one of these,
+// unsplit or with its K split over workgroups, whichever combination the model
+// below rates fastest; except interior launches whose ring split fills at
+// least 15/16 of the CUs with ranges at least 4096 deep, which stay on the
+// ring kernels (16384 x 256 x 16384 T/N, 4 x 4096 deep: 995 against 1030 us;
+// with 2048-deep ranges the two are level or these ahead: 4096 x 2048 x 4096 T/N
+// 497 against 490, 2048 x 1024 x 16384 N/N 488 against 490).
+//
+// The model, in us: workgroups run in rounds of per_cu on each CU; one takes
+// (depth + fixed) x `shared` when its CU is full and x `alone` when the last
+// round leaves it the CU; the operands take their bytes over 7.85 TB/s, and the
+// shorter of the two adds 0.56 of itself to the longer; C costs 0.14 us per
+// million elements, a launch 2 us, a split 3.1 us and 0.92 us per million
+// partial elements. Fitted to 165 shapes (squares of 64 to 5500, boxes up to
+// 8192, linear layers of 1 to 1024 columns up to 16384 x 16384, their input and
+// weight gradients, Gram matrices up to K = 65536), each on every tile with one
+// to 32 ranges: the rule's choice ran 2.9 % slower than the fastest measured
+// one on average (25 % at worst) and faster than the launch before on all.
+struct KwaveTile {
+  int mb, nb;    // 32 x 32 blocks of rows and of columns
+  int per_cu;    // workgroups a CU holds
+  int run;       // a fold's k values are a multiple of this; 0 = cannot fold
+  double alone, shared, fixed;
+};
+inline constexpr KwaveTile kKwaveTiles[] = {
+    {1, 1, 2, 64, 0.00493, 0.00949, 213}, {2, 1, 2, 48, 0.00829, 0.0159, 187},
+    {2, 2, 2, 32, 0.01436, 0.02617, 189}, {4, 1, 2, 32, 0.01428, 0.02855, 194},
+    {1, 1, 1, 128, 0.00403, 0.00403, 621}, // slots of 32 k values, deep rings
+    {4, 2, 2, 0, 0.03087, 0.05406, 131},   // N/T only
+};
+constexpr int kKwaveTileCount = 6;
+constexpr int kKwaveNtTile = 5, kKwaveSkinnyTile = 3;
+constexpr uint64_t kKwaveMaxPartialBytes = uint64_t{64} << 20;
+
+struct KwavePlan {
+  int tile = -1;  // index in kKwaveTiles; -1 = not on these
+  int splits = 1; // K ranges over workgroups
+  int depth = 0;  // K per range
+  int fold = 0;   // k values of one wave between folds of its accumulators
+};
+
+// The plan of an m x n x k launch of form `nt` or not, whose operand panels the
+// kernels can address (each spans less than 2^31 bytes), given room for
+// `workspace_bytes` of partials. The chains of a sum are no longer than the
+// ranges of the split that split_k_shape takes for the launch (nor than 1024:
+// a fold that rare costs nothing measurable).
+inline KwavePlan kwave_plan_shape(int64_t m, int64_t n, int64_t k, bool nt,
+                                  uint64_t workspace_bytes) {
+  KwavePlan best;
+  if (m <= 0 || n <= 0 || k < kThinK) return best;
+  if (((m + 255) / 256) * ((n + 255) / 256) >= kComputeUnits) return best;
+  const SplitK old = split_k_shape(m, n, k, nt, true, ~uint64_t{0});
+  if (old.splits > 1 && !old.narrow && old.depth >= 4096 &&
+      16 * (m / 256) * (n / 256) * old.splits >= 15 * kComputeUnits)
+    return best;
+  const int64_t chain = std::min<int64_t>(old.splits > 1 ? old.depth : k, 1024);
+  const double elements = 1e-6 * double(m) * double(n);
+  const double memory = 4e-6 * (double(m) + double(n)) * double(k) / 7.85;
+  const int64_t partial = split_partial_ld(m) * n * 4;
+  double best_time = 0;
+  for (int i = 0; i < kKwaveTileCount; ++i) {
+    const KwaveTile& t = kKwaveTiles[i];
+    // The tiles each shape was measured on: 128 x 64 for N/T, 128 x 32 up to
+    // 128 columns (twice the operand traffic of 64 x 64 beyond), one column
+    // block up to 32 columns.
+    if ((i == kKwaveNtTile && !nt) || (i == kKwaveSkinnyTile && n > 128) || (t.nb > 1 && n <= 32))
+      continue;
+    const int64_t tiles = ((m + 32 * t.mb - 1) / (32 * t.mb)) * ((n + 32 * t.nb - 1) / (32 * t.nb));
+    for (const int s : {1, 2, 3, 4, 5, 6, 8, 11, 16, 24, 32}) {
+      SplitK sk;
+      sk.depth = static_cast<int>(k);
+      if (s > 1) {
+        if (tiles * s > 12 * kComputeUnits || k < 128 * s ||
+            uint64_t(s) * uint64_t(partial) > std::min(workspace_bytes, kKwaveMaxPartialBytes))
+          break;
+        sk = split_ranges(k, s, false);
+        if (sk.splits != s) continue;
+      }
+      const bool folds = (sk.depth + 3) / 4 > chain;
+      if (folds && t.run == 0) continue;
+      const int64_t groups = tiles * s, slots = t.per_cu * kComputeUnits;
+      const int64_t full = (groups - 1) / slots, last = groups - full * slots;
+      const double compute = (sk.depth + t.fixed) *
+                             (t.shared * double(full) + (last > kComputeUnits ? t.shared : t.alone));
+      const double time = 2.0 + std::max(compute, memory) + 0.56 * std::min(compute, memory) +
+                          0.14 * elements + (s > 1 ? 3.1 + 0.92 * s * elements : 0.0);
+      if (best.tile < 0 || time < best_time) {
+        best_time = time;
+        best.tile = i;
+        best.splits = s;
+        best.depth = sk.depth;
+        best.fold = folds ? static_cast<int>(std::max<int64_t>(t.run, chain / t.run * t.run))
+                          : (t.run > 0 ? (1 << 28) / t.run * t.run : 0);
+      }
+    }
+  }
+  return best;
+}
+
+// The plan a launch takes given room for `workspace_bytes` of partials.
+inline KwavePlan kwave_plan_for(const SgemmLaunch& l, uint64_t workspace_bytes) {
+  constexpr int64_t kLimit = int64_t(1) << 31;
+  if (l.a2 != nullptr || l.b2 != nullptr) return {};
+  const int64_t a_bytes = (l.a_kcontig ? int64_t{l.m} : int64_t{l.k}) * l.lda * 4;
+  const int64_t b_bytes = (l.b_ncontig ? int64_t{l.k} : int64_t{l.n}) * l.ldb * 4;
+  if (a_bytes >= kLimit || b_bytes >= kLimit) return {};
+  return kwave_plan_shape(l.m, l.n, l.k, !l.a_kcontig && l.b_ncontig, workspace_bytes);
+}
+
+// The plan of one launch with its own 16-byte aligned workspace (or none).
+inline KwavePlan kwave_plan(const SgemmLaunch& l) {
+  const bool usable = l.workspace != nullptr && reinterpret_cast<uintptr_t>(l.workspace) % 16 == 0;
+  return kwave_plan_for(l, usable ? l.workspace_bytes : 0);
+}
+
 // Tail split. A launch of at least kComputeUnits interior 256 x 256 tiles
 // runs in rounds of one workgroup per CU, and a last round that fills few
 // CUs costs as much as a full one (17 x 17 tiles: 2 rounds for 289 tiles).
@@ -290,6 +412,15 @@ inline uint64_t split_k_bytes_wanted_whole(const SgemmLaunch& l) {
                        : 0;
 }
 
+// The same as launch_sgemm runs a launch without parts.
+inline uint64_t part_bytes_wanted(const SgemmLaunch& l) {
+  const KwavePlan kw = kwave_plan_for(l, ~uint64_t{0});
+  if (kw.tile < 0) return split_k_bytes_wanted_whole(l);
+  return kw.splits > 1
+             ? uint64_t(kw.splits) * uint64_t(split_partial_ld(l.m)) * uint64_t(l.n) * 4
+             : 0;
+}
+
 // Edge split. A launch whose m or n is not a multiple of 256 and that has at
 // least kComputeUnits tiles of 256 x 256 runs every tile on the ring kernels'
 // edge instances (K a multiple of 4 for N/T, of 8 for the other forms), whose
@@ -375,7 +506,7 @@ inline EdgeParts edge_parts(const SgemmLaunch& l) {
   const EdgeParts e = edge_parts_shape(l);
   if (e.count == 0 || l.workspace != nullptr) return e;
   for (int i = 0; i < e.count; ++i)
-    if (split_k_bytes_wanted_whole(e.part[i]) > 0) return {};
+    if (part_bytes_wanted(e.part[i]) > 0) return {};
   return e;
 }
 
@@ -462,11 +593,24 @@ inline uint64_t split_k_bytes_wanted(const SgemmLaunch& l) {
   return most;
 }
 
+// Bytes of partials one launch wants when the workspace is not the limit, as
+// launch_sgemm runs it: its own, or the most that any part of its K remainder
+// or edge split wants (they share the workspace in turn).
+inline uint64_t launch_bytes_wanted(const SgemmLaunch& l) {
+  const KParts kp = k_remainder_parts_shape(l);
+  const SgemmLaunch& base = kp.count > 0 ? kp.part[0] : l;
+  const EdgeParts e = edge_parts_shape(base);
+  if (e.count == 0) return part_bytes_wanted(base);
+  uint64_t most = 0;
+  for (int i = 0; i < e.count; ++i) most = std::max(most, part_bytes_wanted(e.part[i]));
+  return most;
+}
+
 // The two launches of a K remainder (count 0: none): by shape, and without a
 // workspace only when the first part would not split.
 inline KParts k_remainder_parts(const SgemmLaunch& l) {
   const KParts kp = k_remainder_parts_shape(l);
-  if (kp.count == 0 || l.workspace != nullptr || split_k_bytes_wanted(kp.part[0]) == 0) return kp;
+  if (kp.count == 0 || l.workspace != nullptr || launch_bytes_wanted(kp.part[0]) == 0) return kp;
   return {};
 }
 

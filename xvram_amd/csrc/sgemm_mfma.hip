@@ -58,6 +58,8 @@ int wide_tile();
 hipError_t launch_wide(const device::Params& p, bool a_kcontig, bool b_ncontig,
                        hipStream_t stream, hipEvent_t start, hipEvent_t stop);
 hipError_t launch_splitk_reduce(const device::Params& p, hipStream_t stream, hipEvent_t stop);
+hipError_t launch_kwave(const device::Params& p, const KwavePlan& plan, bool a_kcontig,
+                        bool b_ncontig, hipStream_t stream, hipEvent_t start, hipEvent_t stop);
 hipError_t launch_thin_k(const device::Params& p, bool a_kcontig, bool b_ncontig,
                          hipStream_t stream, hipEvent_t start, hipEvent_t stop);
 
@@ -365,6 +367,12 @@ int launch_sgemm(const SgemmLaunch& launch, void* stream) {
   // K below 8: no MFMA tiles (sgemm_wide.hip, thin_k_kernel).
   if (launch.k < kThinK)
     return static_cast<int>(launch_thin_k(p, launch.a_kcontig, launch.b_ncontig, s, e0, e1));
+  // Fewer 256 x 256 tiles than CUs: smaller tiles whose K the waves share
+  // (sgemm_launch.hpp, kwave_plan_shape).
+  if (const KwavePlan kw = kwave_plan(launch); kw.tile >= 0) {
+    p.partial = launch.workspace;
+    return static_cast<int>(launch_kwave(p, kw, launch.a_kcontig, launch.b_ncontig, s, e0, e1));
+  }
   // Fewer tiles than workgroup slots: split K when a workspace is given
   // (fixed-order reduction; sgemm_launch.hpp), on the ring kernels for
   // interior 256 x 256 tiles, else on the 256 x 128 kernel.

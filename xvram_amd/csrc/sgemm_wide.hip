@@ -122,33 +122,9 @@ __device__ __forceinline__ void store_half(float* __restrict__ l, int tid, const
   }
 }
 
-// Raw buffer descriptor (no stride, 32-bit data format word) over `bytes`
-// bytes from `base`; reads at or past `bytes` return zeros.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t panel_rsrc(const float* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, (int)bytes,
-                                           0x00020000);
-}
-
-// One wave-wide direct load: lane l's 16 bytes at rsrc.base + soff + voff land
-// at LDS byte address lds_base + kOff + 16*l (lds_base wave-uniform). Counted
-// by vmcnt only: the caller waits on vmcnt before the data is read (and, when
-// other waves read it, before the barrier that publishes it).
-template <int kOff>
-__device__ __forceinline__ void load_lds16(uint32_t lds_base, uint32_t voff,
-                                           __amdgpu_buffer_rsrc_t rsrc, uint32_t soff) {
-  asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :: "s"(lds_base), "v"(voff), "s"(rsrc), "s"(soff), "i"(kOff)
-               : "memory", "m0", "scc");
-}
-
 __device__ __forceinline__ float4 load_reg16(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff,
                                              uint32_t soff) {
   return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, soff, 0));
-}
-
-__device__ __forceinline__ uint32_t lds_byte_addr(const float* p) {
-  return __builtin_amdgcn_readfirstlane(
-      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p);
 }
 
 template <bool AK, bool BN>
@@ -902,36 +878,7 @@ __global__ __launch_bounds__(kThreads) void splitk_reduce_kernel(Params p) {
     sum.z += v.z;
     sum.w += v.w;
   }
-  float* cp = p.c + (int64_t)col * p.ldc + row;
-  const bool extra = p.bias_row != nullptr || p.bias_col != nullptr || p.relu != 0;
-  const float bias_c = p.bias_col != nullptr ? p.bias_col[col] : 0.f;
-  const auto finish = [&](float v, int r) {
-    if (p.bias_row != nullptr) v += p.bias_row[r];
-    v += bias_c;
-    return (p.relu != 0 && v < 0.f) ? 0.f : v;
-  };
-  if (row + 4 <= p.m) {
-    float r[4] = {p.alpha * sum.x, p.alpha * sum.y, p.alpha * sum.z, p.alpha * sum.w};
-    if (p.beta != 0.f) {
-      const float4 old = *reinterpret_cast<const float4*>(cp);
-      r[0] = p.alpha * sum.x + p.beta * old.x;
-      r[1] = p.alpha * sum.y + p.beta * old.y;
-      r[2] = p.alpha * sum.z + p.beta * old.z;
-      r[3] = p.alpha * sum.w + p.beta * old.w;
-    }
-    if (extra) {
-#pragma unroll
-      for (int t = 0; t < 4; ++t) r[t] = finish(r[t], row + t);
-    }
-    *reinterpret_cast<float4*>(cp) = make_float4(r[0], r[1], r[2], r[3]);
-    return;
-  }
-  const float v[4] = {sum.x, sum.y, sum.z, sum.w};
-  for (int t = 0; t < 4 && row + t < p.m; ++t) {
-    const float val = p.alpha * v[t];
-    const float out = p.beta != 0.f ? val + p.beta * cp[t] : val;
-    cp[t] = extra ? finish(out, row + t) : out;
-  }
+  store_quad(p, sum, row, col);
 }
 
 // A launch of K below 8 (a K remainder's last rows): too little work for the
