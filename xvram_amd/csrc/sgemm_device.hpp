@@ -172,11 +172,9 @@ __device__ __forceinline__ Params partial_target(const Params& p, int split) {
 // a launch would otherwise run at the same moment). Same arithmetic, in the
 // same order, as the general path. Row biases are loaded ahead only with
 // kRowBiasAhead (64 more registers: the 256 x 256 kernels have them, the
-// 256 x 128 kernel at two workgroups per CU does not). store_c_tile uses
-// batches of one column (two would make the kernels that also compile the
-// general path spill); kernels whose tiles are all interior call
-// store_c_interior directly.
-template <int kNJ, int kBatch, bool kRowBiasAhead>
+// 256 x 128 kernel at two workgroups per CU does not). One column of a lane per
+// batch: with two the kernels, which compile the general path as well, spill.
+template <int kNJ, bool kRowBiasAhead>
 __device__ __forceinline__ void store_c_interior(const Params& p, const float16_t (&acc)[4][kNJ],
                                                  int row0, int col0, int lrow, int lhalf) {
   const bool read_c = p.beta != 0.f;
@@ -194,54 +192,57 @@ __device__ __forceinline__ void store_c_interior(const Params& p, const float16_
     v += bias_c;
     return (p.relu != 0 && v < 0.f) ? 0.f : v;
   };
-  static_assert(kNJ % kBatch == 0, "columns come in whole batches");
 #pragma unroll
-  for (int j0 = 0; j0 < kNJ; j0 += kBatch) {
-    float4 old[kBatch][16];
-    float bias_c[kBatch];
+  for (int j = 0; j < kNJ; ++j) {
+    const int col = col0 + kNJ * lrow + j;
+    float* cline = p.c + (int64_t)col * p.ldc;
+    const float bias_c = p.bias_col != nullptr ? p.bias_col[col] : 0.f;
+    float4 old[16];
+    if (read_c) {
 #pragma unroll
-    for (int jb = 0; jb < kBatch; ++jb) {
-      const int col = col0 + kNJ * lrow + j0 + jb;
-      bias_c[jb] = p.bias_col != nullptr ? p.bias_col[col] : 0.f;
-      if (read_c) {
-        const float* cline = p.c + (int64_t)col * p.ldc;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) old[jb][v] = *reinterpret_cast<const float4*>(cline + row_of(v));
-      }
+      for (int v = 0; v < 16; ++v) old[v] = *reinterpret_cast<const float4*>(cline + row_of(v));
     }
 #pragma unroll
-    for (int jb = 0; jb < kBatch; ++jb) {
-      const int j = j0 + jb;
-      float* cline = p.c + (int64_t)(col0 + kNJ * lrow + j) * p.ldc;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        float4 r;
-        if (read_c) {
-          r.x = p.alpha * acc[0][j][v] + p.beta * old[jb][v].x;
-          r.y = p.alpha * acc[1][j][v] + p.beta * old[jb][v].y;
-          r.z = p.alpha * acc[2][j][v] + p.beta * old[jb][v].z;
-          r.w = p.alpha * acc[3][j][v] + p.beta * old[jb][v].w;
-        } else {
-          r.x = p.alpha * acc[0][j][v];
-          r.y = p.alpha * acc[1][j][v];
-          r.z = p.alpha * acc[2][j][v];
-          r.w = p.alpha * acc[3][j][v];
-        }
-        if (extra) {
-          r.x = finish(r.x, v, 0, bias_c[jb]);
-          r.y = finish(r.y, v, 1, bias_c[jb]);
-          r.z = finish(r.z, v, 2, bias_c[jb]);
-          r.w = finish(r.w, v, 3, bias_c[jb]);
-        }
-        *reinterpret_cast<float4*>(cline + row_of(v)) = r;
+    for (int v = 0; v < 16; ++v) {
+      float4 r;
+      if (read_c) {
+        r.x = p.alpha * acc[0][j][v] + p.beta * old[v].x;
+        r.y = p.alpha * acc[1][j][v] + p.beta * old[v].y;
+        r.z = p.alpha * acc[2][j][v] + p.beta * old[v].z;
+        r.w = p.alpha * acc[3][j][v] + p.beta * old[v].w;
+      } else {
+        r.x = p.alpha * acc[0][j][v];
+        r.y = p.alpha * acc[1][j][v];
+        r.z = p.alpha * acc[2][j][v];
+        r.w = p.alpha * acc[3][j][v];
       }
+      if (extra) {
+        r.x = finish(r.x, v, 0, bias_c);
+        r.y = finish(r.y, v, 1, bias_c);
+        r.z = finish(r.z, v, 2, bias_c);
+        r.w = finish(r.w, v, 3, bias_c);
+      }
+      *reinterpret_cast<float4*>(cline + row_of(v)) = r;
     }
   }
+}
+
+typedef float float4_t __attribute__((ext_vector_type(4)));
+
+// Four consecutive floats of C. kStream: past the L2 (a workgroup's C is not
+// read again by its launch, and what the L2 still holds dirty is written back
+// when the launch ends, with every CU idle).
+template <bool kStream>
+__device__ __forceinline__ void store4(float* dst, float x, float y, float z, float w) {
+  const float4_t v = {x, y, z, w};
+  if constexpr (kStream) __builtin_nontemporal_store(v, reinterpret_cast<float4_t*>(dst));
+  else *reinterpret_cast<float4_t*>(dst) = v;
 }
 
 // C(row .. row+3, col) from the sums of four consecutive rows (row a multiple
 // of 4 below m): alpha, beta, biases and ReLU in store_c_tile's arithmetic and
 // order; only rows inside C are touched.
+template <bool kStream>
 __device__ __forceinline__ void store_quad(const Params& p, const float4& sum, int row, int col) {
   float* cp = p.c + (int64_t)col * p.ldc + row;
   const bool extra = p.bias_row != nullptr || p.bias_col != nullptr || p.relu != 0;
@@ -264,7 +265,7 @@ __device__ __forceinline__ void store_quad(const Params& p, const float4& sum, i
 #pragma unroll
       for (int t = 0; t < 4; ++t) r[t] = finish(r[t], row + t);
     }
-    *reinterpret_cast<float4*>(cp) = make_float4(r[0], r[1], r[2], r[3]);
+    store4<kStream>(cp, r[0], r[1], r[2], r[3]);
     return;
   }
   const float v[4] = {sum.x, sum.y, sum.z, sum.w};
@@ -279,7 +280,7 @@ template <int kNJ, bool kRowBiasAhead>
 __device__ __forceinline__ void store_c_tile(const Params& p, const float16_t (&acc)[4][kNJ],
                                              int row0, int col0, int lrow, int lhalf) {
   if (row0 + 128 <= p.m && col0 + 32 * kNJ <= p.n) {
-    store_c_interior<kNJ, 1, kRowBiasAhead>(p, acc, row0, col0, lrow, lhalf);
+    store_c_interior<kNJ, kRowBiasAhead>(p, acc, row0, col0, lrow, lhalf);
     return;
   }
   const bool read_c = p.beta != 0.f;
@@ -330,6 +331,98 @@ __device__ __forceinline__ void store_c_tile(const Params& p, const float16_t (&
             const float val = p.alpha * out[t];
             const float sum = read_c ? val + p.beta * cline[row + t] : val;
             cline[row + t] = extra ? finish(sum, row + t, bias_c) : sum;
+          }
+        }
+      }
+    }
+  }
+}
+
+// The same for the ring kernels' waves (kNJ = 4), through 16 KiB of the wave's
+// own LDS: column block j of the accumulators (every fourth column) goes in as
+// the MFMAs left it and comes out with 32 lanes on 128 consecutive rows of a
+// column, so C is read and written in runs of 512 bytes instead of 16. Written
+// as 16-byte pieces of 64 columns at once, a 256-tile launch spent about 12 us
+// of its last round on its C (4096 x 4096 x 256 N/T: 80 us for 55 us of MFMAs, now 71; 8192 x 8192 x 128
+// 207 -> 165; 4096^3 920 -> 907; 8192^3 7227 -> 7180).
+// No other wave's LDS is touched and the LDS serves a wave in order, so there
+// is no barrier. A lane's four rows stay the same, and so does its row bias.
+template <bool kEdge, bool kStream>
+__device__ __forceinline__ void store_c_ring(const Params& p, const float16_t (&acc)[4][4], float* lds,
+                                             int row0, int col0, int lane) {
+  const int lrow = lane & 31, lhalf = lane >> 5;
+  const int row = row0 + 4 * lrow; // of this lane's C
+  const bool read_c = p.beta != 0.f;
+  float4 bias_r = zero4();
+  if (p.bias_row != nullptr) {
+    if (!kEdge || row + 4 <= p.m) {
+      bias_r = make_float4(p.bias_row[row], p.bias_row[row + 1], p.bias_row[row + 2], p.bias_row[row + 3]);
+    } else {
+      if (row < p.m) bias_r.x = p.bias_row[row];
+      if (row + 1 < p.m) bias_r.y = p.bias_row[row + 1];
+      if (row + 2 < p.m) bias_r.z = p.bias_row[row + 2];
+    }
+  }
+  const bool row_bias = p.bias_row != nullptr;
+  const auto finish = [&](float v, float br, float bc) {
+    if (row_bias) v += br;
+    v += bc;
+    return (p.relu != 0 && v < 0.f) ? 0.f : v;
+  };
+  const bool extra = row_bias || p.bias_col != nullptr || p.relu != 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    // MFMA column lrow, rows 4*u .. 4*u+3; float4s permuted among eight so that
+    // eight lanes' stores hit distinct banks.
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int u = 8 * (v >> 2) + 4 * lhalf + (v & 3);
+      *reinterpret_cast<float4*>(lds + 128 * lrow + 4 * (u ^ (lrow & 7))) =
+          make_float4(acc[0][j][v], acc[1][j][v], acc[2][j][v], acc[3][j][v]);
+    }
+    // Columns in batches of 8 per lane, a batch's old C loaded before its use.
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      float4 old[8];
+      if (read_c) {
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          const int col = col0 + 4 * (16 * b + 2 * t + lhalf) + j;
+          if (!kEdge || (row + 4 <= p.m && col < p.n))
+            old[t] = *reinterpret_cast<const float4*>(p.c + (int64_t)col * p.ldc + row);
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        const int pc = 16 * b + 2 * t + lhalf;
+        const int col = col0 + 4 * pc + j;
+        const float4 s = *reinterpret_cast<const float4*>(lds + 128 * pc + 4 * (lrow ^ (pc & 7)));
+        if (kEdge && (row >= p.m || col >= p.n)) continue;
+        float* dst = p.c + (int64_t)col * p.ldc + row;
+        const float bias_c = p.bias_col != nullptr ? p.bias_col[col] : 0.f;
+        if (!kEdge || row + 4 <= p.m) {
+          float4 r = make_float4(p.alpha * s.x, p.alpha * s.y, p.alpha * s.z, p.alpha * s.w);
+          if (read_c) {
+            r.x = p.alpha * s.x + p.beta * old[t].x;
+            r.y = p.alpha * s.y + p.beta * old[t].y;
+            r.z = p.alpha * s.z + p.beta * old[t].z;
+            r.w = p.alpha * s.w + p.beta * old[t].w;
+          }
+          if (extra) {
+            r.x = finish(r.x, bias_r.x, bias_c);
+            r.y = finish(r.y, bias_r.y, bias_c);
+            r.z = finish(r.z, bias_r.z, bias_c);
+            r.w = finish(r.w, bias_r.w, bias_c);
+          }
+          store4<kStream>(dst, r.x, r.y, r.z, r.w);
+        } else {
+          const float sv[3] = {s.x, s.y, s.z}, br[3] = {bias_r.x, bias_r.y, bias_r.z};
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            if (row + i >= p.m) continue;
+            const float val = p.alpha * sv[i];
+            const float out = read_c ? val + p.beta * dst[i] : val;
+            dst[i] = extra ? finish(out, br[i], bias_c) : out;
           }
         }
       }

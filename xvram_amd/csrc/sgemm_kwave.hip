@@ -425,7 +425,7 @@ __global__ __launch_bounds__(kThreads, kPerCu) void sgemm_kwave_kernel(Params p,
       if (raw) {
         *reinterpret_cast<float4*>(out + (int64_t)colm * ldo + row) = s;
       } else {
-        store_quad(whole, s, row, colm);
+        store_quad<false>(whole, s, row, colm);
       }
     }
   }

@@ -576,11 +576,10 @@ __global__ __launch_bounds__(kThreads, 1) void sgemm_ring_kernel(Params p) {
     }(std::make_integer_sequence<int, kRing>{});
   }
 
-  // Interior tiles: two columns of C per batch of loads. A split launch
-  // stores its range's raw sums instead. Edge tiles: only elements of C.
+  // A split launch stores its range's raw sums (read back at once by the
+  // reduction, so not past the L2). Every load of the ring has landed.
   const Params out = kSplit ? partial_target(p, split) : p;
-  if constexpr (kEdge) store_c_tile<4, false>(out, acc, m0 + wm, n0 + wn, lrow, lhalf);
-  else store_c_interior<4, 2, true>(out, acc, m0 + wm, n0 + wn, lrow, lhalf);
+  store_c_ring<kEdge, !kSplit>(out, acc, ring, m0 + wm, n0 + wn, lane);
 }
 
 // ---- barrier-free kernel for layouts with a k-contiguous operand ------------
@@ -847,8 +846,7 @@ __global__ __launch_bounds__(kThreads, 1) void sgemm_ring8_kernel(Params p) {
   int lane_e;
   asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_e));
   const Params out = kSplit ? partial_target(p, split) : p;
-  if constexpr (kEdge) store_c_tile<4, false>(out, acc, m0 + wm, n0 + wn, lane_e & 31, lane_e >> 5);
-  else store_c_interior<4, 2, true>(out, acc, m0 + wm, n0 + wn, lane_e & 31, lane_e >> 5);
+  store_c_ring<kEdge, !kSplit>(out, acc, ring, m0 + wm, n0 + wn, lane_e);
 }
 
 // ---- split-K reduction --------------------------------------------------------
@@ -878,7 +876,7 @@ __global__ __launch_bounds__(kThreads) void splitk_reduce_kernel(Params p) {
     sum.z += v.z;
     sum.w += v.w;
   }
-  store_quad(p, sum, row, col);
+  store_quad<false>(p, sum, row, col);
 }
 
 // A launch of K below 8 (a K remainder's last rows): too little work for the
