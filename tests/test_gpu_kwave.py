@@ -39,6 +39,13 @@ def plan(m, n, k, form):
     return t, s.value, f.value
 
 
+def many(m, n, k, form):
+    fn = xv.load(hostsim=True).dll.xvram_hostsim_kwave_many
+    fn.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
+    f = ctypes.c_int()
+    return fn(m, n, k, int(form == "NT"), ctypes.byref(f)), 1, f.value
+
+
 def padded_nan(mat, extra):
     rows, cols = mat.shape
     ld = (rows + 3) // 4 * 4 + extra
@@ -53,30 +60,40 @@ CASES = [
     ((1, 1, 8), (0, False, False), None),
     ((33, 31, 9), (0, False, False), None),
     ((100, 84, 260), (0, False, False), None),
-    ((97, 647, 425), (0, False, True), None),
-    ((46, 3, 6081), (0, True, False), None),
-    ((129, 4, 5677), (0, True, True), None),
-    ((606, 2414, 199), (1, False, False), None),
-    ((2231, 599, 619), (1, False, True), None),
-    ((1455, 50, 1263), (1, True, False), None),
-    ((356, 211, 10427), (1, True, True), None),
-    ((2575, 1778, 9), (2, False, False), (5, False, False)),
-    ((3275, 193, 526), (2, False, True), None),
-    ((473, 720, 3809), (2, True, False), None),
-    ((619, 484, 1954), (2, True, True), None),
-    ((3854, 13, 6550), (3, True, False), None),
-    ((6838, 91, 1517), (3, False, True), None),
-    ((7788, 1, 3499), (4, False, True), None),
-    ((11, 1984, 12025), (4, True, True), None),
-    ((6266, 1925, 75), (2, False, False), (5, False, False)),
+    ((5, 3751, 406), (0, False, True), None),
+    ((9, 36, 7124), (0, True, False), None),
+    ((4, 3353, 2220), (0, True, True), None),
+    ((391, 2806, 212), (1, False, False), None),
+    ((1450, 973, 410), (1, False, True), None),
+    ((4910, 7, 2046), (1, True, False), None),
+    ((433, 70, 12283), (1, True, True), None),
+    ((5405, 740, 59), (2, False, False), (6, False, False)),
+    ((3582, 2666, 9), (1, False, False), (6, False, False)),
+    ((1557, 506, 729), (2, False, True), None),
+    ((5417, 43, 1723), (2, True, False), None),
+    ((666, 434, 1525), (2, True, True), None),
+    ((41, 2771, 4028), (2, True, True), (6, True, False)),
+    ((4085, 3, 13738), (3, True, False), None),
+    ((4630, 3, 12564), (3, True, True), None),
+    ((5470, 5, 2545), (4, False, True), None),
+    ((6, 194, 16278), (4, True, False), None),
+    ((2313, 1, 10837), (4, True, True), None),
+]
+# The same for launches of 256 tiles of 256 x 256 and more.
+MANY = [
+    ((100, 65401, 41), (2, False, False), (6, False, False)),
+    ((4098, 4099, 31), (1, False, False), (6, False, False)),
+    ((1501, 15842, 1730), (2, False, False), (5, False, False)),
 ]
 
 
 @pytest.mark.parametrize("form", sorted(FORMS))
-@pytest.mark.parametrize("shape,want,want_nt", CASES, ids=["x".join(map(str, c[0])) for c in CASES])
+@pytest.mark.parametrize("shape,want,want_nt", CASES + MANY,
+                         ids=["x".join(map(str, c[0])) for c in CASES + MANY])
 def test_tile(lib, hip, oracle_mod, shape, want, want_nt, form):
     m, n, k = shape
-    tile, splits, fold = plan(m, n, k, form)
+    rule = many if -(-m // 256) * -(-n // 256) >= 256 else plan
+    tile, splits, fold = rule(m, n, k, form)
     assert (tile, splits > 1, 0 < fold < 1 << 27) == (want_nt if want_nt and form == "NT" else want)
     ops = FORMS[form]
     seed = m + 3 * n + 7 * k

@@ -2,7 +2,7 @@
 (kernels::kwave_plan_shape and launch_bytes_wanted, through the hostsim
 library): over seeded shapes of every form a plan's ranges cover K in multiples
 of 32, its tile is one the form has, no chain of a sum is longer than the ranges
-of the split rule nor than 1024 (up to the tile's fold granularity), a launch
+of the split rule nor than 1024, a launch
 given exactly the partials its plan wants takes the same plan and one byte less
 another that fits, and the partials of any launch fit the allocation-free
 entry's 128 MiB."""
@@ -13,7 +13,7 @@ import numpy as np
 import xvram_amd as xv
 
 ANY = (1 << 64) - 1
-RUN = (64, 48, 32, 32, 128, 0)
+RUN = (32, 32, 32, 32, 128, 0, 0)
 
 
 def fns():
@@ -49,11 +49,11 @@ def test_plan_properties():
             assert not fits or ring
             continue
         tiles.add((tile, nt))
-        assert fits and (tile != 5 or nt)
+        assert fits and (tile < 5 or nt)
         assert (s == 1 and depth == k) or (depth % 32 == 0 and (s - 1) * depth < k <= s * depth)
         chain = min(old[0].value if olds > 1 else k, 1024)
         if (depth + 3) // 4 > chain:
-            assert fold % RUN[tile] == 0 and RUN[tile] <= fold <= max(chain, RUN[tile])
+            assert fold % RUN[tile] == 0 and RUN[tile] <= fold <= chain
         partial = (m + 3) // 4 * 4 * n * 4
         if s > 1:
             split += 1
@@ -62,7 +62,38 @@ def test_plan_properties():
             less = plan(m, n, k, nt, s * partial - 1)
             assert less[1] == 1 or less[1] * partial < s * partial
         assert plan(m, n, k, nt, 0)[1] == 1
-    assert tiles >= {(t, nt) for t in range(5) for nt in (0, 1)} | {(5, 1)} and split > 500
+    assert tiles >= {(t, nt) for t in range(5) for nt in (0, 1)} | {(6, 1)} and split > 500
+
+
+def test_many_tiles():
+    """Launches of 256 tiles of 256 x 256 and more: whole rounds of interior
+    tiles stay on the ring kernels, shallow K and K that is no multiple of
+    their step below 512 do not; the many-tile rule leaves smaller launches
+    alone and a launch it takes wants no partials."""
+    dll = fns()
+    dll.xvram_hostsim_kwave_many.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
+
+    def many(m, n, k, nt):
+        return dll.xvram_hostsim_kwave_many(m, n, k, nt, None)
+
+    assert many(4096, 4096, 256, 1) == many(8192, 8192, 8192, 1) == many(8192, 8192, 1024, 0) == -1
+    assert many(4352, 4352, 4352, 1) == many(5000, 5000, 4999, 1) == -1
+    assert many(3712, 4590, 503, 1) == many(6379, 2968, 32, 1) == 6 and many(5280, 5280, 5280, 0) == 2
+    rng = np.random.default_rng(47)
+    taken = 0
+    for _ in range(2000):
+        m, n = (int(2 ** v) for v in rng.uniform(8, 14, 2))
+        k, nt = int(2 ** rng.uniform(0, 13)), int(rng.integers(0, 2))
+        tile = many(m, n, k, nt)
+        if -(-m // 256) * -(-n // 256) < 256 or k < 8:
+            assert tile == -1
+        elif k < 512 and k % (4 if nt else 8):
+            assert tile >= 0
+        if tile >= 0:
+            taken += 1
+            lda, ldb = (m + 3) // 4 * 4, ((n if nt else k) + 3) // 4 * 4
+            assert dll.xvram_hostsim_launch_bytes_wanted(m, n, k, 0, nt, lda, ldb) == 0
+    assert taken > 100
 
 
 def test_partials_fit_the_scratch():

@@ -641,6 +641,15 @@ extern "C" __attribute__((visibility("default"))) int xvram_hostsim_kwave_plan(
   return p.tile;
 }
 
+// The rule for many 256 x 256 tiles on small ones (kernels::kwave_many_shape):
+// returns the tile's index (-1: the launch runs elsewhere) and *fold.
+extern "C" __attribute__((visibility("default"))) int xvram_hostsim_kwave_many(
+    int64_t m, int64_t n, int64_t k, int nt, int* fold) {
+  const xvram::kernels::KwavePlan p = xvram::kernels::kwave_many_shape(m, n, k, nt != 0);
+  if (fold != nullptr) *fold = p.fold;
+  return p.tile;
+}
+
 // Launches that ran as an interior and edge strips since the last reset.
 extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_edge_split_launches() {
   using namespace xvram;

@@ -23,7 +23,9 @@
 //     read neighbouring pieces of a k-contiguous line at about the same time.
 //     Each load takes 32*KP bytes of a line (KP = 2 or 4: 64 or 128 bytes; at
 //     KP = 1 every 128-byte line is fetched four times, 3001 x 2047 x 4099 T/N
-//     in 436 us against 388).
+//     in 436 us against 388; N/T has no such lines, and there KP = 1 with four
+//     workgroups a CU hides most of a shallow tile's prologue and epilogue:
+//     4096 x 4096 x 256 in 82 us against 94).
 //   * A launch may also split K over workgroups (p.splits > 1: raw sums to the
 //     partials, splitk_reduce_kernel adds them), which the rule in
 //     sgemm_launch.hpp takes when the tiles alone do not fill the chip.
@@ -33,11 +35,14 @@
 //     values, so no chain is longer than it was there.
 //
 // Measured on device memory, before (256 x 128 tiles and split K) -> now, us a
-// launch: 1024^3 41.7 -> 20.9; 128^3 15.8 -> 3.6; 3001 x 2047 x 4099 T/N 474 ->
-// 377, N/T 555 -> 363; 16384 x 4 x 16384 T/N 551 -> 188 (5.7 TB/s); 4096 x 256 x
-// 4096 T/N 97.4 -> 66; 4096 x 300 x 16384 N/N 453 -> 330; 500 x 500 x 60000 T/N
-// 292 -> 234. Bound by: MFMA issue from about 64 x 64 tiles on (120-140
-// TFLOP/s), HBM for n up to 32, the launch itself below 256^3.
+// launch: 1024^3 41.7 -> 20.0; 128^3 15.8 -> 3.6; 3001 x 2047 x 4099 T/N 474 ->
+// 377, N/T 555 -> 363; 16384 x 4 x 16384 T/N 551 -> 190 (5.7 TB/s); 4096 x 256 x
+// 4096 T/N 97.4 -> 63.7; 4096 x 300 x 16384 N/N 453 -> 327; 500 x 500 x 60000
+// T/N 292 -> 224; and, from launches of many tiles whose K is shallow or no
+// multiple of the ring kernels' step, 3712 x 4590 x 503 N/T 313 -> 140, 6379 x
+// 2968 x 32 N/T 67 -> 34. Bound by: MFMA issue from about 64 x 64 tiles on
+// (120-140 TFLOP/s; 95 % of the cycles a CU is busy, the rest the last round),
+// HBM for n up to 32, the launch itself below 256^3. No LDS bank conflicts.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
@@ -112,18 +117,17 @@ __device__ __forceinline__ int piece_place(int lrow, int g) {
 // half it issues the next kGroup loads of the slot R ahead, into the ring place
 // of the slot whose last fragments are in registers, and in its middle it reads
 // the next step's fragments (after waiting for their slot when it is a new one).
-template <bool kAKC, bool kBKC, int MB, int NB, int KP, int R, int kPerCu>
+template <bool kAKC, bool kBKC, int MB, int NB, int KP, int R, int kPerCu, bool kFold>
 __global__ __launch_bounds__(kThreads, kPerCu) void sgemm_kwave_kernel(Params p, int fold) {
   constexpr int TM = 32 * MB, TN = 32 * NB;
   constexpr int kGroup = MB + NB;         // wave loads of 1 KiB per 8 k values
   constexpr int kLoads = kGroup * KP;     // ... per slot
   constexpr int kSlot = 256 * kLoads;     // floats per slot
   constexpr int kSlotK = 8 * KP;
-  constexpr bool kFold = MB * NB < 8; // (a second set of accumulators fits)
   constexpr int kUnroll = KP % 2 == 0 || R % 2 == 0 ? R : 2 * R;
   // Columns of the tile whose sums go through the LDS at once (every wave's).
   constexpr int kAccFloats = TM * TN;
-  constexpr int kPasses = kAccFloats > R * kSlot && NB > 1 ? 2 : 1;
+  constexpr int kPasses = kAccFloats <= R * kSlot || NB == 1 ? 1 : 2;
   constexpr int kPassFloats = kAccFloats / kPasses;
   constexpr int kWaveLds = R * kSlot > kPassFloats ? R * kSlot : kPassFloats;
   static_assert(kWaves * kWaveLds * 4 * kPerCu <= 160 * 1024, "the rings fit the LDS");
@@ -375,6 +379,9 @@ __global__ __launch_bounds__(kThreads, kPerCu) void sgemm_kwave_kernel(Params p,
   float* out = raw ? whole.partial + (int64_t)split * partial_ld(whole.m) * whole.n : whole.c;
   const int64_t ldo = raw ? partial_ld(whole.m) : whole.ldc;
   constexpr int kNJ = NB / kPasses; // column blocks per pass
+  // C past the L2 from 1 MiB on (2048 x 2048 x 256 N/T 24.0 -> 20.8 us; on a C of
+  // 34 KB waiting for memory costs 0.3 us more than the L2).
+  const bool stream = (int64_t)whole.m * whole.n >= (1 << 18);
   static_assert(kPasses == 1 || NB % kPasses == 0, "whole column blocks per pass");
 #pragma unroll
   for (int pass = 0; pass < kPasses; ++pass) {
@@ -422,11 +429,9 @@ __global__ __launch_bounds__(kThreads, kPerCu) void sgemm_kwave_kernel(Params p,
         s.w += x.w;
       }
       if (row >= whole.m || colm >= whole.n) continue;
-      if (raw) {
-        *reinterpret_cast<float4*>(out + (int64_t)colm * ldo + row) = s;
-      } else {
-        store_quad<false>(whole, s, row, colm);
-      }
+      if (raw) *reinterpret_cast<float4*>(out + (int64_t)colm * ldo + row) = s;
+      else if (stream) store_quad<true>(whole, s, row, colm);
+      else store_quad<false>(whole, s, row, colm);
     }
   }
 }
@@ -441,13 +446,16 @@ hipError_t launch_form(const Params& p, int tile, int fold, hipStream_t s, hipEv
   };
   // kKwaveTiles (sgemm_launch.hpp) in its order.
   switch (tile) {
-  case 0: return go(sgemm_kwave_kernel<AK, BK, 1, 1, 2, 4, 2>);
-  case 1: return go(sgemm_kwave_kernel<AK, BK, 2, 1, 2, 3, 2>);
-  case 2: return go(sgemm_kwave_kernel<AK, BK, 2, 2, 2, 2, 2>);
-  case 3: return go(sgemm_kwave_kernel<AK, BK, 4, 1, 2, 2, 2>);
-  case 4: return go(sgemm_kwave_kernel<AK, BK, 1, 1, 4, 4, 1>);
+  case 0: return go(sgemm_kwave_kernel<AK, BK, 1, 1, 2, 2, 4, true>);
+  case 1: return go(sgemm_kwave_kernel<AK, BK, 2, 1, 2, 2, 3, true>);
+  case 2: return go(sgemm_kwave_kernel<AK, BK, 2, 2, 2, 2, 2, true>);
+  case 3: return go(sgemm_kwave_kernel<AK, BK, 4, 1, 2, 2, 2, true>);
+  case 4: return go(sgemm_kwave_kernel<AK, BK, 1, 1, 4, 4, 1, true>);
   case 5:
-    if constexpr (!AK && !BK) return go(sgemm_kwave_kernel<AK, BK, 4, 2, 1, 3, 2>);
+    if constexpr (!AK && !BK) return go(sgemm_kwave_kernel<AK, BK, 4, 2, 1, 3, 2, false>);
+    break;
+  case 6:
+    if constexpr (!AK && !BK) return go(sgemm_kwave_kernel<AK, BK, 2, 2, 1, 2, 4, false>);
   }
   return hipErrorInvalidValue;
 }

@@ -217,30 +217,32 @@ constexpr int kThinK = 8;
 // with 2048-deep ranges the two are level or these ahead: 4096 x 2048 x 4096 T/N
 // 497 against 490, 2048 x 1024 x 16384 N/N 488 against 490).
 //
-// The model, in us: workgroups run in rounds of per_cu on each CU; one takes
-// (depth + fixed) x `shared` when its CU is full and x `alone` when the last
-// round leaves it the CU; the operands take their bytes over 7.85 TB/s, and the
-// shorter of the two adds 0.56 of itself to the longer; C costs 0.14 us per
-// million elements, a launch 2 us, a split 3.1 us and 0.92 us per million
-// partial elements. Fitted to 165 shapes (squares of 64 to 5500, boxes up to
-// 8192, linear layers of 1 to 1024 columns up to 16384 x 16384, their input and
-// weight gradients, Gram matrices up to K = 65536), each on every tile with one
-// to 32 ranges: the rule's choice ran 2.9 % slower than the fastest measured
-// one on average (25 % at worst) and faster than the launch before on all.
+// The model, in us: workgroups run in rounds of per_cu on each CU; a CU that
+// holds x of them takes (depth + fixed) x max(alone, x * each); the operands
+// take their bytes over 9.67 TB/s, and the shorter of the two adds 0.79 of
+// itself to the longer; C costs 0.15 us per million elements, a launch 2 us, a
+// split 3 us and 1.12 us per million partial elements; in a second to fourth
+// round of two a CU a last round of more than a third counts as full. Fitted to 180 shapes
+// (squares, boxes up to 16384, linear layers of 1 to 1024 columns up to 16384 x
+// 16384, their input and weight gradients, Gram matrices up to K = 65536), each
+// on every tile with one to 32 ranges: the rule's choice ran 3.4 % slower than
+// the fastest measured one on average below 256 tiles of 256 x 256 (36 % at
+// worst, on 6 us) and 0.1 % from there on.
 struct KwaveTile {
   int mb, nb;    // 32 x 32 blocks of rows and of columns
   int per_cu;    // workgroups a CU holds
   int run;       // a fold's k values are a multiple of this; 0 = cannot fold
-  double alone, shared, fixed;
+  double alone, each, fixed;
 };
 inline constexpr KwaveTile kKwaveTiles[] = {
-    {1, 1, 2, 64, 0.00493, 0.00949, 213}, {2, 1, 2, 48, 0.00829, 0.0159, 187},
-    {2, 2, 2, 32, 0.01436, 0.02617, 189}, {4, 1, 2, 32, 0.01428, 0.02855, 194},
-    {1, 1, 1, 128, 0.00403, 0.00403, 621}, // slots of 32 k values, deep rings
-    {4, 2, 2, 0, 0.03087, 0.05406, 131},   // N/T only
+    {1, 1, 4, 32, 0.00725, 0.0045, 108},  {2, 1, 3, 32, 0.00981, 0.00764, 117},
+    {2, 2, 2, 32, 0.0145, 0.01308, 145},  {4, 1, 2, 32, 0.01462, 0.01376, 167},
+    {1, 1, 1, 128, 0.0037, 0.00397, 583}, // slots of 32 k values, deep rings
+    {4, 2, 2, 0, 0.0311, 0.0256, 104},    // N/T only
+    {2, 2, 4, 0, 0.0173, 0.0136, 81},     // N/T only, slots of 8 k values
 };
-constexpr int kKwaveTileCount = 6;
-constexpr int kKwaveNtTile = 5, kKwaveSkinnyTile = 3;
+constexpr int kKwaveTileCount = 7;
+constexpr int kKwaveNtTile = 5, kKwaveSkinnyTile = 3; // from kKwaveNtTile on: N/T only
 constexpr uint64_t kKwaveMaxPartialBytes = uint64_t{64} << 20;
 
 struct KwavePlan {
@@ -250,23 +252,22 @@ struct KwavePlan {
   int fold = 0;   // k values of one wave between folds of its accumulators
 };
 
-// The plan of an m x n x k launch of form `nt` or not, whose operand panels the
-// kernels can address (each spans less than 2^31 bytes), given room for
-// `workspace_bytes` of partials. The chains of a sum are no longer than the
-// ranges of the split that split_k_shape takes for the launch (nor than 1024:
-// a fold that rare costs nothing measurable).
-inline KwavePlan kwave_plan_shape(int64_t m, int64_t n, int64_t k, bool nt,
-                                  uint64_t workspace_bytes) {
+// The fastest plan by the model of an m x n x k launch of form `nt` or not,
+// given room for `workspace_bytes` of partials, and in *time its time. A
+// launch of kComputeUnits tiles of 256 x 256 and more is not split over
+// workgroups. The chains of a sum are no longer than the ranges of the split
+// that split_k_shape takes for the launch (nor than 1024: a fold that rare
+// costs nothing measurable; where those ranges are 64 or 96 deep, 32, since
+// the waves' runs end in a rest of their own).
+inline KwavePlan kwave_fastest(int64_t m, int64_t n, int64_t k, bool nt, uint64_t workspace_bytes,
+                               double* time_out) {
   KwavePlan best;
   if (m <= 0 || n <= 0 || k < kThinK) return best;
-  if (((m + 255) / 256) * ((n + 255) / 256) >= kComputeUnits) return best;
+  const bool many = ((m + 255) / 256) * ((n + 255) / 256) >= kComputeUnits;
   const SplitK old = split_k_shape(m, n, k, nt, true, ~uint64_t{0});
-  if (old.splits > 1 && !old.narrow && old.depth >= 4096 &&
-      16 * (m / 256) * (n / 256) * old.splits >= 15 * kComputeUnits)
-    return best;
   const int64_t chain = std::min<int64_t>(old.splits > 1 ? old.depth : k, 1024);
   const double elements = 1e-6 * double(m) * double(n);
-  const double memory = 4e-6 * (double(m) + double(n)) * double(k) / 7.85;
+  const double memory = 4e-6 * (double(m) + double(n)) * double(k) / 9.67;
   const int64_t partial = split_partial_ld(m) * n * 4;
   double best_time = 0;
   for (int i = 0; i < kKwaveTileCount; ++i) {
@@ -274,38 +275,56 @@ inline KwavePlan kwave_plan_shape(int64_t m, int64_t n, int64_t k, bool nt,
     // The tiles each shape was measured on: 128 x 64 for N/T, 128 x 32 up to
     // 128 columns (twice the operand traffic of 64 x 64 beyond), one column
     // block up to 32 columns.
-    if ((i == kKwaveNtTile && !nt) || (i == kKwaveSkinnyTile && n > 128) || (t.nb > 1 && n <= 32))
+    if ((i >= kKwaveNtTile && !nt) || (i == kKwaveSkinnyTile && n > 128) || (t.nb > 1 && n <= 32))
       continue;
     const int64_t tiles = ((m + 32 * t.mb - 1) / (32 * t.mb)) * ((n + 32 * t.nb - 1) / (32 * t.nb));
     for (const int s : {1, 2, 3, 4, 5, 6, 8, 11, 16, 24, 32}) {
       SplitK sk;
       sk.depth = static_cast<int>(k);
       if (s > 1) {
-        if (tiles * s > 12 * kComputeUnits || k < 128 * s ||
+        if (many || tiles * s > 12 * kComputeUnits || k < 128 * s ||
             uint64_t(s) * uint64_t(partial) > std::min(workspace_bytes, kKwaveMaxPartialBytes))
           break;
         sk = split_ranges(k, s, false);
         if (sk.splits != s) continue;
       }
       const bool folds = (sk.depth + 3) / 4 > chain;
-      if (folds && t.run == 0) continue;
+      if (folds && (t.run == 0 || t.run > chain)) continue;
       const int64_t groups = tiles * s, slots = t.per_cu * kComputeUnits;
       const int64_t full = (groups - 1) / slots, last = groups - full * slots;
-      const double compute = (sk.depth + t.fixed) *
-                             (t.shared * double(full) + (last > kComputeUnits ? t.shared : t.alone));
-      const double time = 2.0 + std::max(compute, memory) + 0.56 * std::min(compute, memory) +
-                          0.14 * elements + (s > 1 ? 3.1 + 0.92 * s * elements : 0.0);
+      // After a few rounds the freed places come in pairs.
+      const bool pairs = t.per_cu == 2 && full >= 1 && full <= 3;
+      const double held = double(std::min<int64_t>(
+          t.per_cu, ((pairs ? 3 * last / 2 : last) + kComputeUnits - 1) / kComputeUnits));
+      const double compute = (sk.depth + t.fixed) * (t.each * t.per_cu * double(full) +
+                                                     std::max(t.alone, t.each * held));
+      const double time = 2.0 + std::max(compute, memory) + 0.79 * std::min(compute, memory) +
+                          0.15 * elements + (s > 1 ? 3.0 + 1.12 * s * elements : 0.0);
       if (best.tile < 0 || time < best_time) {
         best_time = time;
         best.tile = i;
         best.splits = s;
         best.depth = sk.depth;
-        best.fold = folds ? static_cast<int>(std::max<int64_t>(t.run, chain / t.run * t.run))
-                          : (t.run > 0 ? (1 << 28) / t.run * t.run : 0);
+        best.fold = t.run == 0 ? 0
+                               : folds ? static_cast<int>((chain <= 96 ? 32 : chain) / t.run * t.run)
+                                       : (1 << 28) / t.run * t.run;
       }
     }
   }
+  if (time_out != nullptr) *time_out = best_time;
   return best;
+}
+
+// The plan of a launch of fewer than kComputeUnits tiles of 256 x 256, whose
+// operand panels the kernels can address (each spans less than 2^31 bytes).
+inline KwavePlan kwave_plan_shape(int64_t m, int64_t n, int64_t k, bool nt,
+                                  uint64_t workspace_bytes) {
+  if (m <= 0 || n <= 0 || ((m + 255) / 256) * ((n + 255) / 256) >= kComputeUnits) return {};
+  const SplitK old = split_k_shape(m, n, k, nt, true, ~uint64_t{0});
+  if (old.splits > 1 && !old.narrow && old.depth >= 4096 &&
+      16 * (m / 256) * (n / 256) * old.splits >= 15 * kComputeUnits)
+    return {};
+  return kwave_fastest(m, n, k, nt, workspace_bytes, nullptr);
 }
 
 // The plan a launch takes given room for `workspace_bytes` of partials.
@@ -545,6 +564,74 @@ inline int64_t k_remainder_shape(int64_t m, int64_t n, int64_t k, bool nt) {
   return gains ? k1 : 0;
 }
 
+// Many tiles on small ones. A launch of kComputeUnits tiles of 256 x 256 and
+// more runs on the tiles of kKwaveTiles instead where they model at least 4 %
+// faster than what the rules above make of it: shallow or odd K (no ring kernel
+// takes a K that is not a multiple of its step below 512) and ragged shapes
+// whose last round or strips cost much. The ring kernels are modelled, in us,
+// at rounds x (0.2155 K + 14) + 2 (4 % more K and 16 for edge instances; 4096 x
+// 4096 at K = 256 71 us, at 4096 907, 8192^3 7180, 8191^2 x 2048 1894), a
+// split's partials at 1.2 us per million elements and 8, strips at what
+// kwave_fastest says, a K remainder at 2.3 us per million elements of C and 4;
+// the small tiles at 7 % over kwave_fastest's time from K = 1500 on (their
+// operands no longer stay in the L2), proportionally less below. On 48 shapes
+// from 4096^2 x 256 to 6499^3 the choice was within 0.4 % of the better of the
+// two on average (6 % at worst): 3712 x 4590 x 503 N/T 313 -> 140 us, 5994 x
+// 3000 x 146 N/T 125 -> 62, 6379 x 2968 x 32 N/T 67 -> 34, 1504 x 15840 x 1728
+// N/T 785 -> 607, 5280^3 N/N 2344 -> 2127.
+inline double ring_time(int64_t tiles, int64_t k) {
+  return double(cu_rounds(tiles)) * (0.2155 * double(k) + 14.0);
+}
+
+// The model's time of an interior launch with its tail split.
+inline double interior_time(int64_t m, int64_t n, int64_t k) {
+  const TailSplit ts = (m / 256) * (n / 256) >= kComputeUnits
+                           ? tail_split_timed(m, n, k, ~uint64_t{0}, nullptr)
+                           : TailSplit{};
+  if (ts.head_m == 0) return ring_time((m / 256) * (n / 256), k) + 2.0;
+  const int64_t tail_m = m - ts.head_m;
+  return ring_time(ts.head_m / 256 * (n / 256), k) +
+         ring_time(tail_m / 256 * (n / 256) * ts.tail.splits, ts.tail.depth) +
+         1.2e-6 * double(ts.tail.splits) * double(tail_m) * double(n) + 8.0;
+}
+
+// The plan on small tiles of a launch of many tiles (tile -1: the rules above).
+inline KwavePlan kwave_many_shape(int64_t m, int64_t n, int64_t k, bool nt) {
+  if (m <= 0 || n <= 0 || k < kThinK ||
+      ((m + 255) / 256) * ((n + 255) / 256) < kComputeUnits)
+    return {};
+  double small = 0;
+  const KwavePlan plan = kwave_fastest(m, n, k, nt, 0, &small);
+  small *= 1.0 + 0.07 * std::min(1.0, double(k) / 1500.0);
+  const int64_t k1 = k - k % (nt ? 4 : 8);
+  if (k1 != k && k1 < 512) return plan; // the general kernel's K
+  double ring = k1 == k ? 0.0 : 2.3e-6 * double(m) * double(n) + 4.0;
+  if (m % 256 == 0 && n % 256 == 0) {
+    ring += interior_time(m, n, k1);
+  } else if (edge_split_rated_faster(m, n, k1, nt)) {
+    const int64_t mi = m / 256 * 256, ni = n / 256 * 256;
+    ring += interior_time(mi, ni, k1);
+    double strip = 0;
+    if (ni < n && kwave_fastest(mi, n - ni, k1, nt, ~uint64_t{0}, &strip).tile >= 0)
+      ring += strip + 3.0;
+    if (mi < m && kwave_fastest(m - mi, n, k1, nt, ~uint64_t{0}, &strip).tile >= 0)
+      ring += strip + 3.0;
+  } else {
+    ring += double(cu_rounds(((m + 255) / 256) * ((n + 255) / 256))) *
+                (0.2241 * double(k1) + 16.0) + 2.0;
+  }
+  return small < 0.96 * ring ? plan : KwavePlan{};
+}
+
+inline KwavePlan kwave_many_plan(const SgemmLaunch& l) {
+  constexpr int64_t kLimit = int64_t(1) << 31;
+  if (l.a2 != nullptr || l.b2 != nullptr) return {};
+  const int64_t a_bytes = (l.a_kcontig ? int64_t{l.m} : int64_t{l.k}) * l.lda * 4;
+  const int64_t b_bytes = (l.b_ncontig ? int64_t{l.k} : int64_t{l.n}) * l.ldb * 4;
+  if (a_bytes >= kLimit || b_bytes >= kLimit) return {};
+  return kwave_many_shape(l.m, l.n, l.k, !l.a_kcontig && l.b_ncontig);
+}
+
 struct KParts {
   int count = 0; // 0 = no K remainder
   SgemmLaunch part[2];
@@ -597,6 +684,7 @@ inline uint64_t split_k_bytes_wanted(const SgemmLaunch& l) {
 // launch_sgemm runs it: its own, or the most that any part of its K remainder
 // or edge split wants (they share the workspace in turn).
 inline uint64_t launch_bytes_wanted(const SgemmLaunch& l) {
+  if (kwave_many_plan(l).tile >= 0) return 0;
   const KParts kp = k_remainder_parts_shape(l);
   const SgemmLaunch& base = kp.count > 0 ? kp.part[0] : l;
   const EdgeParts e = edge_parts_shape(base);

@@ -318,20 +318,6 @@ int launch_sgemm(const SgemmLaunch& launch, void* stream) {
   // out-of-memory hipMemCreate the cache already handled, for one): consume
   // that first so it is not reported as a launch failure.
   (void)hipGetLastError();
-  // K not a multiple of the ring kernels' step where a tail or edge split
-  // would pay: the rounded K, then the rest (sgemm_launch.hpp).
-  if (const KParts kp = k_remainder_parts(launch); kp.count > 0) {
-    for (int i = 0; i < kp.count; ++i)
-      if (const int rc = launch_sgemm(kp.part[i], stream); rc != 0) return rc;
-    return 0;
-  }
-  // Ragged m or n over many tiles: the interior and the edge strips as
-  // launches of their own (sgemm_launch.hpp), one after another.
-  if (const EdgeParts e = edge_parts(launch); e.count > 0) {
-    for (int i = 0; i < e.count; ++i)
-      if (const int rc = launch_sgemm(e.part[i], stream); rc != 0) return rc;
-    return 0;
-  }
   Params p;
   p.a = launch.a;
   p.b = launch.b;
@@ -356,6 +342,23 @@ int launch_sgemm(const SgemmLaunch& launch, void* stream) {
   auto* s = static_cast<hipStream_t>(stream);
   auto* e0 = static_cast<hipEvent_t>(launch.start_event);
   auto* e1 = static_cast<hipEvent_t>(launch.stop_event);
+  // Many 256 x 256 tiles that smaller ones run faster (sgemm_launch.hpp).
+  if (const KwavePlan kw = kwave_many_plan(launch); kw.tile >= 0)
+    return static_cast<int>(launch_kwave(p, kw, launch.a_kcontig, launch.b_ncontig, s, e0, e1));
+  // K not a multiple of the ring kernels' step where a tail or edge split
+  // would pay: the rounded K, then the rest (sgemm_launch.hpp).
+  if (const KParts kp = k_remainder_parts(launch); kp.count > 0) {
+    for (int i = 0; i < kp.count; ++i)
+      if (const int rc = launch_sgemm(kp.part[i], stream); rc != 0) return rc;
+    return 0;
+  }
+  // Ragged m or n over many tiles: the interior and the edge strips as
+  // launches of their own (sgemm_launch.hpp), one after another.
+  if (const EdgeParts e = edge_parts(launch); e.count > 0) {
+    for (int i = 0; i < e.count; ++i)
+      if (const int rc = launch_sgemm(e.part[i], stream); rc != 0) return rc;
+    return 0;
+  }
   if (launch.a2 != nullptr || launch.b2 != nullptr) {
     // Two K panels: the barrier-free kernels only.
     if (!two_panel_valid(launch)) return static_cast<int>(hipErrorInvalidValue);
