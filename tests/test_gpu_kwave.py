@@ -41,9 +41,10 @@ def plan(m, n, k, form):
 
 def many(m, n, k, form):
     fn = xv.load(hostsim=True).dll.xvram_hostsim_kwave_many
-    fn.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
+    fn.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int, ctypes.POINTER(ctypes.c_int), ctypes.c_void_p,
+                                          ctypes.c_void_p]
     f = ctypes.c_int()
-    return fn(m, n, k, int(form == "NT"), ctypes.byref(f)), 1, f.value
+    return fn(m, n, k, int(form == "NT"), ctypes.byref(f), None, None), 1, f.value
 
 
 def padded_nan(mat, extra):

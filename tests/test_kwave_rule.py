@@ -66,34 +66,47 @@ def test_plan_properties():
 
 
 def test_many_tiles():
-    """Launches of 256 tiles of 256 x 256 and more: whole rounds of interior
-    tiles stay on the ring kernels, shallow K and K that is no multiple of
-    their step below 512 do not; the many-tile rule leaves smaller launches
-    alone and a launch it takes wants no partials."""
+    """Launches of 256 tiles of 256 x 256 and more (kernels::many_shape): whole
+    rounds of interior tiles stay on the ring kernels; shallow K and K that is no
+    multiple of their step below 512 go to small tiles and want no partials; a
+    rectangle of whole rounds is whole 256 x 256 tiles inside C that fill at
+    least 19/20 of their rounds, smaller than C, and needs K of the ring
+    kernels' step from 1024 on."""
     dll = fns()
-    dll.xvram_hostsim_kwave_many.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
+    i64, pint = ctypes.c_int64, ctypes.POINTER(ctypes.c_int)
+    dll.xvram_hostsim_kwave_many.argtypes = [i64] * 3 + [ctypes.c_int, pint] + [ctypes.POINTER(i64)] * 2
 
     def many(m, n, k, nt):
-        return dll.xvram_hostsim_kwave_many(m, n, k, nt, None)
+        mi, ni = i64(), i64()
+        t = dll.xvram_hostsim_kwave_many(m, n, k, nt, None, ctypes.byref(mi), ctypes.byref(ni))
+        return t, mi.value, ni.value
 
-    assert many(4096, 4096, 256, 1) == many(8192, 8192, 8192, 1) == many(8192, 8192, 1024, 0) == -1
-    assert many(4352, 4352, 4352, 1) == many(5000, 5000, 4999, 1) == -1
-    assert many(3712, 4590, 503, 1) == many(6379, 2968, 32, 1) == 6 and many(5280, 5280, 5280, 0) == 2
+    for whole in ((4096, 4096, 256, 1), (8192, 8192, 8192, 1), (8192, 8192, 1024, 0)):
+        assert many(*whole) == (-1, 0, 0)
+    assert many(5000, 5000, 5000, 0) == many(5000, 5000, 5000, 1) == (-1, 4096, 4096)
+    assert many(3712, 4590, 503, 1)[0] == many(6379, 2968, 32, 1)[0] == 6
     rng = np.random.default_rng(47)
-    taken = 0
+    small = rect = 0
     for _ in range(2000):
         m, n = (int(2 ** v) for v in rng.uniform(8, 14, 2))
         k, nt = int(2 ** rng.uniform(0, 13)), int(rng.integers(0, 2))
-        tile = many(m, n, k, nt)
+        k = k // 8 * 8 if rng.random() < 0.5 else k
+        tile, mi, ni = many(m, n, k, nt)
         if -(-m // 256) * -(-n // 256) < 256 or k < 8:
-            assert tile == -1
+            assert (tile, mi, ni) == (-1, 0, 0)
         elif k < 512 and k % (4 if nt else 8):
             assert tile >= 0
+        lda, ldb = (m + 3) // 4 * 4, ((n if nt else k) + 3) // 4 * 4
         if tile >= 0:
-            taken += 1
-            lda, ldb = (m + 3) // 4 * 4, ((n if nt else k) + 3) // 4 * 4
-            assert dll.xvram_hostsim_launch_bytes_wanted(m, n, k, 0, nt, lda, ldb) == 0
-    assert taken > 100
+            small += 1
+            assert mi == 0 and dll.xvram_hostsim_launch_bytes_wanted(m, n, k, 0, nt, lda, ldb) == 0
+        if mi:
+            rect += 1
+            assert mi % 256 == ni % 256 == 0 and 0 < mi <= m and 0 < ni <= n and (mi < m or ni < n)
+            groups = mi // 256 * (ni // 256)
+            assert 20 * groups >= 19 * -(-groups // 256) * 256
+            assert k >= 1024 and k % (4 if nt else 8) == 0
+    assert small > 100 and rect > 30
 
 
 def test_partials_fit_the_scratch():

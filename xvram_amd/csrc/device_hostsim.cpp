@@ -641,13 +641,15 @@ extern "C" __attribute__((visibility("default"))) int xvram_hostsim_kwave_plan(
   return p.tile;
 }
 
-// The rule for many 256 x 256 tiles on small ones (kernels::kwave_many_shape):
-// returns the tile's index (-1: the launch runs elsewhere) and *fold.
+// The rule for many 256 x 256 tiles (kernels::many_shape): returns the small
+// tile's index (-1: none) with *fold, or the rectangle's *mi x *ni (0: none).
 extern "C" __attribute__((visibility("default"))) int xvram_hostsim_kwave_many(
-    int64_t m, int64_t n, int64_t k, int nt, int* fold) {
-  const xvram::kernels::KwavePlan p = xvram::kernels::kwave_many_shape(m, n, k, nt != 0);
-  if (fold != nullptr) *fold = p.fold;
-  return p.tile;
+    int64_t m, int64_t n, int64_t k, int nt, int* fold, int64_t* mi, int64_t* ni) {
+  const xvram::kernels::ManyPlan p = xvram::kernels::many_shape(m, n, k, nt != 0);
+  if (fold != nullptr) *fold = p.small.fold;
+  if (mi != nullptr) *mi = p.mi;
+  if (ni != nullptr) *ni = p.ni;
+  return p.small.tile;
 }
 
 // Launches that ran as an interior and edge strips since the last reset.

@@ -595,41 +595,99 @@ inline double interior_time(int64_t m, int64_t n, int64_t k) {
          1.2e-6 * double(ts.tail.splits) * double(tail_m) * double(n) + 8.0;
 }
 
-// The plan on small tiles of a launch of many tiles (tile -1: the rules above).
-inline KwavePlan kwave_many_shape(int64_t m, int64_t n, int64_t k, bool nt) {
-  if (m <= 0 || n <= 0 || k < kThinK ||
-      ((m + 255) / 256) * ((n + 255) / 256) < kComputeUnits)
-    return {};
-  double small = 0;
-  const KwavePlan plan = kwave_fastest(m, n, k, nt, 0, &small);
-  small *= 1.0 + 0.07 * std::min(1.0, double(k) / 1500.0);
-  const int64_t k1 = k - k % (nt ? 4 : 8);
-  if (k1 != k && k1 < 512) return plan; // the general kernel's K
-  double ring = k1 == k ? 0.0 : 2.3e-6 * double(m) * double(n) + 4.0;
-  if (m % 256 == 0 && n % 256 == 0) {
-    ring += interior_time(m, n, k1);
-  } else if (edge_split_rated_faster(m, n, k1, nt)) {
-    const int64_t mi = m / 256 * 256, ni = n / 256 * 256;
-    ring += interior_time(mi, ni, k1);
-    double strip = 0;
-    if (ni < n && kwave_fastest(mi, n - ni, k1, nt, ~uint64_t{0}, &strip).tile >= 0)
-      ring += strip + 3.0;
-    if (mi < m && kwave_fastest(m - mi, n, k1, nt, ~uint64_t{0}, &strip).tile >= 0)
-      ring += strip + 3.0;
-  } else {
-    ring += double(cu_rounds(((m + 255) / 256) * ((n + 255) / 256))) *
-                (0.2241 * double(k1) + 16.0) + 2.0;
-  }
-  return small < 0.96 * ring ? plan : KwavePlan{};
+// The model's time of a launch of many tiles as the rules above run it (K a
+// multiple of the ring kernels' step).
+inline double ring_rules_time(int64_t m, int64_t n, int64_t k, bool nt) {
+  if (m % 256 == 0 && n % 256 == 0) return interior_time(m, n, k);
+  if (!edge_split_rated_faster(m, n, k, nt))
+    return double(cu_rounds(((m + 255) / 256) * ((n + 255) / 256))) *
+               (0.2241 * double(k) + 16.0) + 2.0;
+  const int64_t mi = m / 256 * 256, ni = n / 256 * 256;
+  double time = interior_time(mi, ni, k), strip = 0;
+  if (ni < n && kwave_fastest(mi, n - ni, k, nt, ~uint64_t{0}, &strip).tile >= 0) time += strip + 3.0;
+  if (mi < m && kwave_fastest(m - mi, n, k, nt, ~uint64_t{0}, &strip).tile >= 0) time += strip + 3.0;
+  return time;
 }
 
-inline KwavePlan kwave_many_plan(const SgemmLaunch& l) {
+// Whole rounds. A launch of many tiles may also run as the rectangle of
+// interior 256 x 256 tiles that fills whole rounds of the CUs best, on the ring
+// kernels, and the rest of C, a right and a bottom strip, on small tiles: no
+// round is mostly empty, no tile is padded to 256 and nothing is split and
+// reduced. 5000^3 T/T, 16 x 16 tiles and strips 904 wide: 1867 -> 1770 us; 4500^3
+// N/N 1380 -> 1307, 4576^3 N/T 1406 -> 1317, 11378 x 2374 x 7040 T/T 2870 -> 2705.
+// Modelled like the rest, the strips at 131 TFLOP/s and 8 us each, for K from
+// 1024 on, and taken where that is 3 % faster than the rules above and than
+// small tiles alone (53 shapes: none more than 1.1 % slower than before).
+struct ManyPlan {
+  KwavePlan small;        // on small tiles (tile >= 0), or
+  int64_t mi = 0, ni = 0; // the rectangle's rows and columns; neither: the rules above
+};
+
+inline ManyPlan many_shape(int64_t m, int64_t n, int64_t k, bool nt) {
+  ManyPlan plan;
+  if (m <= 0 || n <= 0 || k < kThinK ||
+      ((m + 255) / 256) * ((n + 255) / 256) < kComputeUnits)
+    return plan;
+  double small = 0;
+  const KwavePlan kw = kwave_fastest(m, n, k, nt, 0, &small);
+  small *= 1.0 + 0.07 * std::min(1.0, double(k) / 1500.0);
+  const int64_t k1 = k - k % (nt ? 4 : 8);
+  if (k1 != k && k1 < 512) { // the general kernel's K
+    plan.small = kw;
+    return plan;
+  }
+  const double rest = k1 == k ? 0.0 : 2.3e-6 * double(m) * double(n) + 4.0;
+  double ring = ring_rules_time(m, n, k1, nt) + rest;
+  if (k >= 1024) {
+    const int64_t tm = m / 256, tn = n / 256;
+    int64_t best_m = 0, best_n = 0;
+    double best = 0.97 * std::min(ring, small);
+    for (int64_t rounds = 1; rounds <= tm * tn / kComputeUnits; ++rounds) {
+      for (int64_t a = 1; a <= tm; ++a) {
+        const int64_t b = std::min(tn, rounds * kComputeUnits / a);
+        if (20 * a * b < 19 * rounds * kComputeUnits) continue;
+        const double area = double(m) * double(n) - 65536.0 * double(a * b);
+        const double time = double(rounds) * (0.2155 * double(k1) + 14.0) + 2.0 +
+                            2e-6 * double(k1) * area / 131.0 + (a * 256 < m ? 8.0 : 0.0) +
+                            (b * 256 < n ? 8.0 : 0.0) + rest;
+        if (time < best) {
+          best = time;
+          best_m = a * 256;
+          best_n = b * 256;
+        }
+      }
+    }
+    if (best_m > 0 && (best_m < m || best_n < n)) {
+      if (k1 == k) { // else the K remainder's first part comes here again
+        plan.mi = best_m;
+        plan.ni = best_n;
+      }
+      return plan;
+    }
+  }
+  if (small < 0.96 * ring) plan.small = kw;
+  return plan;
+}
+
+inline ManyPlan many_plan(const SgemmLaunch& l) {
   constexpr int64_t kLimit = int64_t(1) << 31;
   if (l.a2 != nullptr || l.b2 != nullptr) return {};
   const int64_t a_bytes = (l.a_kcontig ? int64_t{l.m} : int64_t{l.k}) * l.lda * 4;
   const int64_t b_bytes = (l.b_ncontig ? int64_t{l.k} : int64_t{l.n}) * l.ldb * 4;
   if (a_bytes >= kLimit || b_bytes >= kLimit) return {};
-  return kwave_many_shape(l.m, l.n, l.k, !l.a_kcontig && l.b_ncontig);
+  return many_shape(l.m, l.n, l.k, !l.a_kcontig && l.b_ncontig);
+}
+
+// The parts of a launch on the rectangle of `plan` and its strips.
+inline EdgeParts many_parts(const SgemmLaunch& l, const ManyPlan& plan) {
+  const int mi = static_cast<int>(plan.mi), ni = static_cast<int>(plan.ni);
+  EdgeParts e;
+  e.part[e.count++] = sub_launch(l, 0, mi, 0, ni);
+  if (ni < l.n) e.part[e.count++] = sub_launch(l, 0, mi, ni, l.n - ni);
+  if (mi < l.m) e.part[e.count++] = sub_launch(l, mi, l.m - mi, 0, l.n);
+  e.part[0].start_event = l.start_event;
+  e.part[e.count - 1].stop_event = l.stop_event;
+  return e;
 }
 
 struct KParts {
@@ -681,17 +739,22 @@ inline uint64_t split_k_bytes_wanted(const SgemmLaunch& l) {
 }
 
 // Bytes of partials one launch wants when the workspace is not the limit, as
-// launch_sgemm runs it: its own, or the most that any part of its K remainder
-// or edge split wants (they share the workspace in turn).
+// launch_sgemm runs it: its own, or the most that any of its parts wants (they
+// share the workspace in turn).
 inline uint64_t launch_bytes_wanted(const SgemmLaunch& l) {
-  if (kwave_many_plan(l).tile >= 0) return 0;
-  const KParts kp = k_remainder_parts_shape(l);
-  const SgemmLaunch& base = kp.count > 0 ? kp.part[0] : l;
-  const EdgeParts e = edge_parts_shape(base);
-  if (e.count == 0) return part_bytes_wanted(base);
-  uint64_t most = 0;
-  for (int i = 0; i < e.count; ++i) most = std::max(most, part_bytes_wanted(e.part[i]));
-  return most;
+  const auto most = [](const SgemmLaunch* parts, int count) {
+    uint64_t bytes = 0;
+    for (int i = 0; i < count; ++i) bytes = std::max(bytes, launch_bytes_wanted(parts[i]));
+    return bytes;
+  };
+  if (const ManyPlan mp = many_plan(l); mp.small.tile >= 0) return 0;
+  else if (mp.mi > 0) {
+    const EdgeParts e = many_parts(l, mp);
+    return most(e.part, e.count);
+  }
+  if (const KParts kp = k_remainder_parts_shape(l); kp.count > 0) return most(kp.part, 1);
+  if (const EdgeParts e = edge_parts_shape(l); e.count > 0) return most(e.part, e.count);
+  return part_bytes_wanted(l);
 }
 
 // The two launches of a K remainder (count 0: none): by shape, and without a

@@ -342,9 +342,17 @@ int launch_sgemm(const SgemmLaunch& launch, void* stream) {
   auto* s = static_cast<hipStream_t>(stream);
   auto* e0 = static_cast<hipEvent_t>(launch.start_event);
   auto* e1 = static_cast<hipEvent_t>(launch.stop_event);
-  // Many 256 x 256 tiles that smaller ones run faster (sgemm_launch.hpp).
-  if (const KwavePlan kw = kwave_many_plan(launch); kw.tile >= 0)
-    return static_cast<int>(launch_kwave(p, kw, launch.a_kcontig, launch.b_ncontig, s, e0, e1));
+  // Many 256 x 256 tiles: smaller ones where they run faster, or whole rounds of
+  // them and the rest on smaller ones (sgemm_launch.hpp).
+  if (const ManyPlan mp = many_plan(launch); mp.small.tile >= 0) {
+    return static_cast<int>(
+        launch_kwave(p, mp.small, launch.a_kcontig, launch.b_ncontig, s, e0, e1));
+  } else if (mp.mi > 0) {
+    const EdgeParts e = many_parts(launch, mp);
+    for (int i = 0; i < e.count; ++i)
+      if (const int rc = launch_sgemm(e.part[i], stream); rc != 0) return rc;
+    return 0;
+  }
   // K not a multiple of the ring kernels' step where a tail or edge split
   // would pay: the rounded K, then the rest (sgemm_launch.hpp).
   if (const KParts kp = k_remainder_parts(launch); kp.count > 0) {
