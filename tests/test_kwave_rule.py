@@ -125,3 +125,33 @@ def test_partials_fit_the_scratch():
         split += wanted > 0
         assert wanted <= 128 << 20, (m, n, k, ak, bn)
     assert split > 300
+
+
+def test_planner_gives_the_partials_frame_to_a_larger_block(oracle_mod):
+    """1024 x 1024 x 8192 N/T under 12 frames of 2 MiB: 2 x 2 C tiles of 512 x
+    512 and 8 K panels. Its launches run on small tiles, so the plan takes all
+    four C tiles in one block instead of keeping a frame for partials: A and B
+    cross the link once, and the product is exact on the analytic pattern."""
+    from gemm_cases import pattern_operands
+    from xvram_amd import abi
+
+    m, n, k = 1024, 1024, 8192
+    a_op, b_op = pattern_operands(m, n, k)
+    lib = xv.load(hostsim=True)
+    lib.dll.xvram_hostsim_reset()
+    with xv.Session(lib, chunk_size_bytes=2 << 20, cache_target_bytes=24 << 20, workspace_cap_bytes=0,
+                    device_headroom_bytes=0, max_transaction_ms=600000) as s:
+        A, B, C = s.allocation(4 * m * k), s.allocation(4 * n * k), s.allocation(4 * m * n)
+        A.write(np.ascontiguousarray(a_op.T, dtype=np.float32))
+        B.write(np.ascontiguousarray(b_op, dtype=np.float32))
+        plan = xv.GemmPlan(s, xv.matrix(A, m, k, m), xv.matrix(B, n, k, n), xv.matrix(C, m, n, m),
+                           abi.OP_N, abi.OP_T)
+        info = plan.info()
+        plan.execute()
+        out = C.read(dtype=np.float32).reshape(n, m).T
+        h2d = s.telemetry().bytes_h2d
+        plan.release()
+    assert (info.tile_m, info.tile_n, info.tile_count) == (512, 512, 32)
+    assert info.maximum_working_set_bytes == 3 * (2 << 20)
+    assert h2d == 4 * (m * k + n * k)
+    assert np.array_equal(out.astype(np.float64), oracle_mod.pattern_expected_matrix(m, n, k))
