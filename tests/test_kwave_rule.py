@@ -85,6 +85,8 @@ def test_many_tiles():
         assert many(*whole) == (-1, 0, 0)
     assert many(5000, 5000, 5000, 0) == many(5000, 5000, 5000, 1) == (-1, 4096, 4096)
     assert many(3712, 4590, 503, 1)[0] == many(6379, 2968, 32, 1)[0] == 6
+    # A grid of 2^24 workgroups of 256 threads is past what one launch holds.
+    assert many(1 << 17, 1 << 18, 9, 0)[0] == 2 and many(1 << 19, 1 << 19, 9, 0)[0] == -1
     rng = np.random.default_rng(47)
     small = rect = 0
     for _ in range(2000):

@@ -278,6 +278,7 @@ inline KwavePlan kwave_fastest(int64_t m, int64_t n, int64_t k, bool nt, uint64_
     if ((i >= kKwaveNtTile && !nt) || (i == kKwaveSkinnyTile && n > 128) || (t.nb > 1 && n <= 32))
       continue;
     const int64_t tiles = ((m + 32 * t.mb - 1) / (32 * t.mb)) * ((n + 32 * t.nb - 1) / (32 * t.nb));
+    if (tiles >= int64_t{1} << 24) continue; // a grid holds fewer than 2^32 threads
     for (const int s : {1, 2, 3, 4, 5, 6, 8, 11, 16, 24, 32}) {
       SplitK sk;
       sk.depth = static_cast<int>(k);

@@ -291,7 +291,8 @@ hipError_t launch_variant(const Params& p, hipStream_t stream, hipEvent_t start,
 
 // A launch with at least this many 256 x 256 tiles (one per CU of the chip)
 // runs a 256 x 256 kernel (sgemm_wide.hip picks a barrier-free one for
-// launches of interior tiles); smaller ones keep two 256 x 128 tiles per CU.
+// launches of interior tiles); smaller ones run on smaller tiles
+// (sgemm_kwave.hip), or, with panels that those cannot address, here.
 constexpr int64_t kWideMinTiles = 256;
 
 // The 256 x 256 kernels address each operand panel with 32-bit buffer
