@@ -338,6 +338,16 @@ __device__ __forceinline__ void store_c_tile(const Params& p, const float16_t (&
   }
 }
 
+// Between LDS accesses of one wave by which its lanes hand each other values: the
+// compiler keeps the accesses before it before those after it, also where it could
+// prove their per-lane addresses apart. No instruction: the LDS serves a wave's
+// accesses in order.
+__device__ __forceinline__ void lanes_exchange() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The same for the ring kernels' waves (kNJ = 4), through 16 KiB of the wave's
 // own LDS: column block j of the accumulators (every fourth column) goes in as
 // the MFMAs left it and comes out with 32 lanes on 128 consecutive rows of a
@@ -346,7 +356,8 @@ __device__ __forceinline__ void store_c_tile(const Params& p, const float16_t (&
 // of its last round on its C (4096 x 4096 x 256 N/T: 80 us for 55 us of MFMAs, now 71; 8192 x 8192 x 128
 // 207 -> 165; 4096^3 920 -> 907; 8192^3 7227 -> 7180).
 // No other wave's LDS is touched and the LDS serves a wave in order, so there
-// is no barrier. A lane's four rows stay the same, and so does its row bias.
+// is no barrier; lanes_exchange keeps the compiler to that order too. A lane's
+// four rows stay the same, and so does its row bias.
 template <bool kEdge, bool kStream>
 __device__ __forceinline__ void store_c_ring(const Params& p, const float16_t (&acc)[4][4], float* lds,
                                              int row0, int col0, int lane) {
@@ -380,6 +391,7 @@ __device__ __forceinline__ void store_c_ring(const Params& p, const float16_t (&
       *reinterpret_cast<float4*>(lds + 128 * lrow + 4 * (u ^ (lrow & 7))) =
           make_float4(acc[0][j][v], acc[1][j][v], acc[2][j][v], acc[3][j][v]);
     }
+    lanes_exchange();
     // Columns in batches of 8 per lane, a batch's old C loaded before its use.
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
@@ -427,6 +439,7 @@ __device__ __forceinline__ void store_c_ring(const Params& p, const float16_t (&
         }
       }
     }
+    if (j < 3) lanes_exchange(); // the next block goes over this one
   }
 }
 
