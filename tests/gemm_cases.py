@@ -2,6 +2,8 @@
 the C ABI, and read C back in logical form. Not a test module."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 
 import xvram_amd as xv
@@ -96,3 +98,30 @@ def pattern_operands(m, n, k):
     j = np.arange(n)[None, :]
     b = (1 + j % 5 + p2 % 3).astype(np.float32)
     return np.asfortranarray(a), np.asfortranarray(b)
+
+
+def route(m, n, k, form, room=(1 << 64) - 1, lda=None, ldb=None):
+    """How a launch of that shape and form runs (kernels::route_with), in words,
+    its parts in brackets, with room for `room` bytes of partials (None: without
+    a workspace); leading dimensions are whole float4s unless given."""
+    fn = xv.load(hostsim=True).dll.xvram_hostsim_route
+    fn.argtypes = [ctypes.c_int] * 5 + [ctypes.c_int64] * 2 + [ctypes.c_int, ctypes.c_uint64,
+                                                              ctypes.c_char_p, ctypes.c_int]
+    ak, bn = form[0] == "T", form[1] == "T"
+    lda = lda or ((k if ak else m) + 3) // 4 * 4
+    ldb = ldb or ((n if bn else k) + 3) // 4 * 4
+    text = ctypes.create_string_buffer(2048)
+    fn(m, n, k, ak, bn, lda, ldb, room is not None, room or 0, text, len(text))
+    return text.value.decode()
+
+
+RUNS = ("two panels", "rectangle", "k remainder", "edge split", "small", "thin", "ring split",
+        "narrow split", "tail split", "ring", "general", "narrow")
+
+
+def runs(lib):
+    """Launches (and parts of launches) the host simulation ran since its last
+    reset, by route: those that occurred."""
+    lib.dll.xvram_hostsim_runs.restype = ctypes.c_uint64
+    counts = {name: lib.dll.xvram_hostsim_runs(i) for i, name in enumerate(RUNS)}
+    return {name: count for name, count in counts.items() if count}

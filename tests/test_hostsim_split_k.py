@@ -1,21 +1,21 @@
-"""CPU tests of split-K launches over libxvram_hostsim.so.
+"""CPU tests of launches that split, over libxvram_hostsim.so.
 
-A launch that would leave workgroup slots idle cuts its K into ranges
-(kernels::split_k_shape: on the ring kernels as many as one round of the CUs
-takes when those are at least 256 deep, else on the 256 x 128 kernel the count
-its timing model rates fastest; each at least 64 deep, in multiples of 32),
-accumulates each range into a partial held in one frame of
-the pool (leading dimension m rounded up to 4), and adds the partials in range
-order before alpha, beta and the epilogue. Launches of interior 256 x 256 tiles
-split on the ring kernels (one workgroup per CU); the others on the 256 x 128
-kernel (two per CU). The simulated device performs exactly that data flow
-(partials written to and read back from the frame, which must be mapped) and
-counts the launches that split, so these tests check the rule itself (through
-the library's own split_k_shape), the planner's reservation of the frame, the
-executor's use of it, the split arithmetic (bit-exact analytic pattern, FP64
-bound with K tails, beta and the epilogue, ragged m and n) and that repeated
-runs give identical bits. The same launches on the GPU are in
-tests/test_gpu_split_k.py."""
+The simulated device takes every launch on the GPU's route (kernels::route): a
+launch that would leave CUs idle runs on small tiles with its K cut into ranges
+over workgroups, accumulates each range into a partial held in one frame of the
+pool (leading dimension m rounded up to 4), and adds the partials in range order
+before alpha, beta and the epilogue; one of many tiles may run as parts (a
+rectangle of whole rounds and strips, an edge split, a K remainder), one after
+another. It performs that data flow (partials written to and read back from the
+frame, which must be mapped) and counts the routes, so these tests check the
+planner's reservation of the frame, the executor's use of it, the arithmetic
+(bit-exact analytic pattern, FP64 bound with K tails, beta and the epilogue,
+ragged m and n) and that repeated runs give identical bits. The rules of the
+larger kernels' splits (kernels::split_k_shape, tail_split_shape,
+edge_split_rated_faster, k_remainder_shape) are checked by themselves: their
+launches are too large to simulate. The same launches on the GPU are in
+tests/test_gpu_kwave.py, test_gpu_split_k.py, test_gpu_tail_split.py and
+test_gpu_edge_split.py."""
 import ctypes
 
 import numpy as np
@@ -24,7 +24,7 @@ import pytest
 import xvram_amd as xv
 from xvram_amd import abi
 
-from gemm_cases import pattern_operands, storage, uniform
+from gemm_cases import pattern_operands, route, runs, storage, uniform
 
 MiB = 1 << 20
 FORMS = {"NN": (abi.OP_N, abi.OP_N), "NT": (abi.OP_N, abi.OP_T), "TN": (abi.OP_T, abi.OP_N),
@@ -39,11 +39,6 @@ def sim():
     lib.dll.xvram_hostsim_split_launches.argtypes = [ctypes.POINTER(ctypes.c_int)]
     yield lib
     lib.dll.xvram_hostsim_reset()
-
-
-def narrow_splits(lib):
-    lib.dll.xvram_hostsim_narrow_split_launches.restype = ctypes.c_uint64
-    return lib.dll.xvram_hostsim_narrow_split_launches()
 
 
 def split_stats(lib):
@@ -90,36 +85,34 @@ def session(lib, frame_mib=16, frames=12):
 
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_split_pattern_is_exact(sim, oracle_mod, form):
-    """512 x 256 x 2048: two 256 x 256 tiles, whose ring split would take
-    64-deep ranges, so the 256 x 128 kernel's 2 x 2 tiles split K into 32
-    ranges of 64 (one launch)."""
+    """512 x 256 x 2048: 128 tiles of 32 x 32, whose K splits into four ranges
+    (one launch)."""
     m, n, k = 512, 256, 2048
     a_op, b_op = pattern_operands(m, n, k)
     with session(sim) as s:
         (out,), info = run(s, a_op, b_op, FORMS[form])
     assert (info.tile_m, info.tile_n, info.tile_k, info.tile_count) == (m, n, k, 1)
     assert info.maximum_working_set_bytes == 4 * 16 * MiB  # C, A, B and the partials' frame
-    assert split_stats(sim) == (1, 32) and narrow_splits(sim) == 1
+    assert split_stats(sim) == (1, 4) and runs(sim) == {"small": 1}
     assert np.array_equal(out.astype(np.float64), oracle_mod.pattern_expected_matrix(m, n, k))
 
 
-
 @pytest.mark.parametrize("form", ["NN", "NT"])
-def test_ring_split_pattern_is_exact(sim, oracle_mod, form):
-    """1024 x 512 x 8192 under 64 MiB frames: eight 256 x 256 tiles whose K
-    splits into 32 ranges of 256 on the ring kernels (one round of the CUs;
-    the 32 partials of 2 MiB fill the partials' frame)."""
+def test_deep_split_pattern_is_exact(sim, oracle_mod, form):
+    """1024 x 512 x 8192 under 64 MiB frames: 128 tiles of 64 x 64, whose K
+    splits into four ranges of 2048."""
     m, n, k = 1024, 512, 8192
     a_op, b_op = pattern_operands(m, n, k)
     with session(sim, frame_mib=64, frames=8) as s:
         (out,), info = run(s, a_op, b_op, FORMS[form])
     assert (info.tile_m, info.tile_n, info.tile_k, info.tile_count) == (m, n, k, 1)
-    assert split_stats(sim) == (1, 32) and narrow_splits(sim) == 0
+    assert split_stats(sim) == (1, 4) and runs(sim) == {"small": 1}
     assert np.array_equal(out.astype(np.float64), oracle_mod.pattern_expected_matrix(m, n, k))
+
 
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_split_with_k_tail_beta_and_epilogue(sim, oracle_mod, form):
-    """K = 1000: eleven ranges, ten of 96 and a tail of 40 (no multiple of
+    """K = 1000: four ranges, three of 256 and a tail of 232 (no multiple of
     32); alpha, beta and a per-column bias with ReLU after the reduction.
     Within the FP64 bound, and the same bits on every run."""
     m, n, k = 512, 256, 1000
@@ -130,7 +123,7 @@ def test_split_with_k_tail_beta_and_epilogue(sim, oracle_mod, form):
     with session(sim) as s:
         outs, _ = run(s, a_op, b_op, FORMS[form], c0, alpha=-0.75, beta=0.5, bias=bias,
                       relu=True, repeat=2)
-    assert split_stats(sim) == (2, 11)
+    assert split_stats(sim) == (2, 4)
     assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
     a64, b64 = a_op.astype(np.float64), b_op.astype(np.float64)
     ref = np.maximum(-0.75 * (a64 @ b64) + 0.5 * c0 + bias[None, :], 0.0)
@@ -141,19 +134,21 @@ def test_split_with_k_tail_beta_and_epilogue(sim, oracle_mod, form):
 
 def test_split_across_k_panels(sim, oracle_mod):
     """K panels smaller than K (frames of 2 MiB: 512 x 1024 panels): each
-    launch splits its own panel; later panels accumulate onto C (beta 1)."""
+    launch takes its own panel, split where that is rated faster; later
+    panels accumulate onto C (beta 1)."""
     m, n, k = 512, 256, 4096
     a_op, b_op = pattern_operands(m, n, k)
     with session(sim, frame_mib=2, frames=16) as s:
         (out,), info = run(s, a_op, b_op, FORMS["NT"])
     assert info.tile_k < k and info.tile_count == k // info.tile_k
-    count, last = split_stats(sim)
-    assert count == info.tile_count and last >= 2
+    wants = "ranges 1 " not in route(m, n, info.tile_k, "NT", 2 * MiB)
+    assert runs(sim) == {"small": info.tile_count}
+    assert split_stats(sim)[0] == (info.tile_count if wants else 0)
     assert np.array_equal(out.astype(np.float64), oracle_mod.pattern_expected_matrix(m, n, k))
 
 
 def test_no_split_when_k_is_shallow(sim, oracle_mod):
-    """K = 120 leaves fewer than two ranges of 64: unsplit."""
+    """K = 120 leaves fewer than two ranges of 128: unsplit."""
     m, n, k = 512, 256, 120
     a_op, b_op = pattern_operands(m, n, k)
     with session(sim) as s:
@@ -212,24 +207,22 @@ def test_split_rule(sim, m, n, k, nt, ring, ws, expect):
 
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_ragged_split_pattern_is_exact(sim, oracle_mod, form):
-    """501 x 200 x 2048: not whole 256 x 256 tiles, so the 256 x 128 kernel's
-    2 x 2 tiles split K into 32 ranges of 64; the partials' leading dimension
-    is 504 (m rounded up to 4) and the reduction's last quad of each column
-    holds one row."""
+    """501 x 200 x 2048: 112 tiles of 32 x 32, cut by m and n, in four K ranges;
+    the partials' leading dimension is 504 (m rounded up to 4) and the
+    reduction's last quad of each column holds one row."""
     m, n, k = 501, 200, 2048
     a_op, b_op = pattern_operands(m, n, k)
     with session(sim) as s:
         (out,), info = run(s, a_op, b_op, FORMS[form])
     assert info.tile_count == 1
-    assert split_stats(sim) == (1, 32) and narrow_splits(sim) == 1
+    assert split_stats(sim) == (1, 4) and runs(sim) == {"small": 1}
     assert np.array_equal(out.astype(np.float64), oracle_mod.pattern_expected_matrix(m, n, k))
 
 
 @pytest.mark.parametrize("axis", [abi.BIAS_PER_ROW, abi.BIAS_PER_COLUMN], ids=["row", "col"])
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_ragged_split_with_k_tail_beta_and_epilogue(sim, oracle_mod, form, axis):
-    """501 x 200 x 1000 on the 256 x 128 kernel: eleven ranges (ten of 96, 40),
-    alpha, beta and a per-row or per-column bias with ReLU after the
+    """501 x 200 x 1000: four ranges (three of 256, 232), alpha, beta and a per-row or per-column bias with ReLU after the
     reduction. Within the FP64 bound, and the same bits on every run."""
     m, n, k = 501, 200, 1000
     a_op = uniform(oracle_mod, m, k, 81)
@@ -240,7 +233,7 @@ def test_ragged_split_with_k_tail_beta_and_epilogue(sim, oracle_mod, form, axis)
     with session(sim) as s:
         outs, _ = run(s, a_op, b_op, FORMS[form], c0, alpha=1.25, beta=-0.5, bias=bias,
                       relu=True, repeat=2, axis=axis)
-    assert split_stats(sim) == (2, 11) and narrow_splits(sim) == 2
+    assert split_stats(sim) == (2, 4) and runs(sim) == {"small": 2}
     assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
     a64, b64 = a_op.astype(np.float64), b_op.astype(np.float64)
     badd = bias[:, None] if axis == abi.BIAS_PER_ROW else bias[None, :]
@@ -273,7 +266,7 @@ def test_split_rule_properties(sim):
     ranges of at least 64 in multiples of 32, keeps to one round of the CUs
     (ring kernels: partials <= 64 MiB) or two rounds of the 256 x 128 kernel's
     slots (partials <= 128 MiB), and a launch given exactly the workspace its
-    split wants (split_k_bytes_wanted) takes the same split, family included;
+    split wants takes the same split, family included;
     one byte less takes fewer ranges on the same family."""
     fn = sim.dll.xvram_hostsim_split_shape
     fn.restype = ctypes.c_int
@@ -442,20 +435,34 @@ def test_edge_split_rule(sim, m, n, k, nt, expect):
 def test_edge_split_pattern_is_exact(sim, oracle_mod):
     """4100 x 4100 x 248 under 128 MiB frames, one launch of 17 x 17 ragged
     tiles: it runs as the 16 x 16 interior tiles, the right strip (4096 x 4)
-    and the bottom strip (4 x 4100), each a launch of its own (the strips
-    split K in the partials' frame the planner reserved); every element of C
-    bit-exact on the analytic pattern."""
+    and the bottom strip (4 x 4100), each a launch of its own; every element of
+    C bit-exact on the analytic pattern."""
     m, n, k = 4100, 4100, 248
     a_op, b_op = pattern_operands(m, n, k)
-    sim.dll.xvram_hostsim_edge_split_launches.restype = ctypes.c_uint64
     sim.dll.xvram_hostsim_kernel_launches.restype = ctypes.c_uint64
     with session(sim, frame_mib=128, frames=8) as s:
         (out,), info = run(s, a_op, b_op, FORMS["NN"])
     assert info.tile_count == 1
-    assert info.maximum_working_set_bytes == 4 * 128 * MiB  # C, A, B and the partials' frame
-    assert sim.dll.xvram_hostsim_edge_split_launches() == 1
+    assert runs(sim) == {"edge split": 1, "ring": 1, "small": 2}
     assert sim.dll.xvram_hostsim_kernel_launches() == 3
     assert np.array_equal(out.astype(np.float64), oracle_mod.pattern_expected_matrix(m, n, k))
+
+
+def test_rectangle_pattern_is_exact(sim, oracle_mod):
+    """4100 x 4100 x 1024 N/T: 16 x 16 interior tiles in one launch, the right
+    strip (4096 x 4) and the bottom strip (4 x 4100), with beta and a bias
+    along each axis' offsets; bit-exact on the analytic pattern."""
+    m, n, k = 4100, 4100, 1024
+    a_op, b_op = pattern_operands(m, n, k)
+    c0 = np.asfortranarray(np.add.outer(np.arange(m) % 5, np.arange(n) % 7).astype(np.float32))
+    bias = (np.arange(m) % 11).astype(np.float32)
+    with session(sim, frame_mib=128, frames=8) as s:
+        (out,), info = run(s, a_op, b_op, FORMS["NT"], c0, beta=2.0, bias=bias,
+                           axis=abi.BIAS_PER_ROW)
+    assert info.tile_count == 1
+    assert runs(sim) == {"rectangle": 1, "ring": 1, "small": 2}
+    expect = oracle_mod.pattern_expected_matrix(m, n, k) + 2.0 * c0 + bias[:, None]
+    assert np.array_equal(out.astype(np.float64), expect)
 
 
 @pytest.mark.parametrize("m,n,k,nt,expect", [
@@ -485,20 +492,19 @@ def test_k_remainder_rule(sim, m, n, k, nt, expect):
 
 
 def test_k_remainder_pattern_is_exact(sim, oracle_mod):
-    """4100 x 4100 x 516 N/N under 128 MiB frames: K % 8 = 4, and the rounded
-    512 takes an edge split, so the launch runs as the 512-deep edge split
-    (no epilogue) and a 4-deep launch onto its result; every element of C
-    bit-exact on the analytic pattern."""
-    m, n, k = 4100, 4100, 516
+    """3072 x 5441 x 1238 N/T: K % 4 = 2, so the launch runs as the 1236-deep
+    product (no epilogue), itself an edge split, and a 2-deep launch onto its
+    result, with the bias; every element of C bit-exact on the analytic
+    pattern."""
+    m, n, k = 3072, 5441, 1238
     a_op, b_op = pattern_operands(m, n, k)
-    sim.dll.xvram_hostsim_k_remainder_launches.restype = ctypes.c_uint64
-    sim.dll.xvram_hostsim_edge_split_launches.restype = ctypes.c_uint64
+    bias = (np.arange(n) % 11).astype(np.float32)
     with session(sim, frame_mib=128, frames=8) as s:
-        (out,), info = run(s, a_op, b_op, FORMS["NN"])
-    assert info.tile_count == 1 and info.maximum_working_set_bytes == 4 * 128 * MiB
-    assert sim.dll.xvram_hostsim_k_remainder_launches() == 1
-    assert sim.dll.xvram_hostsim_edge_split_launches() == 1
-    assert np.array_equal(out.astype(np.float64), oracle_mod.pattern_expected_matrix(m, n, k))
+        (out,), info = run(s, a_op, b_op, FORMS["NT"], bias=bias)
+    assert info.tile_count == 1
+    assert runs(sim) == {"k remainder": 1, "edge split": 1, "small": 2, "thin": 1}
+    expect = oracle_mod.pattern_expected_matrix(m, n, k) + bias[None, :]
+    assert np.array_equal(out.astype(np.float64), expect)
 
 
 def test_partials_never_exceed_the_allocation_free_scratch(sim):
@@ -507,7 +513,7 @@ def test_partials_never_exceed_the_allocation_free_scratch(sim):
     limit): the partials any launch wants -- its split, tail split, the
     largest part of its edge split or the first part of its K remainder --
     fit the allocation-free entry's 128 MiB scratch."""
-    fn = sim.dll.xvram_hostsim_bytes_wanted
+    fn = sim.dll.xvram_hostsim_launch_bytes_wanted
     fn.restype = ctypes.c_uint64
     fn.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                    ctypes.c_int64, ctypes.c_int64]

@@ -60,12 +60,9 @@ struct SimState {
   uint64_t free_bytes = 16ull << 30;
   uint64_t total_bytes = 16ull << 30;
   uint64_t kernel_launches = 0;
-  uint64_t split_launches = 0;  // launches that split K (kernels::split_k_plan)
-  uint64_t narrow_splits = 0;   // of those, split on the 256 x 128 kernel
-  int last_splits = 0;          // K ranges of the last split launch (or tail split)
-  uint64_t tail_splits = 0;     // launches that ran as a head and a split tail
-  uint64_t edge_splits = 0;     // launches that ran as an interior and edge strips
-  uint64_t k_remainders = 0;    // launches that ran as a rounded K and its remainder
+  uint64_t runs[kernels::kRunCount] = {}; // launches and parts by their route (kernels::Run)
+  uint64_t small_splits = 0; // of kSmallTiles, those that split K over workgroups
+  int last_splits = 0;       // K ranges of the last launch that split (or tail split)
   int device_count = 1;       // simulated devices 0 .. device_count-1
   int current_device = 0;     // what the calling thread sees as current (-1: none)
   int last_init_ordinal = -1; // the device the last session set up on
@@ -258,29 +255,24 @@ public:
 
   int launch_sgemm(const kernels::SgemmLaunch& l, Stream) override {
     if (int f = fault(kLaunch)) return f;
-    // A K remainder runs its two launches one after another, and so does an
-    // edge split its parts (sgemm_launch.hpp).
-    if (const kernels::KParts kp = kernels::k_remainder_parts(l); kp.count > 0) {
-      for (int i = 0; i < kp.count; ++i)
-        if (const int rc = dispatch(kp.part[i]); rc != 0) return rc;
-      std::lock_guard<std::mutex> lock(g_sim.mutex);
-      ++g_sim.k_remainders;
-      return 0;
-    }
-    return dispatch(l);
-  }
-
-  int dispatch(const kernels::SgemmLaunch& l) {
-    if (const kernels::EdgeParts e = kernels::edge_parts(l); e.count > 0) {
-      for (int i = 0; i < e.count; ++i)
-        if (const int rc = run_launch(e.part[i]); rc != 0) return rc;
-      std::lock_guard<std::mutex> lock(g_sim.mutex);
-      ++g_sim.edge_splits;
-      return 0;
-    }
     return run_launch(l);
   }
 
+  // sum[i] += x[i * stride] * y.
+  static void add_products(float* __restrict sum, const float* __restrict x, int64_t stride, float y,
+                           int64_t count) {
+    if (stride != 1) {
+      for (int64_t i = 0; i < count; ++i) sum[i] += x[i * stride] * y;
+      return;
+    }
+    int64_t i = 0;
+    for (; i + 8 <= count; i += 8)
+      for (int t = 0; t < 8; ++t) sum[i + t] += x[i + t] * y;
+    for (; i < count; ++i) sum[i] += x[i] * y;
+  }
+
+  // The launch on the GPU's route (kernels::route), its parts one after
+  // another.
   int run_launch(const kernels::SgemmLaunch& l) {
     // Same launch contract as the gfx950 kernel (sgemm_launch.hpp).
     const bool aligned = reinterpret_cast<uintptr_t>(l.a) % 16 == 0 &&
@@ -309,11 +301,22 @@ public:
     if ((l.bias_row && !accessible(reinterpret_cast<uint64_t>(l.bias_row), l.m * 4ull)) ||
         (l.bias_col && !accessible(reinterpret_cast<uint64_t>(l.bias_col), l.n * 4ull)))
       return kSimBadAccess;
+    const kernels::Route route = kernels::route(l);
+    count(route);
+    if (route.count > 0) {
+      for (int i = 0; i < route.count; ++i)
+        if (const int rc = run_launch(route.part[i]); rc != 0) return rc;
+      return 0;
+    }
     // A split launch writes its partials to the workspace (sgemm_launch.hpp);
     // a tail split runs its head rows unsplit and splits its tail rows.
-    const kernels::SplitK sk = two ? kernels::SplitK{} : kernels::split_k_plan(l);
+    kernels::SplitK sk;
+    if (route.run == kernels::Run::kSmallTiles && route.small.splits > 1)
+      sk = kernels::SplitK{route.small.splits, route.small.depth, false};
+    if (route.run == kernels::Run::kRingSplit || route.run == kernels::Run::kNarrowSplit)
+      sk = route.split;
     const kernels::TailSplit ts =
-        two || sk.splits > 1 ? kernels::TailSplit{} : kernels::tail_split_plan(l);
+        route.run == kernels::Run::kTailSplit ? route.tail : kernels::TailSplit{};
     struct Rows {
       int64_t first, count;
       kernels::SplitK split;
@@ -335,6 +338,9 @@ public:
     // (p ascending, the second panel after the first), in FP32. A split
     // launch (or tail) accumulates each K range into its partial, then adds
     // the partials in range order.
+    const auto a_at = [&](int64_t i, int64_t p) {
+      return l.a_kcontig ? l.a + p + i * l.lda : l.a + i + p * l.lda;
+    };
     std::vector<float> acc(static_cast<size_t>(l.m));
     for (int64_t j = 0; j < l.n; ++j) {
       std::fill(acc.begin(), acc.end(), 0.f);
@@ -348,18 +354,14 @@ public:
           const int64_t p_end = std::min<int64_t>(l.k, int64_t{s + 1} * r.split.depth);
           for (int64_t p = int64_t{s} * r.split.depth; p < p_end; ++p) {
             const float y = l.b_ncontig ? l.b[j + p * l.ldb] : l.b[p + j * l.ldb];
-            for (int64_t i = i0; i < i1; ++i)
-              part[i - i0] += (l.a_kcontig ? l.a[p + i * l.lda] : l.a[i + p * l.lda]) * y;
+            add_products(part, a_at(i0, p), l.a_kcontig ? l.lda : 1, y, r.count);
           }
           for (int64_t i = i0; i < i1; ++i)
             acc[i] = s == 0 ? part[i - i0] : acc[i] + part[i - i0];
         }
         for (int64_t p = 0; p < k1 && r.split.splits == 1; ++p) {
           const float y = l.b_ncontig ? l.b[j + p * l.ldb] : l.b[p + j * l.ldb];
-          for (int64_t i = i0; i < i1; ++i) {
-            const float x = l.a_kcontig ? l.a[p + i * l.lda] : l.a[i + p * l.lda];
-            acc[i] += x * y;
-          }
+          add_products(acc.data() + i0, a_at(i0, p), l.a_kcontig ? l.lda : 1, y, r.count);
         }
       }
       for (int64_t p = 0; p < k2; ++p) { // second panel
@@ -381,16 +383,18 @@ public:
     if (l.stop_event) recorded_[l.stop_event] = std::chrono::steady_clock::now();
     std::lock_guard<std::mutex> lock(g_sim.mutex);
     ++g_sim.kernel_launches;
-    if (sk.splits > 1) {
-      ++g_sim.split_launches;
-      if (sk.narrow) ++g_sim.narrow_splits;
-      g_sim.last_splits = sk.splits;
-    }
-    if (ts.head_m > 0) {
-      ++g_sim.tail_splits;
-      g_sim.last_splits = ts.tail.splits;
-    }
     return 0;
+  }
+
+  static void count(const kernels::Route& r) {
+    std::lock_guard<std::mutex> lock(g_sim.mutex);
+    ++g_sim.runs[static_cast<int>(r.run)];
+    if (r.run == kernels::Run::kSmallTiles && r.small.splits > 1) {
+      ++g_sim.small_splits;
+      g_sim.last_splits = r.small.splits;
+    }
+    if (r.split.splits > 1) g_sim.last_splits = r.split.splits;
+    if (r.run == kernels::Run::kTailSplit) g_sim.last_splits = r.tail.tail.splits;
   }
 
   const char* error_name(int code) override {
@@ -498,12 +502,9 @@ extern "C" __attribute__((visibility("default"))) void xvram_hostsim_reset() {
   for (auto& s : g_sim.sites) s = Injection{};
   g_sim.free_bytes = g_sim.total_bytes = 16ull << 30;
   g_sim.kernel_launches = 0;
-  g_sim.split_launches = 0;
-  g_sim.narrow_splits = 0;
+  std::fill(std::begin(g_sim.runs), std::end(g_sim.runs), uint64_t{0});
+  g_sim.small_splits = 0;
   g_sim.last_splits = 0;
-  g_sim.tail_splits = 0;
-  g_sim.edge_splits = 0;
-  g_sim.k_remainders = 0;
   g_sim.device_count = 1;
   g_sim.current_device = 0;
   g_sim.last_init_ordinal = -1;
@@ -534,14 +535,15 @@ extern "C" __attribute__((visibility("default"))) void xvram_hostsim_set_memory(
   g_sim.total_bytes = total_b;
 }
 
-// Launches that split K since the last reset; *last_splits = the K ranges of
-// the last one.
+// Launches that split K over workgroups since the last reset; *last_splits =
+// the K ranges of the last one.
 extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_split_launches(
     int* last_splits) {
   using namespace xvram;
   std::lock_guard<std::mutex> lock(g_sim.mutex);
   if (last_splits != nullptr) *last_splits = g_sim.last_splits;
-  return g_sim.split_launches;
+  return g_sim.small_splits + g_sim.runs[static_cast<int>(kernels::Run::kRingSplit)] +
+         g_sim.runs[static_cast<int>(kernels::Run::kNarrowSplit)];
 }
 
 // The split rule itself (kernels::split_k_shape) for a launch shape: returns
@@ -557,8 +559,6 @@ extern "C" __attribute__((visibility("default"))) int xvram_hostsim_split_shape(
   return sk.splits;
 }
 
-// Of those, the launches whose ranges ran on the 256 x 128 kernel (tiles that
-// are not all interior 256 x 256 ones).
 // The tail split rule (kernels::tail_split_shape) for a launch shape: returns
 // the number of K ranges of the tail (1 = no tail split), *head_m the head's
 // rows and *depth the tail's range depth.
@@ -582,37 +582,14 @@ extern "C" __attribute__((visibility("default"))) int xvram_hostsim_edge_split_s
   return xvram::kernels::edge_split_rated_faster(m, n, k, nt != 0) ? 1 : 0;
 }
 
-// Launches that ran as a rounded K and its remainder since the last reset.
-extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_k_remainder_launches() {
-  using namespace xvram;
-  std::lock_guard<std::mutex> lock(g_sim.mutex);
-  return g_sim.k_remainders;
-}
-
 // The K remainder rule for a launch shape: the rounded K (0: none).
 extern "C" __attribute__((visibility("default"))) int64_t xvram_hostsim_k_remainder_shape(
     int64_t m, int64_t n, int64_t k, int nt) {
   return xvram::kernels::k_remainder_shape(m, n, k, nt != 0);
 }
 
-// The partials' bytes a launch wants (kernels::split_k_bytes_wanted) for a
+// The partials' bytes a launch wants (kernels::launch_bytes_wanted) for a
 // launch of that shape, form and leading dimensions (pointers unused).
-extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_bytes_wanted(
-    int m, int n, int k, int a_kcontig, int b_ncontig, int64_t lda, int64_t ldb) {
-  xvram::kernels::SgemmLaunch l;
-  l.m = m;
-  l.n = n;
-  l.k = k;
-  l.a_kcontig = a_kcontig != 0;
-  l.b_ncontig = b_ncontig != 0;
-  l.lda = lda;
-  l.ldb = ldb;
-  l.ldc = m;
-  return xvram::kernels::split_k_bytes_wanted(l);
-}
-
-// The same as the GPU's launch_sgemm runs the launch
-// (kernels::launch_bytes_wanted).
 extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_launch_bytes_wanted(
     int m, int n, int k, int a_kcontig, int b_ncontig, int64_t lda, int64_t ldb) {
   xvram::kernels::SgemmLaunch l;
@@ -652,24 +629,73 @@ extern "C" __attribute__((visibility("default"))) int xvram_hostsim_kwave_many(
   return p.small.tile;
 }
 
-// Launches that ran as an interior and edge strips since the last reset.
-extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_edge_split_launches() {
+// Launches and parts of launches whose route had that number in kernels::Run
+// since the last reset.
+extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_runs(int run) {
   using namespace xvram;
   std::lock_guard<std::mutex> lock(g_sim.mutex);
-  return g_sim.edge_splits;
+  return run < 0 || run >= kernels::kRunCount ? 0 : g_sim.runs[run];
 }
 
-// Launches that ran as a head and a split tail since the last reset.
-extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_tail_split_launches() {
-  using namespace xvram;
-  std::lock_guard<std::mutex> lock(g_sim.mutex);
-  return g_sim.tail_splits;
+namespace {
+
+std::string route_text(const xvram::kernels::SgemmLaunch& l, bool workspace, uint64_t room) {
+  using namespace xvram::kernels;
+  const auto number = [](int64_t v) { return std::to_string(v); };
+  const Route r = route_with(l, workspace, room);
+  const auto parts = [&](std::string name) {
+    name += "[";
+    for (int i = 0; i < r.count; ++i) {
+      const SgemmLaunch& p = r.part[i];
+      name += (i ? "; " : "") + number(p.m) + "x" + number(p.n) + "x" + number(p.k) + " " +
+              route_text(p, workspace, room);
+    }
+    return name + "]";
+  };
+  switch (r.run) {
+  case Run::kTwoPanel: return "two panels";
+  case Run::kRectangle: return parts("rectangle");
+  case Run::kKRemainder: return parts("k remainder");
+  case Run::kEdgeSplit: return parts("edge split");
+  case Run::kSmallTiles: {
+    const KwaveTile& t = kKwaveTiles[r.small.tile];
+    return "small " + number(32 * t.mb) + "x" + number(32 * t.nb) + " ranges " +
+           number(r.small.splits) + " fold " + number(r.small.fold);
+  }
+  case Run::kThinK: return "thin";
+  case Run::kRingSplit: return "ring split " + number(r.split.splits) + "x" + number(r.split.depth);
+  case Run::kNarrowSplit:
+    return "narrow split " + number(r.split.splits) + "x" + number(r.split.depth);
+  case Run::kTailSplit:
+    return "tail split " + number(r.tail.head_m) + " " + number(r.tail.tail.splits) + "x" +
+           number(r.tail.tail.depth);
+  case Run::kRing: return l.m % 256 == 0 && l.n % 256 == 0 ? "ring" : "edge ring";
+  case Run::kGeneral: return "general";
+  case Run::kNarrow: return "narrow";
+  }
+  return {};
 }
 
-extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_narrow_split_launches() {
-  using namespace xvram;
-  std::lock_guard<std::mutex> lock(g_sim.mutex);
-  return g_sim.narrow_splits;
+} // namespace
+
+// The route of a launch of that shape, form and leading dimensions (pointers
+// unused) with room for `room` bytes of partials (workspace = 0: without one),
+// in words; the text's length.
+extern "C" __attribute__((visibility("default"))) int xvram_hostsim_route(
+    int m, int n, int k, int a_kcontig, int b_ncontig, int64_t lda, int64_t ldb, int workspace,
+    uint64_t room, char* text, int size) {
+  xvram::kernels::SgemmLaunch l;
+  l.m = m;
+  l.n = n;
+  l.k = k;
+  l.a_kcontig = a_kcontig != 0;
+  l.b_ncontig = b_ncontig != 0;
+  l.lda = lda;
+  l.ldb = ldb;
+  l.ldc = m;
+  const std::string t = route_text(l, workspace != 0, workspace != 0 ? room : 0);
+  if (text != nullptr && size > 0) std::snprintf(text, static_cast<size_t>(size), "%s", t.c_str());
+  return static_cast<int>(t.size());
 }
 
 extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_kernel_launches() {

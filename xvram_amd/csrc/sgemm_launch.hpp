@@ -28,7 +28,7 @@
 // interior ranges (ring kernels).
 //
 // Split K (optional, workspace set): a launch that would leave CUs idle may
-// cut its K into ranges (split_k_plan below), one workgroup per tile and
+// cut its K into ranges (split_k_shape below), one workgroup per tile and
 // range; each stores the raw partial sums of its range to the workspace
 // (`splits` column-major m x n matrices, leading dimension m rounded up to 4,
 // split_partial_ld), and a second kernel adds them in range order and applies
@@ -41,7 +41,7 @@
 // is the same from run to run. Without a workspace large enough for two
 // partials the launch runs unsplit. One K panel only. A launch of at least
 // 256 interior tiles whose last round would leave CUs idle may run as a
-// head and a split tail instead (tail_split_plan below).
+// head and a split tail instead (tail_split_shape below).
 //
 // start_event / stop_event (hipEvent_t, optional) are recorded by the dispatch
 // itself (hipExtLaunchKernelGGL): no separate marker packets run between
@@ -159,7 +159,7 @@ inline SplitK split_k_shape(int64_t m, int64_t n, int64_t k, bool nt, bool ring,
   if (interior) {
     // The kernel family follows from the shape alone, not from the
     // workspace: a launch given exactly the workspace its split wants
-    // (split_k_bytes_wanted) takes that same split.
+    // (launch_bytes_wanted) takes that same split.
     const int64_t tiles = (m / 256) * (n / 256);
     const int64_t one_round = std::min(deepest, kComputeUnits / tiles);
     if (one_round < 2) return {};
@@ -196,12 +196,6 @@ inline SplitK split_k_for(const SgemmLaunch& l, uint64_t workspace_bytes) {
   const int64_t b_bytes = (l.b_ncontig ? int64_t{l.k} : int64_t{l.n}) * l.ldb * 4;
   return split_k_shape(l.m, l.n, l.k, !l.a_kcontig && l.b_ncontig,
                        a_bytes < kLimit && b_bytes < kLimit, workspace_bytes);
-}
-
-// The split of one launch with its own 16-byte aligned workspace.
-inline SplitK split_k_plan(const SgemmLaunch& l) {
-  if (l.workspace == nullptr || reinterpret_cast<uintptr_t>(l.workspace) % 16 != 0) return {};
-  return split_k_for(l, l.workspace_bytes);
 }
 
 // K below this runs on a plain kernel (each thread four rows of one column of
@@ -338,12 +332,6 @@ inline KwavePlan kwave_plan_for(const SgemmLaunch& l, uint64_t workspace_bytes) 
   return kwave_plan_shape(l.m, l.n, l.k, !l.a_kcontig && l.b_ncontig, workspace_bytes);
 }
 
-// The plan of one launch with its own 16-byte aligned workspace (or none).
-inline KwavePlan kwave_plan(const SgemmLaunch& l) {
-  const bool usable = l.workspace != nullptr && reinterpret_cast<uintptr_t>(l.workspace) % 16 == 0;
-  return kwave_plan_for(l, usable ? l.workspace_bytes : 0);
-}
-
 // Tail split. A launch of at least kComputeUnits interior 256 x 256 tiles
 // runs in rounds of one workgroup per CU, and a last round that fills few
 // CUs costs as much as a full one (17 x 17 tiles: 2 rounds for 289 tiles).
@@ -412,33 +400,6 @@ inline TailSplit tail_split_for(const SgemmLaunch& l, uint64_t workspace_bytes) 
   const int64_t b_bytes = (l.b_ncontig ? int64_t{l.k} : int64_t{l.n}) * l.ldb * 4;
   return tail_split_shape(l.m, l.n, l.k, !l.a_kcontig && l.b_ncontig,
                           a_bytes < kLimit && b_bytes < kLimit, workspace_bytes);
-}
-
-// The tail split of one launch with its own 16-byte aligned workspace.
-inline TailSplit tail_split_plan(const SgemmLaunch& l) {
-  if (l.workspace == nullptr || reinterpret_cast<uintptr_t>(l.workspace) % 16 != 0) return {};
-  return tail_split_for(l, l.workspace_bytes);
-}
-
-// Bytes of partials a launch's split (or tail split) wants when the
-// workspace is not the limit (0: it does not split).
-inline uint64_t split_k_bytes_wanted_whole(const SgemmLaunch& l) {
-  const SplitK sk = split_k_for(l, ~uint64_t{0});
-  if (sk.splits > 1)
-    return static_cast<uint64_t>(sk.splits) * uint64_t(split_partial_ld(l.m)) * uint64_t(l.n) * 4;
-  const TailSplit ts = tail_split_for(l, ~uint64_t{0});
-  return ts.head_m > 0 ? static_cast<uint64_t>(ts.tail.splits) * uint64_t(l.m - ts.head_m) *
-                             uint64_t(l.n) * 4
-                       : 0;
-}
-
-// The same as launch_sgemm runs a launch without parts.
-inline uint64_t part_bytes_wanted(const SgemmLaunch& l) {
-  const KwavePlan kw = kwave_plan_for(l, ~uint64_t{0});
-  if (kw.tile < 0) return split_k_bytes_wanted_whole(l);
-  return kw.splits > 1
-             ? uint64_t(kw.splits) * uint64_t(split_partial_ld(l.m)) * uint64_t(l.n) * 4
-             : 0;
 }
 
 // Edge split. A launch whose m or n is not a multiple of 256 and that has at
@@ -517,16 +478,6 @@ inline EdgeParts edge_parts_shape(const SgemmLaunch& l) {
   if (mi < l.m) e.part[e.count++] = sub_launch(l, mi, l.m - mi, 0, l.n);
   e.part[0].start_event = l.start_event;
   e.part[e.count - 1].stop_event = l.stop_event;
-  return e;
-}
-
-// The parts of a launch's edge split (count 0: none): by shape, and without a
-// workspace only when no part would split.
-inline EdgeParts edge_parts(const SgemmLaunch& l) {
-  const EdgeParts e = edge_parts_shape(l);
-  if (e.count == 0 || l.workspace != nullptr) return e;
-  for (int i = 0; i < e.count; ++i)
-    if (part_bytes_wanted(e.part[i]) > 0) return {};
   return e;
 }
 
@@ -725,45 +676,119 @@ inline KParts k_remainder_parts_shape(const SgemmLaunch& l) {
   return r;
 }
 
-// Bytes of partials a launch wants when the workspace is not the limit: the
-// first part's of a K remainder; else the most any part of its edge split
-// wants (they run one after another on the stream, so they share it); else
-// its own split's (0: it does not split).
-inline uint64_t split_k_bytes_wanted(const SgemmLaunch& l) {
-  const KParts kp = k_remainder_parts_shape(l);
-  const SgemmLaunch& base = kp.count > 0 ? kp.part[0] : l;
-  const EdgeParts e = edge_parts_shape(base);
-  if (e.count == 0) return split_k_bytes_wanted_whole(base);
-  uint64_t most = 0;
-  for (int i = 0; i < e.count; ++i) most = std::max(most, split_k_bytes_wanted_whole(e.part[i]));
-  return most;
-}
+// How a launch runs: on one kernel, as head and tail, or as parts of its own.
+enum class Run {
+  kTwoPanel,   // ring kernels' two-panel instances
+  kRectangle,  // parts: whole rounds of interior tiles, right strip, bottom strip (many_parts)
+  kKRemainder, // parts: the rounded K, the rest (k_remainder_parts_shape)
+  kEdgeSplit,  // parts: interior tiles, right strip, bottom strip (edge_parts_shape)
+  kSmallTiles, // `small`
+  kThinK,      // thin_k_kernel
+  kRingSplit,  // `split` on the ring kernels
+  kNarrowSplit, // `split` on the 256 x 128 kernel
+  kTailSplit,  // `tail`
+  kRing,       // ring kernels, interior or edge instances
+  kGeneral,    // sgemm_wide_kernel
+  kNarrow,     // 256 x 128 kernel
+};
+constexpr int kRunCount = static_cast<int>(Run::kNarrow) + 1;
 
-// Bytes of partials one launch wants when the workspace is not the limit, as
-// launch_sgemm runs it: its own, or the most that any of its parts wants (they
-// share the workspace in turn).
-inline uint64_t launch_bytes_wanted(const SgemmLaunch& l) {
-  const auto most = [](const SgemmLaunch* parts, int count) {
-    uint64_t bytes = 0;
-    for (int i = 0; i < count; ++i) bytes = std::max(bytes, launch_bytes_wanted(parts[i]));
-    return bytes;
+struct Route {
+  Run run = Run::kNarrow;
+  KwavePlan small;
+  SplitK split;
+  TailSplit tail;
+  int count = 0; // parts, run one after another
+  SgemmLaunch part[3];
+};
+
+inline uint64_t launch_bytes_wanted(const SgemmLaunch& l);
+
+// The route of a launch whose operands and workspace are aligned, given room
+// for `room` bytes of partials; `workspace` = it has any (without one a K
+// remainder or edge split is taken only where its parts would not split).
+inline Route route_with(const SgemmLaunch& l, bool workspace, uint64_t room) {
+  constexpr int64_t kLimit = int64_t(1) << 31;
+  Route r;
+  const auto parts = [&](Run run, const SgemmLaunch* part, int count) {
+    r.run = run;
+    r.count = count;
+    std::copy(part, part + count, r.part);
   };
-  if (const ManyPlan mp = many_plan(l); mp.small.tile >= 0) return 0;
-  else if (mp.mi > 0) {
-    const EdgeParts e = many_parts(l, mp);
-    return most(e.part, e.count);
+  if (l.a2 != nullptr || l.b2 != nullptr) {
+    r.run = Run::kTwoPanel;
+    return r;
   }
-  if (const KParts kp = k_remainder_parts_shape(l); kp.count > 0) return most(kp.part, 1);
-  if (const EdgeParts e = edge_parts_shape(l); e.count > 0) return most(e.part, e.count);
-  return part_bytes_wanted(l);
+  if (const ManyPlan mp = many_plan(l); mp.small.tile >= 0) {
+    r.run = Run::kSmallTiles;
+    r.small = mp.small;
+    return r;
+  } else if (mp.mi > 0) {
+    const EdgeParts e = many_parts(l, mp);
+    parts(Run::kRectangle, e.part, e.count);
+    return r;
+  }
+  if (const KParts kp = k_remainder_parts_shape(l);
+      kp.count > 0 && (workspace || launch_bytes_wanted(kp.part[0]) == 0)) {
+    parts(Run::kKRemainder, kp.part, kp.count);
+    return r;
+  }
+  if (const EdgeParts e = edge_parts_shape(l); e.count > 0) {
+    // A part with parts of its own does without a workspace.
+    bool alone = true;
+    for (int i = 0; i < e.count && !workspace; ++i)
+      alone = alone && (route_with(e.part[i], true, ~uint64_t{0}).count > 0 ||
+                        launch_bytes_wanted(e.part[i]) == 0);
+    if (alone) {
+      parts(Run::kEdgeSplit, e.part, e.count);
+      return r;
+    }
+  }
+  if (l.k < kThinK) {
+    r.run = Run::kThinK;
+    return r;
+  }
+  if (r.small = kwave_plan_for(l, room); r.small.tile >= 0) {
+    r.run = Run::kSmallTiles;
+    return r;
+  }
+  if (r.split = split_k_for(l, room); r.split.splits > 1) {
+    r.run = r.split.narrow ? Run::kNarrowSplit : Run::kRingSplit;
+    return r;
+  }
+  if (r.tail = tail_split_for(l, room); r.tail.head_m > 0) {
+    r.run = Run::kTailSplit;
+    return r;
+  }
+  const int64_t tiles = ((int64_t{l.m} + 255) / 256) * ((int64_t{l.n} + 255) / 256);
+  const int64_t a_bytes = (l.a_kcontig ? int64_t{l.m} : int64_t{l.k}) * l.lda * 4;
+  const int64_t b_bytes = (l.b_ncontig ? int64_t{l.k} : int64_t{l.n}) * l.ldb * 4;
+  if (tiles >= kComputeUnits && a_bytes < kLimit && b_bytes < kLimit)
+    r.run = l.k % (!l.a_kcontig && l.b_ncontig ? 4 : 8) == 0 ? Run::kRing : Run::kGeneral;
+  return r;
 }
 
-// The two launches of a K remainder (count 0: none): by shape, and without a
-// workspace only when the first part would not split.
-inline KParts k_remainder_parts(const SgemmLaunch& l) {
-  const KParts kp = k_remainder_parts_shape(l);
-  if (kp.count == 0 || l.workspace != nullptr || launch_bytes_wanted(kp.part[0]) == 0) return kp;
-  return {};
+// The route of a launch with its own workspace (or none).
+inline Route route(const SgemmLaunch& l) {
+  const bool usable = l.workspace != nullptr && reinterpret_cast<uintptr_t>(l.workspace) % 16 == 0;
+  return route_with(l, l.workspace != nullptr, usable ? l.workspace_bytes : 0);
+}
+
+// Bytes of partials one launch wants when the workspace is not the limit: its
+// own, or the most that any of its parts wants (they share the workspace in
+// turn).
+inline uint64_t launch_bytes_wanted(const SgemmLaunch& l) {
+  const Route r = route_with(l, true, ~uint64_t{0});
+  const auto partials = [](int splits, int64_t m, int64_t n) {
+    return uint64_t(splits) * uint64_t(split_partial_ld(m)) * uint64_t(n) * 4;
+  };
+  uint64_t bytes = 0;
+  for (int i = 0; i < r.count; ++i) bytes = std::max(bytes, launch_bytes_wanted(r.part[i]));
+  if (r.run == Run::kSmallTiles && r.small.splits > 1) bytes = partials(r.small.splits, l.m, l.n);
+  if (r.run == Run::kRingSplit || r.run == Run::kNarrowSplit)
+    bytes = partials(r.split.splits, l.m, l.n);
+  if (r.run == Run::kTailSplit) bytes = partials(r.tail.tail.splits, l.m - r.tail.head_m, l.n);
+  return bytes;
 }
 
 // Whether a plan's m x n x k launch of form `nt` would take a K remainder

@@ -289,23 +289,6 @@ hipError_t launch_variant(const Params& p, hipStream_t stream, hipEvent_t start,
 
 } // namespace
 
-// A launch with at least this many 256 x 256 tiles (one per CU of the chip)
-// runs a 256 x 256 kernel (sgemm_wide.hip picks a barrier-free one for
-// launches of interior tiles); smaller ones run on smaller tiles
-// (sgemm_kwave.hip), or, with panels that those cannot address, here.
-constexpr int64_t kWideMinTiles = 256;
-
-// The 256 x 256 kernels address each operand panel with 32-bit buffer
-// offsets, so every panel must span less than 2^31 bytes.
-bool wide_fits(const SgemmLaunch& l) {
-  constexpr int64_t kLimit = int64_t(1) << 31;
-  const int64_t t = wide_tile();
-  const int64_t tiles = ((l.m + t - 1) / t) * ((l.n + t - 1) / t);
-  const int64_t a_bytes = (l.a_kcontig ? (int64_t)l.m : (int64_t)l.k) * l.lda * 4;
-  const int64_t b_bytes = (l.b_ncontig ? (int64_t)l.k : (int64_t)l.n) * l.ldb * 4;
-  return tiles >= kWideMinTiles && a_bytes < kLimit && b_bytes < kLimit;
-}
-
 int launch_sgemm(const SgemmLaunch& launch, void* stream) {
   const bool aligned =
       (reinterpret_cast<uintptr_t>(launch.a) % 16 == 0) &&
@@ -343,107 +326,76 @@ int launch_sgemm(const SgemmLaunch& launch, void* stream) {
   auto* s = static_cast<hipStream_t>(stream);
   auto* e0 = static_cast<hipEvent_t>(launch.start_event);
   auto* e1 = static_cast<hipEvent_t>(launch.stop_event);
-  // Many 256 x 256 tiles: smaller ones where they run faster, or whole rounds of
-  // them and the rest on smaller ones (sgemm_launch.hpp).
-  if (const ManyPlan mp = many_plan(launch); mp.small.tile >= 0) {
-    return static_cast<int>(
-        launch_kwave(p, mp.small, launch.a_kcontig, launch.b_ncontig, s, e0, e1));
-  } else if (mp.mi > 0) {
-    const EdgeParts e = many_parts(launch, mp);
-    for (int i = 0; i < e.count; ++i)
-      if (const int rc = launch_sgemm(e.part[i], stream); rc != 0) return rc;
+  const Route r = route(launch);
+  p.tiles_m = (launch.m + wide_tile() - 1) / wide_tile();
+  p.tiles_n = (launch.n + wide_tile() - 1) / wide_tile();
+  if (r.run != Run::kTwoPanel) p.k_split = 0;
+  switch (r.run) {
+  case Run::kRectangle:
+  case Run::kKRemainder:
+  case Run::kEdgeSplit:
+    for (int i = 0; i < r.count; ++i)
+      if (const int rc = launch_sgemm(r.part[i], stream); rc != 0) return rc;
     return 0;
-  }
-  // K not a multiple of the ring kernels' step where a tail or edge split
-  // would pay: the rounded K, then the rest (sgemm_launch.hpp).
-  if (const KParts kp = k_remainder_parts(launch); kp.count > 0) {
-    for (int i = 0; i < kp.count; ++i)
-      if (const int rc = launch_sgemm(kp.part[i], stream); rc != 0) return rc;
-    return 0;
-  }
-  // Ragged m or n over many tiles: the interior and the edge strips as
-  // launches of their own (sgemm_launch.hpp), one after another.
-  if (const EdgeParts e = edge_parts(launch); e.count > 0) {
-    for (int i = 0; i < e.count; ++i)
-      if (const int rc = launch_sgemm(e.part[i], stream); rc != 0) return rc;
-    return 0;
-  }
-  if (launch.a2 != nullptr || launch.b2 != nullptr) {
-    // Two K panels: the barrier-free kernels only.
+  case Run::kTwoPanel:
     if (!two_panel_valid(launch)) return static_cast<int>(hipErrorInvalidValue);
-    p.tiles_m = launch.m / wide_tile();
-    p.tiles_n = launch.n / wide_tile();
     return static_cast<int>(launch_wide(p, launch.a_kcontig, launch.b_ncontig, s, e0, e1));
-  }
-  p.k_split = 0;
-  // K below 8: no MFMA tiles (sgemm_wide.hip, thin_k_kernel).
-  if (launch.k < kThinK)
+  case Run::kThinK:
     return static_cast<int>(launch_thin_k(p, launch.a_kcontig, launch.b_ncontig, s, e0, e1));
-  // Fewer 256 x 256 tiles than CUs: smaller tiles whose K the waves share
-  // (sgemm_launch.hpp, kwave_plan_shape).
-  if (const KwavePlan kw = kwave_plan(launch); kw.tile >= 0) {
+  case Run::kSmallTiles:
     p.partial = launch.workspace;
-    return static_cast<int>(launch_kwave(p, kw, launch.a_kcontig, launch.b_ncontig, s, e0, e1));
-  }
-  // Fewer tiles than workgroup slots: split K when a workspace is given
-  // (fixed-order reduction; sgemm_launch.hpp), on the ring kernels for
-  // interior 256 x 256 tiles, else on the 256 x 128 kernel.
-  if (const SplitK sk = split_k_plan(launch); sk.splits > 1) {
-    p.splits = sk.splits;
-    p.split_depth = sk.depth;
+    return static_cast<int>(
+        launch_kwave(p, r.small, launch.a_kcontig, launch.b_ncontig, s, e0, e1));
+  case Run::kRingSplit:
+    p.splits = r.split.splits;
+    p.split_depth = r.split.depth;
     p.partial = launch.workspace;
-    if (!sk.narrow) {
-      p.tiles_m = launch.m / wide_tile();
-      p.tiles_n = launch.n / wide_tile();
-      return static_cast<int>(launch_wide(p, launch.a_kcontig, launch.b_ncontig, s, e0, e1));
-    }
-    p.tiles_m = (launch.m + kTileM - 1) / kTileM;
-    p.tiles_n = (launch.n + kTileN - 1) / kTileN;
-    hipError_t err;
-    if (!launch.a_kcontig && !launch.b_ncontig) err = launch_variant<false, false>(p, s, e0, nullptr);
-    else if (!launch.a_kcontig && launch.b_ncontig) err = launch_variant<false, true>(p, s, e0, nullptr);
-    else if (launch.a_kcontig && !launch.b_ncontig) err = launch_variant<true, false>(p, s, e0, nullptr);
-    else err = launch_variant<true, true>(p, s, e0, nullptr);
-    if (err != hipSuccess) return static_cast<int>(err);
-    return static_cast<int>(launch_splitk_reduce(p, s, e1));
-  }
-  // A last round of 256 x 256 tiles that would fill few CUs: the head's
-  // tile rows unsplit, then the tail's rows split (sgemm_launch.hpp); the
-  // start event rides on the head's dispatch, the stop event on the tail's
-  // reduction.
-  if (const TailSplit ts = tail_split_plan(launch); ts.head_m > 0) {
+    return static_cast<int>(launch_wide(p, launch.a_kcontig, launch.b_ncontig, s, e0, e1));
+  case Run::kTailSplit: {
+    // The start event rides on the head's dispatch, the stop event on the
+    // tail's reduction.
+    const int head_m = static_cast<int>(r.tail.head_m);
     Params head = p;
-    head.m = static_cast<int>(ts.head_m);
-    head.tiles_m = static_cast<int>(ts.head_m / wide_tile());
-    head.tiles_n = launch.n / wide_tile();
+    head.m = head_m;
+    head.tiles_m = head_m / wide_tile();
     if (const hipError_t e = launch_wide(head, launch.a_kcontig, launch.b_ncontig, s, e0, nullptr);
         e != hipSuccess)
       return static_cast<int>(e);
     Params tail = p;
-    tail.a = launch.a_kcontig ? launch.a + ts.head_m * launch.lda : launch.a + ts.head_m;
-    tail.c = launch.c + ts.head_m;
-    if (tail.bias_row != nullptr) tail.bias_row += ts.head_m;
-    tail.m = launch.m - static_cast<int>(ts.head_m);
+    tail.a = launch.a_kcontig ? launch.a + head_m * launch.lda : launch.a + head_m;
+    tail.c = launch.c + head_m;
+    if (tail.bias_row != nullptr) tail.bias_row += head_m;
+    tail.m = launch.m - head_m;
     tail.tiles_m = tail.m / wide_tile();
-    tail.tiles_n = launch.n / wide_tile();
-    tail.splits = ts.tail.splits;
-    tail.split_depth = ts.tail.depth;
+    tail.splits = r.tail.tail.splits;
+    tail.split_depth = r.tail.tail.depth;
     tail.partial = launch.workspace;
     return static_cast<int>(launch_wide(tail, launch.a_kcontig, launch.b_ncontig, s, nullptr, e1));
   }
-  if (wide_fits(launch)) {
-    p.tiles_m = (launch.m + wide_tile() - 1) / wide_tile();
-    p.tiles_n = (launch.n + wide_tile() - 1) / wide_tile();
+  case Run::kRing:
+  case Run::kGeneral:
     return static_cast<int>(launch_wide(p, launch.a_kcontig, launch.b_ncontig, s, e0, e1));
+  case Run::kNarrowSplit:
+  case Run::kNarrow:
+    break;
   }
+  // The 256 x 128 kernel, its K split or not.
+  const bool split = r.run == Run::kNarrowSplit;
+  if (split) {
+    p.splits = r.split.splits;
+    p.split_depth = r.split.depth;
+    p.partial = launch.workspace;
+  }
+  const hipEvent_t last = split ? nullptr : e1;
   p.tiles_m = (launch.m + kTileM - 1) / kTileM;
   p.tiles_n = (launch.n + kTileN - 1) / kTileN;
   hipError_t err;
-  if (!launch.a_kcontig && !launch.b_ncontig) err = launch_variant<false, false>(p, s, e0, e1);
-  else if (!launch.a_kcontig && launch.b_ncontig) err = launch_variant<false, true>(p, s, e0, e1);
-  else if (launch.a_kcontig && !launch.b_ncontig) err = launch_variant<true, false>(p, s, e0, e1);
-  else err = launch_variant<true, true>(p, s, e0, e1);
-  return static_cast<int>(err);
+  if (!launch.a_kcontig && !launch.b_ncontig) err = launch_variant<false, false>(p, s, e0, last);
+  else if (!launch.a_kcontig && launch.b_ncontig) err = launch_variant<false, true>(p, s, e0, last);
+  else if (launch.a_kcontig && !launch.b_ncontig) err = launch_variant<true, false>(p, s, e0, last);
+  else err = launch_variant<true, true>(p, s, e0, last);
+  if (err != hipSuccess || !split) return static_cast<int>(err);
+  return static_cast<int>(launch_splitk_reduce(p, s, e1));
 }
 
 } // namespace xvram::kernels

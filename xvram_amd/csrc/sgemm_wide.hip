@@ -1022,7 +1022,7 @@ hipError_t launch_wide(const Params& p, bool a_kcontig, bool b_ncontig, hipStrea
                        hipEvent_t start, hipEvent_t stop) {
   const dim3 block(kThreads);
   if (p.splits > 1) {
-    // Split K (the caller has checked split_k_plan's conditions): the ring
+    // Split K (the caller has checked split_k_shape's conditions): the ring
     // kernel over tiles x ranges into the partials, then the reduction; the
     // start event rides on the first dispatch, the stop event on the second.
     const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n * p.splits));
