@@ -13,6 +13,7 @@ import pytest
 import xvram_amd as xv
 from xvram_amd import abi
 
+from gemm_cases import route
 from test_gpu_sgemm_device import FORMS, Hip, desc_for
 
 pytestmark = pytest.mark.gpu
@@ -88,6 +89,21 @@ MANY = [
 ]
 
 
+# Launches of many tiles whose sums may not be added in longer chains than the
+# large kernels' rules add them in, and how they run.
+BOUNDED = [
+    ((4762, 5194, 1208), "rectangle[4096x4096x608 ring; 4096x4096x600 ring; 4096x1098x1208 small"),
+    ((2304, 8512, 2080), "small 64x64 ranges 1 fold 320 edge 32"),
+]
+
+
+@pytest.mark.parametrize("form", sorted(FORMS))
+@pytest.mark.parametrize("shape,how", BOUNDED, ids=["x".join(map(str, c[0])) for c in BOUNDED])
+def test_bounded_chains(lib, hip, oracle_mod, shape, how, form):
+    assert route(*shape, form).startswith(how)
+    check(lib, hip, oracle_mod, shape, form)
+
+
 @pytest.mark.parametrize("form", sorted(FORMS))
 @pytest.mark.parametrize("shape,want,want_nt", CASES + MANY,
                          ids=["x".join(map(str, c[0])) for c in CASES + MANY])
@@ -96,6 +112,12 @@ def test_tile(lib, hip, oracle_mod, shape, want, want_nt, form):
     rule = many if -(-m // 256) * -(-n // 256) >= 256 else plan
     tile, splits, fold = rule(m, n, k, form)
     assert (tile, splits > 1, 0 < fold < 1 << 27) == (want_nt if want_nt and form == "NT" else want)
+    print(f"[kwave] tile {tile}, {splits} ranges, fold {fold}", flush=True)
+    check(lib, hip, oracle_mod, shape, form)
+
+
+def check(lib, hip, oracle_mod, shape, form):
+    m, n, k = shape
     ops = FORMS[form]
     seed = m + 3 * n + 7 * k
     bias_axis = abi.BIAS_PER_ROW if (m + n) % 2 else abi.BIAS_PER_COLUMN
@@ -107,7 +129,7 @@ def test_tile(lib, hip, oracle_mod, shape, want, want_nt, form):
     fa, lda = padded_nan(a if ops[0] == abi.OP_N else a.T, 4)
     fb, ldb = padded_nan(b if ops[1] == abi.OP_N else b.T, 0)
     fc, ldc = padded_nan(c0, 8)
-    print(f"[kwave] {form} {shape} tile {tile}, {splits} ranges, fold {fold}", flush=True)
+    print(f"[kwave] {form} {shape}: {route(m, n, k, form)}", flush=True)
     ptrs = [hip.alloc(x.nbytes) for x in (fa, fb, fc, bias)]
     s = hip.stream()
     outs = []

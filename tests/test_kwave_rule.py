@@ -12,6 +12,8 @@ import numpy as np
 
 import xvram_amd as xv
 
+from gemm_cases import route
+
 ANY = (1 << 64) - 1
 RUN = (32, 32, 32, 32, 128, 0, 0)
 
@@ -109,6 +111,48 @@ def test_many_tiles():
             assert 20 * groups >= 19 * -(-groups // 256) * 256
             assert k >= 1024 and k % (4 if nt else 8) == 0
     assert small > 100 and rect > 30
+
+
+def test_no_chain_is_longer_than_the_large_kernels_make_it():
+    """Over seeded launches of 256 tiles and more, elements at the corners, on both
+    sides of the interior's edges and anywhere: small tiles, rectangles and strips
+    add no more k values in one accumulator than the rules of the large kernels
+    alone would for that element (a split tail's ranges, an edge strip's)."""
+    dll = fns()
+    fn = dll.xvram_hostsim_longest_chain
+    fn.restype = ctypes.c_int64
+    fn.argtypes = [ctypes.c_int] * 5 + [ctypes.c_int64] * 4 + [ctypes.c_int]
+    rng = np.random.default_rng(53)
+    rect = passes = edges = 0
+    for _ in range(6000):
+        m, n = (int(2 ** v) for v in rng.uniform(10, 14, 2))
+        k = int(2 ** rng.uniform(8, 13))
+        if rng.random() < 0.5:
+            k = k // 8 * 8
+        if rng.random() < 0.3:
+            m, n = m // 256 * 256, n // 256 * 256
+        if -(-m // 256) * -(-n // 256) < 256:
+            continue
+        form = ("NN", "NT", "TN", "TT")[int(rng.integers(0, 4))]
+        ak, bn = form[0] == "T", form[1] == "T"
+        lda, ldb = ((k if ak else m) + 3) // 4 * 4, ((n if bn else k) + 3) // 4 * 4
+        how = route(m, n, k, form)
+        rect += how.startswith("rectangle")
+        first = how[10:].split(";") if how.startswith("rectangle") else ["", ""]
+        passes += len(first) > 1 and first[0].split("x")[:2] == first[1].strip().split("x")[:2]
+        edges += " edge " in how and "edge split" not in how
+        rows = {0, m - 1, m // 256 * 256 - 1, *(int(v) for v in rng.integers(0, m, 4))}
+        cols = {0, n - 1, n // 256 * 256 - 1, *(int(v) for v in rng.integers(0, n, 4))}
+        for i in rows:
+            for j in cols:
+                now, before = (fn(m, n, k, ak, bn, lda, ldb, i, j, large) for large in (0, 1))
+                assert now <= before, (m, n, k, form, i, j, now, before, how)
+    assert rect > 100 and passes > 20 and edges > 100, (rect, passes, edges)
+    # The rectangle reaches past the head of the rules' tail split (13 of its 16 tile
+    # rows), whose tail's ranges are 2528 deep: two passes.
+    assert route(5000, 5000, 5000, "TT").startswith("rectangle[4096x4096x2528 ring; 4096x4096x2472 ring;")
+    # Rows that lie in a tail of 320-deep ranges.
+    assert fn(2304, 8512, 2080, 0, 0, 2304, 2080, 1800, 0, 0) <= 320
 
 
 def test_partials_fit_the_scratch():

@@ -660,7 +660,8 @@ std::string route_text(const xvram::kernels::SgemmLaunch& l, bool workspace, uin
   case Run::kSmallTiles: {
     const KwaveTile& t = kKwaveTiles[r.small.tile];
     return "small " + number(32 * t.mb) + "x" + number(32 * t.nb) + " ranges " +
-           number(r.small.splits) + " fold " + number(r.small.fold);
+           number(r.small.splits) + " fold " + number(r.small.fold) +
+           (r.small.edge_fold == r.small.fold ? "" : " edge " + number(r.small.edge_fold));
   }
   case Run::kThinK: return "thin";
   case Run::kRingSplit: return "ring split " + number(r.split.splits) + "x" + number(r.split.depth);
@@ -674,6 +675,58 @@ std::string route_text(const xvram::kernels::SgemmLaunch& l, bool workspace, uin
   case Run::kNarrow: return "narrow";
   }
   return {};
+}
+
+// The part of a launch's parts that holds element (i, j) of its C, made
+// relative to that part (rows and columns told from the parts' extents).
+const xvram::kernels::SgemmLaunch& part_of(const xvram::kernels::SgemmLaunch* part, int count,
+                                           int64_t& i, int64_t& j) {
+  const auto& first = part[0];
+  int at = 0;
+  if (i >= first.m) {
+    i -= first.m;
+    at = count - 1; // the bottom strip
+  } else if (j >= first.n) {
+    j -= first.n;
+    for (at = 1; part[at].m == first.m && part[at].n == first.n; ++at) {
+    } // past a rectangle's passes: the right strip
+  }
+  return part[at];
+}
+
+// The most k values one accumulator adds in a row for element (i, j) of a
+// launch on its route, or by the rules of the large kernels alone.
+int64_t longest_chain(const xvram::kernels::SgemmLaunch& l, int64_t i, int64_t j, bool large) {
+  using namespace xvram::kernels;
+  constexpr uint64_t kAny = ~uint64_t{0};
+  const auto tail_chain = [&](const TailSplit& ts) {
+    return ts.head_m > 0 && i >= ts.head_m ? int64_t{ts.tail.depth} : int64_t{l.k};
+  };
+  if (large) {
+    if (const KParts kp = k_remainder_parts_shape(l); kp.count > 0)
+      return longest_chain(kp.part[0], i, j, true);
+    if (const EdgeParts e = edge_parts_shape(l); e.count > 0)
+      return longest_chain(part_of(e.part, e.count, i, j), i, j, true);
+    if (const SplitK sk = split_k_for(l, kAny); sk.splits > 1) return sk.depth;
+    return tail_chain(tail_split_for(l, kAny));
+  }
+  const Route r = route_with(l, true, kAny);
+  switch (r.run) {
+  case Run::kKRemainder: return longest_chain(r.part[0], i, j, false);
+  case Run::kRectangle:
+  case Run::kEdgeSplit: return longest_chain(part_of(r.part, r.count, i, j), i, j, false);
+  case Run::kRingSplit:
+  case Run::kNarrowSplit: return r.split.depth;
+  case Run::kTailSplit: return tail_chain(r.tail);
+  case Run::kSmallTiles: {
+    const KwaveTile& t = kKwaveTiles[r.small.tile];
+    const int64_t row_end = (i / (32 * t.mb) + 1) * 32 * t.mb, col_end = (j / (32 * t.nb) + 1) * 32 * t.nb;
+    const int fold = row_end <= r.small.rows && col_end <= r.small.cols ? r.small.fold : r.small.edge_fold;
+    const int64_t quarter = ((r.small.splits > 1 ? r.small.depth : l.k) + 3) / 4;
+    return fold > 0 ? std::min<int64_t>(fold, quarter) : quarter;
+  }
+  default: return l.k;
+  }
 }
 
 } // namespace
@@ -696,6 +749,24 @@ extern "C" __attribute__((visibility("default"))) int xvram_hostsim_route(
   const std::string t = route_text(l, workspace != 0, workspace != 0 ? room : 0);
   if (text != nullptr && size > 0) std::snprintf(text, static_cast<size_t>(size), "%s", t.c_str());
   return static_cast<int>(t.size());
+}
+
+// The most k values one accumulator adds in a row for element (i, j) of a
+// launch of that shape and form: on its route, or (large = 1) by the rules of
+// the large kernels alone.
+extern "C" __attribute__((visibility("default"))) int64_t xvram_hostsim_longest_chain(
+    int m, int n, int k, int a_kcontig, int b_ncontig, int64_t lda, int64_t ldb, int64_t i,
+    int64_t j, int large) {
+  xvram::kernels::SgemmLaunch l;
+  l.m = m;
+  l.n = n;
+  l.k = k;
+  l.a_kcontig = a_kcontig != 0;
+  l.b_ncontig = b_ncontig != 0;
+  l.lda = lda;
+  l.ldb = ldb;
+  l.ldc = m;
+  return longest_chain(l, i, j, large != 0);
 }
 
 extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_kernel_launches() {

@@ -30,9 +30,9 @@
 //     partials, splitk_reduce_kernel adds them), which the rule in
 //     sgemm_launch.hpp takes when the tiles alone do not fill the chip.
 //   * Precision: the sum of an element is cut into at least four chains (one a
-//     wave). Where the earlier rule's K ranges were shorter than a wave's
-//     quarter, the wave adds its accumulators into a second set every `fold` k
-//     values, so no chain is longer than it was there.
+//     wave). Where the large kernels' rules would cut the element's K into
+//     shorter ranges than a wave's quarter, the wave adds its accumulators into
+//     a second set every so many k values, so no chain is longer than there.
 //
 // Measured on device memory, before (256 x 128 tiles and split K) -> now, us a
 // launch: 1024^3 41.7 -> 20.0; 128^3 15.8 -> 3.6; 3001 x 2047 x 4099 T/N 474 ->
@@ -60,6 +60,12 @@ using namespace device;
 
 constexpr int kThreads = 256;
 constexpr int kWaves = 4;
+
+// k values of one wave between folds, of tiles inside rows [0, rows) x columns
+// [0, cols) and of the others (a tile cut by m or n among them).
+struct Folds {
+  int inside, edge, rows, cols;
+};
 
 template <int N> using Int = std::integral_constant<int, N>;
 
@@ -118,7 +124,7 @@ __device__ __forceinline__ int piece_place(int lrow, int g) {
 // of the slot whose last fragments are in registers, and in its middle it reads
 // the next step's fragments (after waiting for their slot when it is a new one).
 template <bool kAKC, bool kBKC, int MB, int NB, int KP, int R, int kPerCu, bool kFold>
-__global__ __launch_bounds__(kThreads, kPerCu) void sgemm_kwave_kernel(Params p, int fold) {
+__global__ __launch_bounds__(kThreads, kPerCu) void sgemm_kwave_kernel(Params p, Folds folds) {
   constexpr int TM = 32 * MB, TN = 32 * NB;
   constexpr int kGroup = MB + NB;         // wave loads of 1 KiB per 8 k values
   constexpr int kLoads = kGroup * KP;     // ... per slot
@@ -344,7 +350,8 @@ __global__ __launch_bounds__(kThreads, kPerCu) void sgemm_kwave_kernel(Params p,
         }(std::make_integer_sequence<int, kUnroll>{});
       }
     };
-    const int run = fold / kSlotK; // slots per run: a multiple of kUnroll
+    // Slots per run: a multiple of kUnroll.
+    const int run = (m0 + TM <= folds.rows && n0 + TN <= folds.cols ? folds.inside : folds.edge) / kSlotK;
     int from = 0;                  // first slot of the current run
     if constexpr (kFold) {
       for (int to = run - kUnroll; ; to += run) {
@@ -437,11 +444,11 @@ __global__ __launch_bounds__(kThreads, kPerCu) void sgemm_kwave_kernel(Params p,
 }
 
 template <bool AK, bool BK>
-hipError_t launch_form(const Params& p, int tile, int fold, hipStream_t s, hipEvent_t e0,
+hipError_t launch_form(const Params& p, int tile, const Folds& folds, hipStream_t s, hipEvent_t e0,
                        hipEvent_t e1) {
   const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n * p.splits)), block(kThreads);
   const auto go = [&](auto kernel) {
-    hipExtLaunchKernelGGL(kernel, grid, block, 0, s, e0, e1, 0, p, fold);
+    hipExtLaunchKernelGGL(kernel, grid, block, 0, s, e0, e1, 0, p, folds);
     return hipGetLastError();
   };
   // kKwaveTiles (sgemm_launch.hpp) in its order.
@@ -474,12 +481,14 @@ hipError_t launch_kwave(const Params& p0, const KwavePlan& plan, bool a_kcontig,
   p.tiles_n = (p.n + 32 * t.nb - 1) / (32 * t.nb);
   p.splits = plan.splits;
   p.split_depth = plan.depth;
+  // Where all fold alike, tiles cut by m or n do too.
+  const Folds folds{plan.fold, plan.edge_fold, static_cast<int>(plan.rows), static_cast<int>(plan.cols)};
   hipEvent_t last = p.splits > 1 ? nullptr : stop;
   hipError_t e;
-  if (!a_kcontig && !b_ncontig) e = launch_form<false, true>(p, plan.tile, plan.fold, stream, start, last);
-  else if (!a_kcontig && b_ncontig) e = launch_form<false, false>(p, plan.tile, plan.fold, stream, start, last);
-  else if (a_kcontig && !b_ncontig) e = launch_form<true, true>(p, plan.tile, plan.fold, stream, start, last);
-  else e = launch_form<true, false>(p, plan.tile, plan.fold, stream, start, last);
+  if (!a_kcontig && !b_ncontig) e = launch_form<false, true>(p, plan.tile, folds, stream, start, last);
+  else if (!a_kcontig && b_ncontig) e = launch_form<false, false>(p, plan.tile, folds, stream, start, last);
+  else if (a_kcontig && !b_ncontig) e = launch_form<true, true>(p, plan.tile, folds, stream, start, last);
+  else e = launch_form<true, false>(p, plan.tile, folds, stream, start, last);
   if (e != hipSuccess || p.splits <= 1) return e;
   return launch_splitk_reduce(p, stream, stop);
 }

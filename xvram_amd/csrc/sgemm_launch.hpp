@@ -56,6 +56,13 @@
 
 namespace xvram::kernels {
 
+// The most k values one accumulator may add in a row (0: as a launch's own rules
+// have it): `inside` for the elements of rows [0, rows) and columns [0, cols),
+// `edge` for the others.
+struct ChainBound {
+  int64_t inside = 0, edge = 0, rows = 0, cols = 0;
+};
+
 struct SgemmLaunch {
   const float* a = nullptr;
   const float* b = nullptr;
@@ -76,6 +83,8 @@ struct SgemmLaunch {
   void* stop_event = nullptr;
   float* workspace = nullptr; // split-K partials (16-byte aligned), nullptr = none
   uint64_t workspace_bytes = 0;
+  ChainBound bound;   // of a part of another launch
+  bool whole = false; // interior tiles that run unsplit on the ring kernels, also few of them
 };
 
 // MI355X: 256 compute units; a launch with fewer tiles than this leaves CUs
@@ -202,6 +211,9 @@ inline SplitK split_k_for(const SgemmLaunch& l, uint64_t workspace_bytes) {
 // C), not the MFMA tiles: a K remainder's last 1-7 rows, or any such launch.
 constexpr int kThinK = 8;
 
+// Launches over parts of K that one rectangle may run as (many_shape).
+constexpr int64_t kMaxPasses = 4;
+
 // Tiles whose K the waves share (sgemm_kwave.hip). A one-panel launch of K >= 8
 // with fewer than kComputeUnits tiles of 256 x 256 runs on one of these,
 // unsplit or with its K split over workgroups, whichever combination the model
@@ -243,23 +255,28 @@ struct KwavePlan {
   int tile = -1;  // index in kKwaveTiles; -1 = not on these
   int splits = 1; // K ranges over workgroups
   int depth = 0;  // K per range
-  int fold = 0;   // k values of one wave between folds of its accumulators
+  int fold = 0;   // k values of one wave between folds of its accumulators, in tiles of
+  int edge_fold = 0;          // rows [0, rows) x columns [0, cols) / that reach past them
+  int64_t rows = 0, cols = 0;
 };
 
 // The fastest plan by the model of an m x n x k launch of form `nt` or not,
 // given room for `workspace_bytes` of partials, and in *time its time. A
 // launch of kComputeUnits tiles of 256 x 256 and more is not split over
 // workgroups. The chains of a sum are no longer than the ranges of the split
-// that split_k_shape takes for the launch (nor than 1024: a fold that rare
-// costs nothing measurable; where those ranges are 64 or 96 deep, 32, since
-// the waves' runs end in a rest of their own).
+// that split_k_shape takes for the launch, nor than `bound` says, nor than 1024
+// (where that is 64 or 96, 32, since the waves' runs end in a rest of their
+// own). Folding costs 9 % at 32, 4.5 % at 64, 2 % at 128, 1 % at 256 and nothing
+// measurable from 512 on (64 x 64 tiles, 4500 x 4300 x 4096 and five others).
 inline KwavePlan kwave_fastest(int64_t m, int64_t n, int64_t k, bool nt, uint64_t workspace_bytes,
-                               double* time_out) {
+                               double* time_out, const ChainBound& bound = {}) {
   KwavePlan best;
   if (m <= 0 || n <= 0 || k < kThinK) return best;
   const bool many = ((m + 255) / 256) * ((n + 255) / 256) >= kComputeUnits;
   const SplitK old = split_k_shape(m, n, k, nt, true, ~uint64_t{0});
-  const int64_t chain = std::min<int64_t>(old.splits > 1 ? old.depth : k, 1024);
+  int64_t chain = std::min<int64_t>(old.splits > 1 ? old.depth : k, 1024);
+  if (bound.inside > 0) chain = std::min(chain, bound.inside);
+  const int64_t edge = bound.edge > 0 ? std::min(chain, bound.edge) : chain;
   const double elements = 1e-6 * double(m) * double(n);
   const double memory = 4e-6 * (double(m) + double(n)) * double(k) / 9.67;
   const int64_t partial = split_partial_ld(m) * n * 4;
@@ -283,8 +300,13 @@ inline KwavePlan kwave_fastest(int64_t m, int64_t n, int64_t k, bool nt, uint64_
         sk = split_ranges(k, s, false);
         if (sk.splits != s) continue;
       }
-      const bool folds = (sk.depth + 3) / 4 > chain;
-      if (folds && (t.run == 0 || t.run > chain)) continue;
+      const int64_t quarter = (sk.depth + 3) / 4;
+      if (quarter > edge && (t.run == 0 || t.run > edge)) continue;
+      const auto fold_at = [&](int64_t longest) {
+        if (t.run == 0) return 0;
+        if (quarter <= longest) return (1 << 28) / t.run * t.run;
+        return static_cast<int>((longest <= 96 ? 32 : longest) / t.run * t.run);
+      };
       const int64_t groups = tiles * s, slots = t.per_cu * kComputeUnits;
       const int64_t full = (groups - 1) / slots, last = groups - full * slots;
       // After a few rounds the freed places come in pairs.
@@ -300,9 +322,10 @@ inline KwavePlan kwave_fastest(int64_t m, int64_t n, int64_t k, bool nt, uint64_
         best.tile = i;
         best.splits = s;
         best.depth = sk.depth;
-        best.fold = t.run == 0 ? 0
-                               : folds ? static_cast<int>((chain <= 96 ? 32 : chain) / t.run * t.run)
-                                       : (1 << 28) / t.run * t.run;
+        best.fold = fold_at(chain);
+        best.edge_fold = fold_at(edge);
+        best.rows = edge < chain ? bound.rows : m;
+        best.cols = edge < chain ? bound.cols : n;
       }
     }
   }
@@ -313,13 +336,14 @@ inline KwavePlan kwave_fastest(int64_t m, int64_t n, int64_t k, bool nt, uint64_
 // The plan of a launch of fewer than kComputeUnits tiles of 256 x 256, whose
 // operand panels the kernels can address (each spans less than 2^31 bytes).
 inline KwavePlan kwave_plan_shape(int64_t m, int64_t n, int64_t k, bool nt,
-                                  uint64_t workspace_bytes) {
+                                  uint64_t workspace_bytes, const ChainBound& bound = {}) {
   if (m <= 0 || n <= 0 || ((m + 255) / 256) * ((n + 255) / 256) >= kComputeUnits) return {};
   const SplitK old = split_k_shape(m, n, k, nt, true, ~uint64_t{0});
   if (old.splits > 1 && !old.narrow && old.depth >= 4096 &&
-      16 * (m / 256) * (n / 256) * old.splits >= 15 * kComputeUnits)
+      16 * (m / 256) * (n / 256) * old.splits >= 15 * kComputeUnits &&
+      (bound.inside == 0 || old.depth <= std::min(bound.inside, bound.edge)))
     return {};
-  return kwave_fastest(m, n, k, nt, workspace_bytes, nullptr);
+  return kwave_fastest(m, n, k, nt, workspace_bytes, nullptr, bound);
 }
 
 // The plan a launch takes given room for `workspace_bytes` of partials.
@@ -329,7 +353,7 @@ inline KwavePlan kwave_plan_for(const SgemmLaunch& l, uint64_t workspace_bytes) 
   const int64_t a_bytes = (l.a_kcontig ? int64_t{l.m} : int64_t{l.k}) * l.lda * 4;
   const int64_t b_bytes = (l.b_ncontig ? int64_t{l.k} : int64_t{l.n}) * l.ldb * 4;
   if (a_bytes >= kLimit || b_bytes >= kLimit) return {};
-  return kwave_plan_shape(l.m, l.n, l.k, !l.a_kcontig && l.b_ncontig, workspace_bytes);
+  return kwave_plan_shape(l.m, l.n, l.k, !l.a_kcontig && l.b_ncontig, workspace_bytes, l.bound);
 }
 
 // Tail split. A launch of at least kComputeUnits interior 256 x 256 tiles
@@ -462,6 +486,25 @@ inline SgemmLaunch sub_launch(const SgemmLaunch& l, int64_t r0, int rows, int64_
   return s;
 }
 
+// K rows [k0, k0 + depth) of a launch as a launch of its own (no events): alpha,
+// on C as the caller left it from the first rows, onto the sum so far from the
+// others; the epilogue with the last.
+inline SgemmLaunch k_range(const SgemmLaunch& l, int64_t k0, int64_t depth) {
+  SgemmLaunch s = l;
+  s.k = static_cast<int>(depth);
+  s.a = l.a_kcontig ? l.a + k0 : l.a + k0 * l.lda;
+  s.b = l.b_ncontig ? l.b + k0 * l.ldb : l.b + k0;
+  if (k0 > 0) s.beta = 1.f;
+  if (k0 + depth < l.k) {
+    s.bias_row = nullptr;
+    s.bias_col = nullptr;
+    s.relu = false;
+  }
+  s.start_event = nullptr;
+  s.stop_event = nullptr;
+  return s;
+}
+
 // The parts of a launch's edge split by shape alone (count 0: none).
 inline EdgeParts edge_parts_shape(const SgemmLaunch& l) {
   constexpr int64_t kLimit = int64_t(1) << 31;
@@ -573,39 +616,86 @@ inline double ring_rules_time(int64_t m, int64_t n, int64_t k, bool nt) {
 struct ManyPlan {
   KwavePlan small;        // on small tiles (tile >= 0), or
   int64_t mi = 0, ni = 0; // the rectangle's rows and columns; neither: the rules above
+  int64_t pass = 0;       // K of one pass of the rectangle (its K: one pass)
+  ChainBound bound;       // of the strips' sums, by rows and columns of C
 };
 
-inline ManyPlan many_shape(int64_t m, int64_t n, int64_t k, bool nt) {
+// The chains of a launch of many tiles under the rules above (K a multiple of
+// the ring kernels' step): rows [0, rows) of its interior add all of K in one
+// accumulator, a split tail's rows `tail` k values, and the shortest chain
+// anywhere in C is `shortest`.
+struct Chains {
+  int64_t rows, tail, shortest;
+};
+
+inline Chains ring_rules_chains(int64_t m, int64_t n, int64_t k, bool nt) {
+  constexpr uint64_t kAny = ~uint64_t{0};
+  Chains c{m, k, k};
+  const bool ragged = m % 256 != 0 || n % 256 != 0;
+  if (ragged && !edge_split_rated_faster(m, n, k, nt)) return c;
+  const int64_t mi = m / 256 * 256, ni = n / 256 * 256;
+  const auto split_depth = [&](int64_t rows, int64_t cols) {
+    const SplitK sk = split_k_shape(rows, cols, k, nt, true, kAny);
+    return sk.splits > 1 ? int64_t{sk.depth} : k;
+  };
+  if (const TailSplit ts = tail_split_shape(mi, ni, k, nt, true, kAny); ts.head_m > 0) {
+    c.rows = ts.head_m;
+    c.tail = ts.tail.depth;
+  } else if (split_depth(mi, ni) < k) { // an edge split's interior of few tiles
+    c.rows = 0;
+    c.tail = split_depth(mi, ni);
+  }
+  c.shortest = c.tail;
+  if (ni < n) c.shortest = std::min(c.shortest, split_depth(mi, n - ni));
+  if (mi < m) c.shortest = std::min(c.shortest, split_depth(m - mi, n));
+  return c;
+}
+
+// No sum is added in longer chains than the rules above would add it in
+// (ring_rules_chains): small tiles and the strips fold where a split tail's or
+// an edge strip's sums lie, and a rectangle that reaches past the rows of whole
+// sums runs its K in passes no deeper than the tail's ranges, each after the
+// first adding to C (24 us a round: first loads, and C read back; 4096 x 4096 x
+// 5000 in two passes 1139 against 1111 us). `bound` is that of a part of another
+// launch: it goes to small tiles.
+inline ManyPlan many_shape(int64_t m, int64_t n, int64_t k, bool nt, const ChainBound& bound = {}) {
   ManyPlan plan;
   if (m <= 0 || n <= 0 || k < kThinK ||
       ((m + 255) / 256) * ((n + 255) / 256) < kComputeUnits)
     return plan;
-  double small = 0;
-  const KwavePlan kw = kwave_fastest(m, n, k, nt, 0, &small);
-  small *= 1.0 + 0.07 * std::min(1.0, double(k) / 1500.0);
   const int64_t k1 = k - k % (nt ? 4 : 8);
-  if (k1 != k && k1 < 512) { // the general kernel's K
-    plan.small = kw;
+  if (bound.inside > 0 || (k1 != k && k1 < 512)) { // or the general kernel's K
+    plan.small = kwave_fastest(m, n, k, nt, 0, nullptr, bound);
     return plan;
   }
+  const Chains chains = ring_rules_chains(m, n, k1, nt);
+  const ChainBound rules{chains.tail, chains.shortest, m / 256 * 256, n / 256 * 256};
+  // Rated as if no chain were bounded: the folds cost little (kwave_fastest).
+  double small = 0;
+  kwave_fastest(m, n, k, nt, 0, &small);
+  const KwavePlan kw = kwave_fastest(m, n, k, nt, 0, nullptr, rules);
+  small *= 1.0 + 0.07 * std::min(1.0, double(k) / 1500.0);
   const double rest = k1 == k ? 0.0 : 2.3e-6 * double(m) * double(n) + 4.0;
   double ring = ring_rules_time(m, n, k1, nt) + rest;
   if (k >= 1024) {
     const int64_t tm = m / 256, tn = n / 256;
-    int64_t best_m = 0, best_n = 0;
+    int64_t best_m = 0, best_n = 0, best_passes = 1;
     double best = 0.97 * std::min(ring, small);
     for (int64_t rounds = 1; rounds <= tm * tn / kComputeUnits; ++rounds) {
       for (int64_t a = 1; a <= tm; ++a) {
         const int64_t b = std::min(tn, rounds * kComputeUnits / a);
         if (20 * a * b < 19 * rounds * kComputeUnits) continue;
+        const int64_t passes = a * 256 <= chains.rows ? 1 : (k1 + chains.tail - 1) / chains.tail;
+        if (passes > kMaxPasses) continue;
         const double area = double(m) * double(n) - 65536.0 * double(a * b);
-        const double time = double(rounds) * (0.2155 * double(k1) + 14.0) + 2.0 +
-                            2e-6 * double(k1) * area / 131.0 + (a * 256 < m ? 8.0 : 0.0) +
+        const double time = double(rounds) * (0.2155 * double(k1) + 14.0 + 24.0 * double(passes - 1)) +
+                            2.0 + 2e-6 * double(k1) * area / 131.0 + (a * 256 < m ? 8.0 : 0.0) +
                             (b * 256 < n ? 8.0 : 0.0) + rest;
         if (time < best) {
           best = time;
           best_m = a * 256;
           best_n = b * 256;
+          best_passes = passes;
         }
       }
     }
@@ -613,6 +703,8 @@ inline ManyPlan many_shape(int64_t m, int64_t n, int64_t k, bool nt) {
       if (k1 == k) { // else the K remainder's first part comes here again
         plan.mi = best_m;
         plan.ni = best_n;
+        plan.pass = best_passes == 1 ? k : split_ranges(k, best_passes, false).depth;
+        if (chains.shortest < k) plan.bound = rules;
       }
       return plan;
     }
@@ -627,16 +719,33 @@ inline ManyPlan many_plan(const SgemmLaunch& l) {
   const int64_t a_bytes = (l.a_kcontig ? int64_t{l.m} : int64_t{l.k}) * l.lda * 4;
   const int64_t b_bytes = (l.b_ncontig ? int64_t{l.k} : int64_t{l.n}) * l.ldb * 4;
   if (a_bytes >= kLimit || b_bytes >= kLimit) return {};
-  return many_shape(l.m, l.n, l.k, !l.a_kcontig && l.b_ncontig);
+  return many_shape(l.m, l.n, l.k, !l.a_kcontig && l.b_ncontig, l.bound);
 }
 
-// The parts of a launch on the rectangle of `plan` and its strips.
-inline EdgeParts many_parts(const SgemmLaunch& l, const ManyPlan& plan) {
+// The parts of a launch on the rectangle of `plan`, its passes first, and its
+// strips.
+struct ManyParts {
+  int count = 0;
+  SgemmLaunch part[kMaxPasses + 2];
+};
+
+inline ManyParts many_parts(const SgemmLaunch& l, const ManyPlan& plan) {
   const int mi = static_cast<int>(plan.mi), ni = static_cast<int>(plan.ni);
-  EdgeParts e;
-  e.part[e.count++] = sub_launch(l, 0, mi, 0, ni);
-  if (ni < l.n) e.part[e.count++] = sub_launch(l, 0, mi, ni, l.n - ni);
-  if (mi < l.m) e.part[e.count++] = sub_launch(l, mi, l.m - mi, 0, l.n);
+  ManyParts e;
+  for (int64_t k0 = 0; k0 < l.k; k0 += plan.pass) {
+    SgemmLaunch p = k_range(sub_launch(l, 0, mi, 0, ni), k0, std::min(l.k - k0, plan.pass));
+    p.whole = plan.mi / 256 * (plan.ni / 256) >= kComputeUnits;
+    e.part[e.count++] = p;
+  }
+  const auto strip = [&](int r0, int rows, int c0, int cols) {
+    SgemmLaunch s = sub_launch(l, r0, rows, c0, cols);
+    s.bound = plan.bound;
+    s.bound.rows -= r0;
+    s.bound.cols -= c0;
+    e.part[e.count++] = s;
+  };
+  if (ni < l.n) strip(0, mi, ni, l.n - ni);
+  if (mi < l.m) strip(mi, l.m - mi, 0, l.n);
   e.part[0].start_event = l.start_event;
   e.part[e.count - 1].stop_event = l.stop_event;
   return e;
@@ -658,20 +767,10 @@ inline KParts k_remainder_parts_shape(const SgemmLaunch& l) {
   if (a_bytes >= kLimit || b_bytes >= kLimit) return r;
   const int64_t k1 = k_remainder_shape(l.m, l.n, l.k, !l.a_kcontig && l.b_ncontig);
   if (k1 == 0) return r;
-  SgemmLaunch first = l;
-  first.k = static_cast<int>(k1);
-  first.bias_row = nullptr;
-  first.bias_col = nullptr;
-  first.relu = false;
-  first.stop_event = nullptr;
-  SgemmLaunch rest = l;
-  rest.k = l.k - static_cast<int>(k1);
-  rest.a = l.a_kcontig ? l.a + k1 : l.a + k1 * l.lda;
-  rest.b = l.b_ncontig ? l.b + k1 * l.ldb : l.b + k1;
-  rest.beta = 1.f;
-  rest.start_event = nullptr;
-  r.part[0] = first;
-  r.part[1] = rest;
+  r.part[0] = k_range(l, 0, k1);
+  r.part[1] = k_range(l, k1, l.k - k1);
+  r.part[0].start_event = l.start_event;
+  r.part[1].stop_event = l.stop_event;
   r.count = 2;
   return r;
 }
@@ -699,7 +798,7 @@ struct Route {
   SplitK split;
   TailSplit tail;
   int count = 0; // parts, run one after another
-  SgemmLaunch part[3];
+  SgemmLaunch part[kMaxPasses + 2];
 };
 
 inline uint64_t launch_bytes_wanted(const SgemmLaunch& l);
@@ -719,12 +818,16 @@ inline Route route_with(const SgemmLaunch& l, bool workspace, uint64_t room) {
     r.run = Run::kTwoPanel;
     return r;
   }
+  if (l.whole) {
+    r.run = Run::kRing;
+    return r;
+  }
   if (const ManyPlan mp = many_plan(l); mp.small.tile >= 0) {
     r.run = Run::kSmallTiles;
     r.small = mp.small;
     return r;
   } else if (mp.mi > 0) {
-    const EdgeParts e = many_parts(l, mp);
+    const ManyParts e = many_parts(l, mp);
     parts(Run::kRectangle, e.part, e.count);
     return r;
   }
