@@ -71,9 +71,9 @@ def test_many_tiles():
     """Launches of 256 tiles of 256 x 256 and more (kernels::many_shape): whole
     rounds of interior tiles stay on the ring kernels; shallow K and K that is no
     multiple of their step below 512 go to small tiles and want no partials; a
-    rectangle of whole rounds is whole 256 x 256 tiles inside C that fill at
-    least 19/20 of their rounds, smaller than C, and needs K of the ring
-    kernels' step from 1024 on."""
+    rectangle of whole rounds is whole 256 x 256 tiles inside C that fill at least
+    19/20 of their rounds, smaller than C, needs K of the ring kernels' step from
+    1024 on and runs on those kernels."""
     dll = fns()
     i64, pint = ctypes.c_int64, ctypes.POINTER(ctypes.c_int)
     dll.xvram_hostsim_kwave_many.argtypes = [i64] * 3 + [ctypes.c_int, pint] + [ctypes.POINTER(i64)] * 2
@@ -86,12 +86,16 @@ def test_many_tiles():
     for whole in ((4096, 4096, 256, 1), (8192, 8192, 8192, 1), (8192, 8192, 1024, 0)):
         assert many(*whole) == (-1, 0, 0)
     assert many(5000, 5000, 5000, 0) == many(5000, 5000, 5000, 1) == (-1, 4096, 4096)
+    # The best rectangle of all would be one round of 252 or 255 tiles: small tiles. Where
+    # only the chains leave it fewer (14 of 18 tile rows), it is taken.
+    assert many(5586, 3566, 3344, 0)[0] == many(4352, 4352, 2048, 0)[0] == 2
+    assert many(4608, 4608, 2048, 0) == (-1, 3584, 4608)
     assert many(3712, 4590, 503, 1)[0] == many(6379, 2968, 32, 1)[0] == 6
     # A grid of 2^24 workgroups of 256 threads is past what one launch holds.
     assert many(1 << 17, 1 << 18, 9, 0)[0] == 2 and many(1 << 19, 1 << 19, 9, 0)[0] == -1
     rng = np.random.default_rng(47)
     small = rect = 0
-    for _ in range(2000):
+    for _ in range(3000):
         m, n = (int(2 ** v) for v in rng.uniform(8, 14, 2))
         k, nt = int(2 ** rng.uniform(0, 13)), int(rng.integers(0, 2))
         k = k // 8 * 8 if rng.random() < 0.5 else k
@@ -109,6 +113,10 @@ def test_many_tiles():
             assert mi % 256 == ni % 256 == 0 and 0 < mi <= m and 0 < ni <= n and (mi < m or ni < n)
             groups = mi // 256 * (ni // 256)
             assert 20 * groups >= 19 * -(-groups // 256) * 256
+            how = route(m, n, k, ("NN", "NT")[nt])
+            assert how.startswith(f"rectangle[{mi}x{ni}x")
+            assert all(part.endswith(" ring") for part in how[10:-1].split("; ")
+                       if part.startswith(f"{mi}x{ni}x"))
             assert k >= 1024 and k % (4 if nt else 8) == 0
     assert small > 100 and rect > 30
 

@@ -84,7 +84,7 @@ struct SgemmLaunch {
   float* workspace = nullptr; // split-K partials (16-byte aligned), nullptr = none
   uint64_t workspace_bytes = 0;
   ChainBound bound;   // of a part of another launch
-  bool whole = false; // interior tiles that run unsplit on the ring kernels, also few of them
+  bool whole = false; // interior tiles that run unsplit on the ring kernels
 };
 
 // MI355X: 256 compute units; a launch with fewer tiles than this leaves CUs
@@ -612,7 +612,14 @@ inline double ring_rules_time(int64_t m, int64_t n, int64_t k, bool nt) {
 // N/N 1380 -> 1307, 4576^3 N/T 1406 -> 1317, 11378 x 2374 x 7040 T/T 2870 -> 2705.
 // Modelled like the rest, the strips at 131 TFLOP/s and 8 us each, for K from
 // 1024 on, and taken where that is 3 % faster than the rules above and than
-// small tiles alone (53 shapes: none more than 1.1 % slower than before).
+// small tiles alone (53 shapes: none more than 1.1 % slower than before). Its tiles
+// run unsplit on the ring kernels, as modelled, also where the chains (below)
+// leave it a few less than a round. Where the best rectangle of all is one round
+// of 244 to 255 tiles, so that the rules above leave most of a round idle too,
+// the small tiles are taken up to 7 % above those rules' modelled time (none of
+// 1086 such launches models above; their chains are at most 1024 instead of K):
+// 5586 x 3566 x 3344 N/T 954 us (those rules 986, the rectangle with its 252 tiles
+// on small ones 967), 1792 x 11520 x 4496 N/T 1315 (1442, 1335).
 struct ManyPlan {
   KwavePlan small;        // on small tiles (tile >= 0), or
   int64_t mi = 0, ni = 0; // the rectangle's rows and columns; neither: the rules above
@@ -676,40 +683,41 @@ inline ManyPlan many_shape(int64_t m, int64_t n, int64_t k, bool nt, const Chain
   const KwavePlan kw = kwave_fastest(m, n, k, nt, 0, nullptr, rules);
   small *= 1.0 + 0.07 * std::min(1.0, double(k) / 1500.0);
   const double rest = k1 == k ? 0.0 : 2.3e-6 * double(m) * double(n) + 4.0;
-  double ring = ring_rules_time(m, n, k1, nt) + rest;
+  const double ring = ring_rules_time(m, n, k1, nt) + rest;
+  bool few = false; // the best rectangle, whatever its chains, is less than one round
   if (k >= 1024) {
     const int64_t tm = m / 256, tn = n / 256;
-    int64_t best_m = 0, best_n = 0, best_passes = 1;
-    double best = 0.97 * std::min(ring, small);
+    struct {
+      int64_t a = 0, b = 0, passes = 1;
+      double time;
+    } any, best;
+    any.time = best.time = 0.97 * std::min(ring, small);
     for (int64_t rounds = 1; rounds <= tm * tn / kComputeUnits; ++rounds) {
       for (int64_t a = 1; a <= tm; ++a) {
         const int64_t b = std::min(tn, rounds * kComputeUnits / a);
-        if (20 * a * b < 19 * rounds * kComputeUnits) continue;
-        const int64_t passes = a * 256 <= chains.rows ? 1 : (k1 + chains.tail - 1) / chains.tail;
-        if (passes > kMaxPasses) continue;
+        if (20 * a * b < 19 * rounds * kComputeUnits || (a * 256 == m && b * 256 == n)) continue;
         const double area = double(m) * double(n) - 65536.0 * double(a * b);
-        const double time = double(rounds) * (0.2155 * double(k1) + 14.0 + 24.0 * double(passes - 1)) +
-                            2.0 + 2e-6 * double(k1) * area / 131.0 + (a * 256 < m ? 8.0 : 0.0) +
+        const double time = double(rounds) * (0.2155 * double(k1) + 14.0) + 2.0 +
+                            2e-6 * double(k1) * area / 131.0 + (a * 256 < m ? 8.0 : 0.0) +
                             (b * 256 < n ? 8.0 : 0.0) + rest;
-        if (time < best) {
-          best = time;
-          best_m = a * 256;
-          best_n = b * 256;
-          best_passes = passes;
-        }
+        if (time < any.time) any = {a, b, 1, time};
+        const int64_t passes = a * 256 <= chains.rows ? 1 : (k1 + chains.tail - 1) / chains.tail;
+        const double bounded = time + 24.0 * double(rounds) * double(passes - 1);
+        if (passes <= kMaxPasses && bounded < best.time) best = {a, b, passes, bounded};
       }
     }
-    if (best_m > 0 && (best_m < m || best_n < n)) {
+    few = any.a > 0 && any.a * any.b < kComputeUnits;
+    if (best.a > 0 && !(few && small < 1.07 * ring)) {
       if (k1 == k) { // else the K remainder's first part comes here again
-        plan.mi = best_m;
-        plan.ni = best_n;
-        plan.pass = best_passes == 1 ? k : split_ranges(k, best_passes, false).depth;
+        plan.mi = best.a * 256;
+        plan.ni = best.b * 256;
+        plan.pass = best.passes == 1 ? k : split_ranges(k, best.passes, false).depth;
         if (chains.shortest < k) plan.bound = rules;
       }
       return plan;
     }
   }
-  if (small < 0.96 * ring) plan.small = kw;
+  if (small < (few ? 1.07 : 0.96) * ring) plan.small = kw;
   return plan;
 }
 
@@ -734,7 +742,7 @@ inline ManyParts many_parts(const SgemmLaunch& l, const ManyPlan& plan) {
   ManyParts e;
   for (int64_t k0 = 0; k0 < l.k; k0 += plan.pass) {
     SgemmLaunch p = k_range(sub_launch(l, 0, mi, 0, ni), k0, std::min(l.k - k0, plan.pass));
-    p.whole = plan.mi / 256 * (plan.ni / 256) >= kComputeUnits;
+    p.whole = true;
     e.part[e.count++] = p;
   }
   const auto strip = [&](int r0, int rows, int c0, int cols) {
