@@ -93,7 +93,7 @@ MANY = [
 # large kernels' rules add them in, and how they run.
 BOUNDED = [
     ((4762, 5194, 1208), "rectangle[4096x4096x608 ring; 4096x4096x600 ring; 4096x1098x1208 small"),
-    ((2304, 8512, 2080), "small 64x64 ranges 1 fold 320 edge 32"),
+    ((2304, 8512, 2080), "small 64x64 ranges 1 fold 320 edge 96"),
 ]
 
 

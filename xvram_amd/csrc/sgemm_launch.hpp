@@ -264,18 +264,20 @@ struct KwavePlan {
 // given room for `workspace_bytes` of partials, and in *time its time. A
 // launch of kComputeUnits tiles of 256 x 256 and more is not split over
 // workgroups. The chains of a sum are no longer than the ranges of the split
-// that split_k_shape takes for the launch, nor than `bound` says, nor than 1024
-// (where that is 64 or 96, 32, since the waves' runs end in a rest of their
-// own). Folding costs 9 % at 32, 4.5 % at 64, 2 % at 128, 1 % at 256 and nothing
-// measurable from 512 on (64 x 64 tiles, 4500 x 4300 x 4096 and five others).
+// that split_k_shape takes for the launch (where those are 64 or 96 deep, 32, as
+// measured against them), nor than `bound` says, nor than 1024. Folding costs 9 %
+// at 32, 4.5 % at 64, 2 % at 128, 1 % at 256 and nothing measurable from 512 on
+// (64 x 64 tiles, 4500 x 4300 x 4096 and five others), and as much where only the
+// edge folds: its tiles are the last XCDs' (2975 x 7265 x 920 N/N, a tenth of the
+// tiles at 32, 64, 128: 340, 327, 316 us against 314).
 inline KwavePlan kwave_fastest(int64_t m, int64_t n, int64_t k, bool nt, uint64_t workspace_bytes,
                                double* time_out, const ChainBound& bound = {}) {
   KwavePlan best;
   if (m <= 0 || n <= 0 || k < kThinK) return best;
   const bool many = ((m + 255) / 256) * ((n + 255) / 256) >= kComputeUnits;
   const SplitK old = split_k_shape(m, n, k, nt, true, ~uint64_t{0});
-  int64_t chain = std::min<int64_t>(old.splits > 1 ? old.depth : k, 1024);
-  if (bound.inside > 0) chain = std::min(chain, bound.inside);
+  const int64_t own = std::min<int64_t>(old.splits > 1 ? old.depth : k, 1024);
+  const int64_t chain = bound.inside > 0 ? std::min(own, bound.inside) : own;
   const int64_t edge = bound.edge > 0 ? std::min(chain, bound.edge) : chain;
   const double elements = 1e-6 * double(m) * double(n);
   const double memory = 4e-6 * (double(m) + double(n)) * double(k) / 9.67;
@@ -305,7 +307,7 @@ inline KwavePlan kwave_fastest(int64_t m, int64_t n, int64_t k, bool nt, uint64_
       const auto fold_at = [&](int64_t longest) {
         if (t.run == 0) return 0;
         if (quarter <= longest) return (1 << 28) / t.run * t.run;
-        return static_cast<int>((longest <= 96 ? 32 : longest) / t.run * t.run);
+        return static_cast<int>((longest == own && own <= 96 ? 32 : longest) / t.run * t.run);
       };
       const int64_t groups = tiles * s, slots = t.per_cu * kComputeUnits;
       const int64_t full = (groups - 1) / slots, last = groups - full * slots;
