@@ -159,6 +159,8 @@ def test_no_chain_is_longer_than_the_large_kernels_make_it():
     # The rectangle reaches past the head of the rules' tail split (13 of its 16 tile
     # rows), whose tail's ranges are 2528 deep: two passes.
     assert route(5000, 5000, 5000, "TT").startswith("rectangle[4096x4096x2528 ring; 4096x4096x2472 ring;")
+    # 13 x 19 tiles in one pass leave strips that end in a nearly empty round.
+    assert route(5000, 5000, 2048, "NN").startswith("rectangle[4096x4096x1024 ring; 4096x4096x1024 ring;")
     # Rows that lie in a tail of 320-deep ranges.
     assert fn(2304, 8512, 2080, 0, 0, 2304, 2080, 1800, 0, 0) <= 320
 

@@ -692,8 +692,8 @@ inline ManyPlan many_shape(int64_t m, int64_t n, int64_t k, bool nt, const Chain
     struct {
       int64_t a = 0, b = 0, passes = 1;
       double time;
-    } any, best;
-    any.time = best.time = 0.97 * std::min(ring, small);
+    } any, once, more; // the best one of all, in one pass, in more
+    any.time = once.time = more.time = 0.97 * std::min(ring, small);
     for (int64_t rounds = 1; rounds <= tm * tn / kComputeUnits; ++rounds) {
       for (int64_t a = 1; a <= tm; ++a) {
         const int64_t b = std::min(tn, rounds * kComputeUnits / a);
@@ -705,10 +705,24 @@ inline ManyPlan many_shape(int64_t m, int64_t n, int64_t k, bool nt, const Chain
         if (time < any.time) any = {a, b, 1, time};
         const int64_t passes = a * 256 <= chains.rows ? 1 : (k1 + chains.tail - 1) / chains.tail;
         const double bounded = time + 24.0 * double(rounds) * double(passes - 1);
+        auto& best = passes == 1 ? once : more;
         if (passes <= kMaxPasses && bounded < best.time) best = {a, b, passes, bounded};
       }
     }
     few = any.a > 0 && any.a * any.b < kComputeUnits;
+    auto best = once.a > 0 ? once : more;
+    if (once.a > 0 && more.a > 0) {
+      // Close to each other as a rule: by the strips' own rounds then.
+      const auto time = [&](const auto& r) {
+        const int64_t mi = r.a * 256, ni = r.b * 256;
+        double t = ring_time(r.a * r.b, k1) + 24.0 * double(cu_rounds(r.a * r.b) * (r.passes - 1));
+        double strip = 0;
+        if (ni < n && kwave_fastest(mi, n - ni, k1, nt, ~uint64_t{0}, &strip, rules).tile >= 0) t += strip;
+        if (mi < m && kwave_fastest(m - mi, n, k1, nt, ~uint64_t{0}, &strip, rules).tile >= 0) t += strip;
+        return t;
+      };
+      if (time(more) < time(once)) best = more;
+    }
     if (best.a > 0 && !(few && small < 1.07 * ring)) {
       if (k1 == k) { // else the K remainder's first part comes here again
         plan.mi = best.a * 256;
