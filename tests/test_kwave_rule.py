@@ -7,6 +7,7 @@ given exactly the partials its plan wants takes the same plan and one byte less
 another that fits, and the partials of any launch fit the allocation-free
 entry's 128 MiB."""
 import ctypes
+import time
 
 import numpy as np
 
@@ -163,6 +164,16 @@ def test_no_chain_is_longer_than_the_large_kernels_make_it():
     assert route(5000, 5000, 2048, "NN").startswith("rectangle[4096x4096x1024 ring; 4096x4096x1024 ring;")
     # Rows that lie in a tail of 320-deep ranges.
     assert fn(2304, 8512, 2080, 0, 0, 2304, 2080, 1800, 0, 0) <= 320
+
+
+def test_rule_is_quick_for_many_tiles():
+    """The rule runs on every enqueue: over 512 x 512 tiles it takes microseconds
+    (a search of rounds x tile rows took 2 ms; the bound leaves a slow machine room)."""
+    dll = fns()
+    start = time.perf_counter()
+    for _ in range(20):
+        dll.xvram_hostsim_launch_bytes_wanted(131072, 131072, 1032, 0, 0, 4, 4)
+    assert (time.perf_counter() - start) / 20 < 0.5e-3
 
 
 def test_partials_fit_the_scratch():

@@ -264,18 +264,17 @@ struct KwavePlan {
 // given room for `workspace_bytes` of partials, and in *time its time. A
 // launch of kComputeUnits tiles of 256 x 256 and more is not split over
 // workgroups. The chains of a sum are no longer than the ranges of the split
-// that split_k_shape takes for the launch (where those are 64 or 96 deep, 32, as
+// that split_k_shape takes for the launch (`old`; where those are 64 or 96 deep, 32, as
 // measured against them), nor than `bound` says, nor than 1024. Folding costs 9 %
 // at 32, 4.5 % at 64, 2 % at 128, 1 % at 256 and nothing measurable from 512 on
 // (64 x 64 tiles, 4500 x 4300 x 4096 and five others), and as much where only the
 // edge folds: its tiles are the last XCDs' (2975 x 7265 x 920 N/N, a tenth of the
 // tiles at 32, 64, 128: 340, 327, 316 us against 314).
 inline KwavePlan kwave_fastest(int64_t m, int64_t n, int64_t k, bool nt, uint64_t workspace_bytes,
-                               double* time_out, const ChainBound& bound = {}) {
+                               double* time_out, const ChainBound& bound, const SplitK& old) {
   KwavePlan best;
   if (m <= 0 || n <= 0 || k < kThinK) return best;
   const bool many = ((m + 255) / 256) * ((n + 255) / 256) >= kComputeUnits;
-  const SplitK old = split_k_shape(m, n, k, nt, true, ~uint64_t{0});
   const int64_t own = std::min<int64_t>(old.splits > 1 ? old.depth : k, 1024);
   const int64_t chain = bound.inside > 0 ? std::min(own, bound.inside) : own;
   const int64_t edge = bound.edge > 0 ? std::min(chain, bound.edge) : chain;
@@ -335,6 +334,12 @@ inline KwavePlan kwave_fastest(int64_t m, int64_t n, int64_t k, bool nt, uint64_
   return best;
 }
 
+inline KwavePlan kwave_fastest(int64_t m, int64_t n, int64_t k, bool nt, uint64_t workspace_bytes,
+                               double* time_out, const ChainBound& bound = {}) {
+  return kwave_fastest(m, n, k, nt, workspace_bytes, time_out, bound,
+                       split_k_shape(m, n, k, nt, true, ~uint64_t{0}));
+}
+
 // The plan of a launch of fewer than kComputeUnits tiles of 256 x 256, whose
 // operand panels the kernels can address (each spans less than 2^31 bytes).
 inline KwavePlan kwave_plan_shape(int64_t m, int64_t n, int64_t k, bool nt,
@@ -345,7 +350,7 @@ inline KwavePlan kwave_plan_shape(int64_t m, int64_t n, int64_t k, bool nt,
       16 * (m / 256) * (n / 256) * old.splits >= 15 * kComputeUnits &&
       (bound.inside == 0 || old.depth <= std::min(bound.inside, bound.edge)))
     return {};
-  return kwave_fastest(m, n, k, nt, workspace_bytes, nullptr, bound);
+  return kwave_fastest(m, n, k, nt, workspace_bytes, nullptr, bound, old);
 }
 
 // The plan a launch takes given room for `workspace_bytes` of partials.
@@ -694,8 +699,11 @@ inline ManyPlan many_shape(int64_t m, int64_t n, int64_t k, bool nt, const Chain
       double time;
     } any, once, more; // the best one of all, in one pass, in more
     any.time = once.time = more.time = 0.97 * std::min(ring, small);
-    for (int64_t rounds = 1; rounds <= tm * tn / kComputeUnits; ++rounds) {
-      for (int64_t a = 1; a <= tm; ++a) {
+    // For each number of tile rows the most rounds that all columns fill, and the
+    // three before: of fewer, none was ever the best (60000 random launches).
+    for (int64_t a = 1; a <= tm; ++a) {
+      const int64_t most = std::min(tm * tn / kComputeUnits, cu_rounds(a * tn));
+      for (int64_t rounds = std::max<int64_t>(1, most - 3); rounds <= most; ++rounds) {
         const int64_t b = std::min(tn, rounds * kComputeUnits / a);
         if (20 * a * b < 19 * rounds * kComputeUnits || (a * 256 == m && b * 256 == n)) continue;
         const double area = double(m) * double(n) - 65536.0 * double(a * b);
