@@ -92,6 +92,10 @@ def test_many_tiles():
     assert many(5586, 3566, 3344, 0)[0] == many(4352, 4352, 2048, 0)[0] == 2
     assert many(4608, 4608, 2048, 0) == (-1, 3584, 4608)
     assert many(3712, 4590, 503, 1)[0] == many(6379, 2968, 32, 1)[0] == 6
+    # K no multiple of the ring kernels' step and no K remainder: the general kernel,
+    # against which the small tiles are rated (a rectangle runs on neither).
+    assert route(4096, 4096, 4099, "NN") == route(8192, 8192, 4099, "NT") == "general"
+    assert route(17152, 7936, 10711, "NN").startswith("small 64x64 ranges 1 ")
     # A grid of 2^24 workgroups of 256 threads is past what one launch holds.
     assert many(1 << 17, 1 << 18, 9, 0)[0] == 2 and many(1 << 19, 1 << 19, 9, 0)[0] == -1
     rng = np.random.default_rng(47)

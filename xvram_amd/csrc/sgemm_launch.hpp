@@ -585,6 +585,13 @@ inline double ring_time(int64_t tiles, int64_t k) {
   return double(cu_rounds(tiles)) * (0.2155 * double(k) + 14.0);
 }
 
+// The same of the general kernel over interior tiles (an odd K): 4096 x 4096 at K
+// = 1029, 2051, 4099 N/N 261, 490, 949 us, N/T 255, 478, 928 (T/N 3 % above N/N);
+// 8192 x 8192 x 4099 N/N 3778.
+inline double general_time(int64_t tiles, int64_t k, bool nt) {
+  return double(cu_rounds(tiles)) * ((nt ? 0.2195 : 0.2241) * double(k) + 28.0);
+}
+
 // The model's time of an interior launch with its tail split.
 inline double interior_time(int64_t m, int64_t n, int64_t k) {
   const TailSplit ts = (m / 256) * (n / 256) >= kComputeUnits
@@ -682,7 +689,9 @@ inline ManyPlan many_shape(int64_t m, int64_t n, int64_t k, bool nt, const Chain
     plan.small = kwave_fastest(m, n, k, nt, 0, nullptr, bound);
     return plan;
   }
-  const Chains chains = ring_rules_chains(m, n, k1, nt);
+  // An odd K without a K remainder: the general kernel, on which no rectangle runs.
+  const bool general = k1 != k && k_remainder_shape(m, n, k, nt) == 0;
+  const Chains chains = general ? Chains{m, k, k} : ring_rules_chains(m, n, k1, nt);
   const ChainBound rules{chains.tail, chains.shortest, m / 256 * 256, n / 256 * 256};
   // Rated as if no chain were bounded: the folds cost little (kwave_fastest).
   double small = 0;
@@ -690,9 +699,10 @@ inline ManyPlan many_shape(int64_t m, int64_t n, int64_t k, bool nt, const Chain
   const KwavePlan kw = kwave_fastest(m, n, k, nt, 0, nullptr, rules);
   small *= 1.0 + 0.07 * std::min(1.0, double(k) / 1500.0);
   const double rest = k1 == k ? 0.0 : 2.3e-6 * double(m) * double(n) + 4.0;
-  const double ring = ring_rules_time(m, n, k1, nt) + rest;
+  const double ring =
+      general ? general_time(m / 256 * (n / 256), k, nt) : ring_rules_time(m, n, k1, nt) + rest;
   bool few = false; // the best rectangle, whatever its chains, is less than one round
-  if (k >= 1024) {
+  if (k >= 1024 && !general) {
     const int64_t tm = m / 256, tn = n / 256;
     struct {
       int64_t a = 0, b = 0, passes = 1;
@@ -741,7 +751,10 @@ inline ManyPlan many_shape(int64_t m, int64_t n, int64_t k, bool nt, const Chain
       return plan;
     }
   }
-  if (small < (few ? 1.07 : 0.96) * ring) plan.small = kw;
+  // Level with the general kernel the small tiles' shorter chains decide, to K = 1200
+  // also where they are 3 % behind (4096 x 4096 x 1029 N/N 269 against 261 us).
+  const double limit = general ? (k < 1200 ? 1.04 : 1.0) : few ? 1.07 : 0.96;
+  if (small < limit * ring) plan.small = kw;
   return plan;
 }
 
