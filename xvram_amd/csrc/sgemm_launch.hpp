@@ -442,7 +442,7 @@ inline TailSplit tail_split_for(const SgemmLaunch& l, uint64_t workspace_bytes) 
 // its stream: the interior rows [0, mi) x columns [0, ni) (mi, ni = m, n
 // rounded down to 256; ring kernels, or their tail split), the right strip
 // rows [0, mi) x columns [ni, n) and the bottom strip rows [mi, m) x columns
-// [0, n), each split by the rules above (the strips on the 256 x 128 kernel),
+// [0, n), each split by the rules above (the strips run on small tiles),
 // sharing the workspace. Every element of C is computed by one of them. The
 // split is modelled as the interior's time (tail_split_timed, one round for
 // fewer than kComputeUnits tiles), plus the strips' 256 x 128 tiles x K x
@@ -453,6 +453,12 @@ inline TailSplit tail_split_for(const SgemmLaunch& l, uint64_t workspace_bytes) 
 // model's split / whole ratio came within 7 % of the measured one and picked
 // the faster plan every time (split 4100^2 x 4096 1.74x, 7000^3 1.31x, 5000^2
 // x 2048 1.09x; whole 8191^2 x 8192 1.17x, 8100^2 x 4096 1.15x, 8000^3 1.07x).
+// The 2.7 is of strips on the 256 x 128 kernel, which took longer than small tiles
+// do now; the line it draws stands: of 21 shapes in two forms, timed again both
+// ways, it picks the slower plan on 5280^3 only (which runs on small tiles), and of
+// 65 in 100000 random launches where kwave_fastest rates the strips otherwise by
+// 4 % and more, the 13 furthest ran up to 5 % faster the other way, 16121 x 1253 x
+// 64 T/N 78 against 59 us.
 // Only for one-panel launches with K a multiple of 4 (N/T) or 8 (the other
 // forms), and panels below 2^31 bytes; when a part would split, only with a
 // workspace (a strip unsplit would leave most CUs idle).
