@@ -373,14 +373,25 @@ def test_tail_split_properties(sim):
     assert taken > 100
 
 
-@pytest.mark.parametrize("m,frames", [(4352, 4), (4096, 3)])
-def test_planner_reserves_a_frame_for_a_tail_split(sim, m, frames):
-    """4352 x 4096 x 1024 under 256 MiB frames is one launch whose last tile
-    row runs as a split tail: the plan counts the partials' frame in its
-    working set (C, A, B and the partials); 4096 x 4096 x 1024 fills whole
-    rounds and needs none. Planned only (nothing executes)."""
-    n, k = 4096, 1024
-    with session(sim, frame_mib=256, frames=8) as s:
+@pytest.mark.parametrize("m,n,k,how,frames", [
+    (4608, 4352, 2560, "tail split", 4),
+    (4100, 4100, 240, "edge split", 3),
+    (5000, 4096, 1024, "rectangle", 3),
+    (4100, 4100, 1024, "rectangle", 4), # its right strip (4096 x 4) splits
+    (16384, 256, 16384, "ring split", 4),
+    (4096, 256, 4096, "small", 3), # unsplit: one tile a CU
+    (1024, 1024, 1024, "small", 3),
+    (2048, 2048, 4096, "small", 3),
+    (512, 256, 2048, "small", 4),
+    (4096, 4096, 1024, "ring", 3), # whole rounds
+    (4096, 4096, 4100, "general", 3),
+])
+def test_planner_reserves_a_frame_where_the_launch_uses_partials(sim, m, n, k, how, frames):
+    """One launch under 1 GiB frames: its plan counts a frame of partials beside
+    C, A and B where the launch as the GPU runs it splits K over workgroups, or a
+    part of it does, and only there. Planned only (nothing executes)."""
+    assert route(m, n, k, "NN").startswith(how)
+    with session(sim, frame_mib=1024, frames=8) as s:
         A, B, C = s.allocation(m * k * 4), s.allocation(k * n * 4), s.allocation(m * n * 4)
         plan = xv.GemmPlan(s, xv.matrix(A, m, k, m), xv.matrix(B, k, n, k), xv.matrix(C, m, n, m))
         info = plan.info()
@@ -388,45 +399,76 @@ def test_planner_reserves_a_frame_for_a_tail_split(sim, m, frames):
         for h in (A, B, C):
             h.release()
     assert info.tile_count == 1
-    assert info.maximum_working_set_bytes == frames * 256 * MiB
+    assert info.maximum_working_set_bytes == frames * 1024 * MiB
+
+
+def gemm_plan(lib, m, n, k, frame_mib, frames, distance, form="NT"):
+    """(block tiles along m, along n, lookahead, lanes, partials' frame, panels per
+    launch, H2D bytes) of the schedule the planner takes."""
+    fn = lib.dll.xvram_hostsim_gemm_plan
+    u64 = ctypes.c_uint64
+    fn.argtypes = [u64] * 3 + [ctypes.c_int] * 2 + [u64] * 2 + [ctypes.c_uint32, ctypes.POINTER(u64)]
+    out = (u64 * 7)()
+    assert fn(m, n, k, form[0] == "T", form[1] == "T", frame_mib * MiB, frames, distance, out) == 0
+    return tuple(out)
+
+
+@pytest.mark.parametrize("m,n,k,frame_mib,frames,distance,want", [
+    # 2 x 2 C tiles of 512 x 512 on small tiles. 16 frames hold all of C in one block
+    # with the caller's lookahead; 14 and 12 frames with a launch or two less than
+    # their third allows.
+    (1024, 1024, 8192, 2, 16, 2, (2, 2, 4, 0)),
+    (1024, 1024, 8192, 2, 16, 8, (2, 2, 4, 0)),
+    (1024, 1024, 8192, 2, 16, 1, (2, 2, 2, 0)),
+    (1024, 1024, 8192, 2, 14, 2, (2, 2, 3, 0)),
+    (1024, 1024, 8192, 2, 12, 2, (2, 2, 2, 0)),
+    (1024, 1024, 8192, 2, 12, 8, (2, 2, 2, 0)),
+    # One block either way: launches that want no partials keep the caller's lookahead
+    # and the frame.
+    (4096, 512, 32768, 32, 24, 2, (2, 1, 4, 0)),
+    (4096, 512, 32768, 32, 24, 4, (2, 1, 7, 0)),
+    # Launches that do (3 of 16 MiB): a frame less.
+    (512, 512, 65536, 4, 12, 2, (1, 1, 2, 1)),
+])
+def test_planner_keeps_the_lookahead(sim, m, n, k, frame_mib, frames, distance, want):
+    """The schedule's lookahead is the caller's (twice the prefetch distance, at
+    least two launches, as far as a third of the frames goes), less only what a
+    block with less H2D traffic needs."""
+    gm, gn, ahead, _, partials, _, _ = gemm_plan(sim, m, n, k, frame_mib, frames, distance)
+    assert (gm, gn, ahead, partials) == want
 
 
 def edge_rule(lib):
     fn = lib.dll.xvram_hostsim_edge_split_shape
     fn.restype = ctypes.c_int
-    fn.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int,
-                   ctypes.POINTER(ctypes.c_int)]
-
-    def edge(m, n, k, nt):
-        wants = ctypes.c_int(0)
-        return fn(m, n, k, int(nt), ctypes.byref(wants)), wants.value
-    return edge
+    fn.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
+    return lambda m, n, k, nt: fn(m, n, k, int(nt))
 
 
 @pytest.mark.parametrize("m,n,k,nt,expect", [
     # ragged, a last round that would fill few CUs: the interior (20 x 20 tiles: 19 x 19 with
-    # a tail split) and two strips, which split
-    (5000, 5000, 5000, True, (1, 1)),
-    (7000, 7000, 7000, False, (1, 1)),
-    (4100, 4100, 1024, False, (1, 1)),
-    (4100, 4100, 240, False, (1, 1)),
-    (5000, 5000, 2048, False, (1, 1)),
-    (6312, 6275, 2176, False, (1, 1)),
+    # a tail split) and two strips
+    (5000, 5000, 5000, True, 1),
+    (7000, 7000, 7000, False, 1),
+    (4100, 4100, 1024, False, 1),
+    (4100, 4100, 240, False, 1),
+    (5000, 5000, 2048, False, 1),
+    (6312, 6275, 2176, False, 1),
     # whole rounds (nearly) full: the whole launch on the ring kernels' edge instances
-    (8191, 8191, 2048, True, (0, 0)),
-    (8191, 8191, 8192, False, (0, 0)),
-    (8100, 8100, 4096, False, (0, 0)),
-    (4000, 4000, 12000, True, (0, 0)),
-    (4001, 3999, 1024, False, (0, 0)),
-    (4001, 4093, 2048, True, (0, 0)),
-    (3900, 4096, 1000, False, (0, 0)),
-    (6981, 4328, 3928, True, (0, 0)),
-    (11500, 11000, 1024, False, (0, 0)),
+    (8191, 8191, 2048, True, 0),
+    (8191, 8191, 8192, False, 0),
+    (8100, 8100, 4096, False, 0),
+    (4000, 4000, 12000, True, 0),
+    (4001, 3999, 1024, False, 0),
+    (4001, 4093, 2048, True, 0),
+    (3900, 4096, 1000, False, 0),
+    (6981, 4328, 3928, True, 0),
+    (11500, 11000, 1024, False, 0),
     # K not a multiple of 8 (N/N; N/T takes it), fewer than 256 tiles, interior
-    (4500, 4500, 4500, False, (0, 0)),
-    (4500, 4500, 4500, True, (1, 1)),
-    (2000, 2000, 2000, True, (0, 0)),
-    (4096, 4096, 4096, True, (0, 0)),
+    (4500, 4500, 4500, False, 0),
+    (4500, 4500, 4500, True, 1),
+    (2000, 2000, 2000, True, 0),
+    (4096, 4096, 4096, True, 0),
 ])
 def test_edge_split_rule(sim, m, n, k, nt, expect):
     assert edge_rule(sim)(m, n, k, nt) == expect

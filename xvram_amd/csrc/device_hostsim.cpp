@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "device.hpp"
+#include "gemm.hpp"
 #include "runtime.hpp"
 
 namespace xvram {
@@ -572,13 +573,10 @@ extern "C" __attribute__((visibility("default"))) int xvram_hostsim_tail_split_s
   return ts.head_m > 0 ? ts.tail.splits : 1;
 }
 
-// The edge split rule for a launch shape (panels the ring kernels can
-// address): 1 if kernels::edge_split_rated_faster takes it, and *wants = 1 if
-// one of its parts would split (kernels::edge_split_wants_workspace).
+// Whether a launch of that shape takes the edge split by its rule
+// (kernels::edge_split_rated_faster; panels the ring kernels can address).
 extern "C" __attribute__((visibility("default"))) int xvram_hostsim_edge_split_shape(
-    int64_t m, int64_t n, int64_t k, int nt, int* wants) {
-  if (wants != nullptr)
-    *wants = xvram::kernels::edge_split_wants_workspace(m, n, k, nt != 0) ? 1 : 0;
+    int64_t m, int64_t n, int64_t k, int nt) {
   return xvram::kernels::edge_split_rated_faster(m, n, k, nt != 0) ? 1 : 0;
 }
 
@@ -879,5 +877,36 @@ extern "C" __attribute__((visibility("default"))) int xvram_hostsim_policy_run(
     default: return -1;
     }
   }
+  return 0;
+}
+
+// The schedule make_gemm_plan takes for C = op(A) * op(B), column-major with
+// tight leading dimensions, under `frames` frames: out[0..6] = the block's tiles
+// along m and n, the lookahead, lanes, whether a frame holds partials, K panels
+// per launch and the H2D bytes planned. A non-zero status where it refuses.
+extern "C" __attribute__((visibility("default"))) int xvram_hostsim_gemm_plan(
+    uint64_t m, uint64_t n, uint64_t k, int transpose_a, int transpose_b, uint64_t frame_bytes,
+    uint64_t frames, uint32_t prefetch_distance, uint64_t* out) {
+  using namespace xvram;
+  GemmSpec spec;
+  const auto matrix = [](MatrixSpec& x, uint64_t rows, uint64_t cols) {
+    x.rows = rows;
+    x.columns = cols;
+    x.leading_dimension = rows;
+    x.layout = XVRAM_MATRIX_COLUMN_MAJOR;
+    x.data_type = XVRAM_DATA_FP32;
+  };
+  matrix(spec.a, transpose_a ? k : m, transpose_a ? m : k);
+  matrix(spec.b, transpose_b ? n : k, transpose_b ? k : n);
+  matrix(spec.c, m, n);
+  spec.operation_a = transpose_a ? XVRAM_MATRIX_OP_T : XVRAM_MATRIX_OP_N;
+  spec.operation_b = transpose_b ? XVRAM_MATRIX_OP_T : XVRAM_MATRIX_OP_N;
+  GemmPlanData p;
+  if (Error e = make_gemm_plan(spec, frame_bytes, frames, prefetch_distance, 0, p))
+    return 1;
+  const uint64_t values[] = {p.block_m,       p.block_n,           p.lookahead,
+                             static_cast<uint64_t>(p.lanes), p.scratch ? 1u : 0u, p.panels_per_launch,
+                             p.h2d_bytes_planned};
+  std::copy(std::begin(values), std::end(values), out);
   return 0;
 }

@@ -413,22 +413,27 @@ Error make_gemm_plan(const GemmSpec& spec, uint64_t frame_bytes, uint64_t total_
   out.tiles_m = ceil_div(p.m, tm);
   out.tiles_n = ceil_div(p.n, tn);
   out.panels_k = ceil_div(p.k, bk);
-  // A launch that leaves workgroup slots idle splits its K (or its tail
-  // rows' K, or that of the parts of its edge split, or of the first part of
-  // its K remainder), its partials in one frame of the pool
-  // (kernels::split_k_shape, tail_split_shape, edge_split_wants_workspace and
-  // k_remainder_wants_workspace for the plan's tile and panel; its panels are
-  // below 2^31 bytes): that frame is taken from the schedule's (see below).
-  {
-    const int64_t sm = static_cast<int64_t>(tm), sn = static_cast<int64_t>(tn),
-                  sk = static_cast<int64_t>(bk);
-    const bool nt_form = !p.a.transposed && p.b.transposed;
-    out.scratch = frame_count >= 4 &&
-                  (kernels::split_k_shape(sm, sn, sk, nt_form, true, F).splits > 1 ||
-                   kernels::tail_split_shape(sm, sn, sk, nt_form, true, F).head_m > 0 ||
-                   kernels::edge_split_wants_workspace(sm, sn, sk, nt_form) ||
-                   kernels::k_remainder_wants_workspace(sm, sn, sk, nt_form));
-  }
+  // How the plan's full tile runs over a whole K panel (its panels are below
+  // 2^31 bytes). Where it splits its K, or a part of it does, its partials take
+  // one frame of the pool, which is taken from the schedule's (see below); the
+  // launches at the problem's edges split too then. Edges alone take none: a
+  // frame would also cost the plan its second lane.
+  kernels::SgemmLaunch tile;
+  tile.m = static_cast<int>(tm);
+  tile.n = static_cast<int>(tn);
+  tile.k = static_cast<int>(bk);
+  tile.a_kcontig = p.a.transposed;
+  tile.b_ncontig = p.b.transposed;
+  tile.lda = static_cast<int64_t>(packed_ld(a_geom(p.a, 0, tm, 0, bk)));
+  tile.ldb = static_cast<int64_t>(packed_ld(b_geom(p.b, 0, bk, 0, tn)));
+  tile.ldc = static_cast<int64_t>(round_up(tm, 4));
+  const kernels::Run run = kernels::route_with(tile, true, F).run;
+  // Small tiles for what the large kernels would split into a frame of partials.
+  const bool small = frame_count >= 4 && run == kernels::Run::kSmallTiles &&
+                     kernels::split_k_shape(tile.m, tile.n, tile.k,
+                                            !tile.a_kcontig && tile.b_ncontig, true, F)
+                             .splits > 1;
+  out.scratch = frame_count >= 4 && kernels::uses_partials(tile, F);
 
   // Lookahead: launches whose panels are acquired (and pinned) before they are
   // enqueued, so copies run ahead of compute. At most 3 frames per one-panel
@@ -461,32 +466,29 @@ Error make_gemm_plan(const GemmSpec& spec, uint64_t frame_bytes, uint64_t total_
     }
     return best;
   };
-  uint32_t lookahead = launches_ahead(frame_count);
-  Block best = search(frame_count, 1, lookahead);
-  // The partials' frame, unless a larger block that needs it (and at most two
-  // launches of lookahead) saves H2D traffic and the launches run on the small
-  // tiles (kernels::kwave_plan_shape), which fill the chip without partials too:
-  // 4096 x 4096 x 32768 N/T under 12 frames of 32 MiB takes blocks of 2 x 2
-  // tiles instead of 1 x 2 and streams 1.07 instead of 1.34 GB (25.6 -> 20.4 ms).
-  if (out.scratch) {
-    const uint32_t ahead = launches_ahead(frame_count - 1);
-    const Block with = search(frame_count - 1, 1, ahead);
-    const uint32_t fewer = std::min<uint32_t>(lookahead, 2);
-    const Block without = search(frame_count, 1, fewer);
-    const bool small = kernels::kwave_plan_shape(static_cast<int64_t>(tm), static_cast<int64_t>(tn),
-                                                 static_cast<int64_t>(bk),
-                                                 !p.a.transposed && p.b.transposed, 0)
-                           .tile >= 0;
-    if (small && without.need <= frame_count && without.h2d < with.h2d) {
+  uint32_t lookahead = launches_ahead(frame_count - (out.scratch ? 1 : 0));
+  Block best = search(frame_count - (out.scratch ? 1 : 0), 1, lookahead);
+  // Where launches run on the small tiles and the large kernels would have split
+  // them into a frame of partials, a larger block may take that frame, and as much of the lookahead as it needs (down to two launches, or
+  // to what such a plan would have), if it saves H2D traffic: 4096 x 4096 x 32768
+  // N/T under 12 frames of 32 MiB takes blocks of 2 x 2 tiles and two launches of
+  // lookahead instead of 1 x 2 and three, and streams 1.07 instead of 1.34 GB (25.6
+  // -> 20.4 ms).
+  bool traded = false;
+  if (small) {
+    const uint32_t most = launches_ahead(frame_count);
+    const uint32_t least = std::min<uint32_t>(launches_ahead(frame_count - 1), 2);
+    const Block larger = search(frame_count, 1, least);
+    if (larger.need <= frame_count && larger.h2d < best.h2d) {
+      traded = true;
       out.scratch = false;
-      lookahead = fewer;
-      best = without;
-    } else {
-      --frame_count;
-      lookahead = ahead;
-      best = with;
+      lookahead = most + 1;
+      do {
+        best = search(frame_count, 1, --lookahead);
+      } while (lookahead > least && (best.need > frame_count || best.h2d > larger.h2d));
     }
   }
+  if (out.scratch) --frame_count;
   // Two K panels per launch: the launch is twice as long, so half the
   // lookahead covers the same time. Taken only where the two-panel kernel
   // applies to every launch (no ragged tiles or panels) and the schedule's H2D
@@ -495,15 +497,15 @@ Error make_gemm_plan(const GemmSpec& spec, uint64_t frame_bytes, uint64_t total_
   // executor keeps the panels of the coming pass out of victim selection
   // (Runtime::set_protected), without which such a tight budget evicted panels
   // before their last use (32768^3 under 2 GiB of 64 MiB frames: 23 % more H2D).
-  // Not with a partials frame: a launch whose tiles leave a last round mostly
-  // idle gains more from a tail split than from a second panel.
+  // Only where one panel runs whole on the ring kernels: a launch whose tiles leave
+  // a last round mostly idle gains more from its parts than from a second panel.
   uint32_t panels = 1;
   const double one_panel_flops = launch_flops(tm, tn, bk);
   const bool nt = !p.a.transposed && p.b.transposed;
   const bool two_panel_kernel = tm % 256 == 0 && tn % 256 == 0 &&
                                 (tm / 256) * (tn / 256) >= 256 && p.m % tm == 0 &&
                                 p.n % tn == 0 && bk % 32 == 0 && p.k % (nt ? 4 : 8) == 0 &&
-                                out.panels_k >= 2 && !out.scratch;
+                                out.panels_k >= 2 && run == kernels::Run::kRing;
   if (two_panel_kernel && one_panel_flops <= kTwoPanelMaxFlops &&
       (max_launch_flops == 0 || 2.0 * one_panel_flops <= static_cast<double>(max_launch_flops))) {
     const uint32_t ahead2 = std::max<uint32_t>(1, lookahead / 2);
@@ -545,8 +547,17 @@ Error make_gemm_plan(const GemmSpec& spec, uint64_t frame_bytes, uint64_t total_
     return make_error(XVRAM_STATUS_INVALID_ARGUMENT, "gemm", "make_plan", "too_many_tiles");
   out.launches.reserve(total);
   // A split launch fills the chip by itself, and its partials' frame serves
-  // one launch at a time: one lane.
-  out.lanes = !out.scratch && panels * one_panel_flops <= kDualLaneMaxFlops ? 2 : 1;
+  // one launch at a time: one lane. One lane too where the launches run on small
+  // tiles and their panels take the link about eight times as long as their
+  // kernels the chip (287 FLOP a byte): two find nothing to overlap there and cost
+  // the copies (the 16384-wide layers of batch 256 under 2 GiB, 65 us kernels of 64
+  // MiB panels: 157.2 ms a forward on two lanes, 156.1 on one; 2424 x 1352 x 10304 of
+  // 32 MiB panels, cached, 1.44 ms on two, 1.51 on one). Plans of a larger block
+  // (above) measure the same either way.
+  const bool copies = small && !traded &&
+                      one_panel_flops < 287.0 * static_cast<double>(a_panel_bytes(p, tm, bk) +
+                                                                    b_panel_bytes(p, bk, tn));
+  out.lanes = !out.scratch && !copies && panels * one_panel_flops <= kDualLaneMaxFlops ? 2 : 1;
   uint64_t block_seq = 0;
   for (uint64_t bi = 0; bi < blocks_m; ++bi) {
     for (uint64_t s = 0; s < blocks_n; ++s, ++block_seq) {

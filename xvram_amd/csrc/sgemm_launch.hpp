@@ -347,6 +347,7 @@ inline KwavePlan kwave_plan_shape(int64_t m, int64_t n, int64_t k, bool nt,
   if (m <= 0 || n <= 0 || ((m + 255) / 256) * ((n + 255) / 256) >= kComputeUnits) return {};
   const SplitK old = split_k_shape(m, n, k, nt, true, ~uint64_t{0});
   if (old.splits > 1 && !old.narrow && old.depth >= 4096 &&
+      uint64_t(old.splits) * uint64_t(m) * uint64_t(n) * 4 <= workspace_bytes &&
       16 * (m / 256) * (n / 256) * old.splits >= 15 * kComputeUnits &&
       (bound.inside == 0 || old.depth <= std::min(bound.inside, bound.edge)))
     return {};
@@ -535,19 +536,6 @@ inline EdgeParts edge_parts_shape(const SgemmLaunch& l) {
   e.part[0].start_event = l.start_event;
   e.part[e.count - 1].stop_event = l.stop_event;
   return e;
-}
-
-// Whether an m x n x k launch of form `nt` whose panels the ring kernels can
-// address would take an edge split one of whose parts splits (the planner
-// then gives its launches a workspace).
-inline bool edge_split_wants_workspace(int64_t m, int64_t n, int64_t k, bool nt) {
-  if (!edge_split_rated_faster(m, n, k, nt)) return false;
-  const int64_t mi = m / 256 * 256, ni = n / 256 * 256;
-  constexpr uint64_t kAny = ~uint64_t{0};
-  return split_k_shape(mi, ni, k, nt, true, kAny).splits > 1 ||
-         tail_split_shape(mi, ni, k, nt, true, kAny).head_m > 0 ||
-         (ni < n && split_k_shape(mi, n - ni, k, nt, true, kAny).splits > 1) ||
-         (mi < m && split_k_shape(m - mi, n, k, nt, true, kAny).splits > 1);
 }
 
 // K remainder. The ring kernels need K a multiple of 4 (N/T) or 8 (the other
@@ -945,13 +933,13 @@ inline uint64_t launch_bytes_wanted(const SgemmLaunch& l) {
   return bytes;
 }
 
-// Whether a plan's m x n x k launch of form `nt` would take a K remainder
-// whose first part splits (the planner then gives its launches a workspace).
-inline bool k_remainder_wants_workspace(int64_t m, int64_t n, int64_t k, bool nt) {
-  const int64_t k1 = k_remainder_shape(m, n, k, nt);
-  if (k1 == 0) return false;
-  return tail_split_shape(m, n, k1, nt, true, ~uint64_t{0}).head_m > 0 ||
-         edge_split_wants_workspace(m, n, k1, nt);
+// Whether a launch given room for `room` bytes of partials, or a part of it,
+// splits its K over workgroups.
+inline bool uses_partials(const SgemmLaunch& l, uint64_t room) {
+  const Route r = route_with(l, true, room);
+  for (int i = 0; i < r.count; ++i)
+    if (uses_partials(r.part[i], room)) return true;
+  return r.small.splits > 1 || r.split.splits > 1 || r.tail.head_m > 0;
 }
 
 // Enqueues the launch on `stream` (a hipStream_t); returns a hipError_t.
