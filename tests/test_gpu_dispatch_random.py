@@ -1,14 +1,13 @@
 """Seeded random shapes across the launch rules, on the MI355X through the C
 ABI (the extension's sgemm_device on device memory), every element checked.
 
-The shapes are drawn so that each of the dispatch rules of sgemm_launch.hpp
-fires several times: split K on the ring kernels and on the 256 x 128 kernel
-(fewer tiles than CUs, one or two rounds of ranges), the tail split (interior
-launches of at least 256 tiles whose last round would leave CUs idle), the
-edge split (ragged launches of at least 256 tiles: interior, right strip,
-bottom strip) and the whole ragged launch on the ring kernels' edge instances
-(6981 x 4328 x 3928 here), in random N/T forms, with K a multiple of 8 and,
-for some, not.
+Shapes are drawn until each route of a launch (kernels::route) has two of them:
+small tiles unsplit and with K split over workgroups, deep interior launches
+split on the ring kernels, the tail split, the edge split with its interior on
+the ring kernels and on small tiles, the rectangle of whole rounds in one pass
+of K and in several, the K remainder, whole ragged launches on the ring kernels'
+edge instances, whole rounds on the ring kernels and odd K on the general kernel;
+in random N/T forms.
 Operands are the analytic pattern (examples' gemm_bench pattern: exact in FP32
 for these K), so every element of C must equal its closed form bit for bit,
 whichever split, order of ranges or part computed it."""
@@ -20,6 +19,7 @@ import pytest
 import xvram_amd as xv
 from xvram_amd import abi
 
+from gemm_cases import route
 from test_gpu_sgemm_device import FORMS, Hip, desc_for, padded
 from test_gpu_tail_split import pattern_stored, synth  # noqa: F401  (fixture)
 
@@ -30,31 +30,52 @@ def log(msg):
     print(f"[dispatch] {msg}", flush=True)
 
 
-def make_cases(seed=4242):
+ROUTES = ["small unsplit", "small split", "many small", "ring split", "tail split",
+          "edge split ring", "edge split small", "rectangle", "rectangle in passes", "k remainder",
+          "edge ring", "ring", "general"]
+
+
+def kind_of(m, n, k, form):
+    how = route(m, n, k, form)
+    if how.startswith("small"):
+        if -(-m // 256) * -(-n // 256) >= 256:
+            return "many small"
+        return "small unsplit" if " ranges 1 " in how else "small split"
+    if how.startswith("rectangle["):
+        parts = how[10:].split("; ")
+        return "rectangle in passes" if parts[1].split("x")[:2] == parts[0].split("x")[:2] else "rectangle"
+    if how.startswith("edge split["):
+        return "edge split " + how[11:].split(" ")[1].rstrip(";")
+    return how.split("[")[0] if "[" in how else " ".join(w for w in how.split(" ") if w.isalpha())
+
+
+def make_cases(seed=4242, each=2):
     rng = np.random.default_rng(seed)
+    wanted = {r: each for r in ROUTES}
     cases = []
-    kinds = ["small", "small", "narrow", "narrow", "tail", "tail", "edge", "edge", "edge", "edge"]
-    for i, kind in enumerate(kinds):
-        if kind == "small":     # interior, fewer tiles than CUs: ring or 256 x 128 split
-            m, n = (256 * int(v) for v in rng.integers(2, 12, 2))
-            k = 8 * int(rng.integers(64, 1024))
-        elif kind == "narrow":  # ragged, fewer than 256 tiles: 256 x 128 split
-            m, n = (int(v) for v in rng.integers(300, 3500, 2))
-            k = int(rng.integers(300, 6000))
-        elif kind == "tail":    # interior, 257..400 tiles
-            tm = int(rng.integers(16, 21))
-            tn = int(rng.integers(max(16, -(-257 // tm)), 21))
-            m, n = 256 * tm, 256 * tn
-            k = 8 * int(rng.integers(128, 512))
-        else:                   # ragged, at least 256 tiles
-            tm, tn = (int(v) for v in rng.choice([16, 19, 24, 27], 2))
-            m, n = (256 * t + int(rng.integers(1, 256)) for t in (tm, tn))
-            k = 8 * int(rng.integers(256, 640))
+    while any(wanted.values()):
+        if wanted["ring split"] and rng.random() < 0.2:  # at least 4096 deep on nearly every CU
+            m, n, k = 256 * int(rng.integers(24, 33)), 256 * int(rng.integers(2, 5)), 8 * int(rng.integers(1024, 1300))
+        elif rng.random() < 0.2:
+            m, n, k = (int(v) for v in rng.integers(300, 3500, 3))
+        else:
+            m, n, k = (int(v) for v in rng.integers(2048, 5600, 3))
+            k //= 2
+        if rng.random() < 0.4:
+            m, n = m // 256 * 256, n // 256 * 256
+        if rng.random() < 0.6:
+            k = k // 8 * 8
+        if min(m, n, k) == 0:
+            continue
         form = sorted(FORMS)[int(rng.integers(0, 4))]
-        if kind == "edge" and i == len(kinds) - 1:
-            k, form = k + 4, "NT"  # K a multiple of 4 only: N/T takes the edge split
-        cases.append((kind, m, n, k, form))
+        kind = kind_of(m, n, k, form)
+        if wanted.get(kind):
+            wanted[kind] -= 1
+            cases.append((kind, m, n, k, form))
     return cases
+
+
+CASES = make_cases()
 
 
 @pytest.fixture(scope="module")
@@ -62,8 +83,8 @@ def lib():
     return xv.load()
 
 
-@pytest.mark.parametrize("kind,m,n,k,form", make_cases(),
-                         ids=[f"{c[0]}-{c[1]}x{c[2]}x{c[3]}-{c[4]}" for c in make_cases()])
+@pytest.mark.parametrize("kind,m,n,k,form", CASES,
+                         ids=[f"{c[0].replace(' ', '-')}-{c[1]}x{c[2]}x{c[3]}-{c[4]}" for c in CASES])
 def test_dispatch_pattern_exact(lib, synth, oracle_mod, kind, m, n, k, form):
     ops = FORMS[form]
     a_st = pattern_stored(synth, "a", *((m, k) if ops[0] == abi.OP_N else (k, m)),

@@ -17,18 +17,23 @@ would show in C.
   element within the FP64 bound, and two executions bit-identical.
 * 4001 x 4093 x 2048 and 3900 x 4096 x 1000, all four forms: the analytic
   pattern, every element bit-exact.
-* A K remainder onto a whole launch: 4001 x 3999 x 1030 (K % 8 = 6, K % 4 =
-  2), all four forms, alpha, beta, a per-row bias and ReLU: the rounded K on
-  the edge instances, the last K rows on the thin-K kernel; within the bound.
+* A K remainder onto a whole launch: 4001 x 3999 x 2051 (K % 8 = 3), and 4102
+  for N/T (K % 4 = 2), all four forms, alpha, beta, a per-row bias and ReLU: the
+  rounded K on the edge instances, the last K rows on the thin-K kernel; within
+  the bound.
 * Thin-K launches (K = 1, 3 and 7; 1001 x 515: a partial row block and a
   partial group of columns), all four forms, alpha, beta, a per-column bias
   and ReLU: within the bound.
 * The other kernels under the same NaN padding, whose predicated loads take
   out-of-range rows, columns and k as zeros in both operands (0 x NaN would
-  be NaN): the general 256 x 256 kernel on 4001 x 3999 x 501 (edge tiles and
-  a K tail; no K remainder below 512) and 4096^2 x 1001 (interior tiles, K
-  tail), and the 256 x 128 kernel's split on config 2 (3001 x 2047 x 4099),
-  all four forms: within the bound, no NaN.
+  be NaN): the general 256 x 256 kernel on 4096^2 x 1403 (interior tiles, K
+  tail; its edge tiles, which only launches without a workspace reach, are in
+  tests/test_gpu_wide.py), and the 256 x 128 kernel, split and unsplit, with an
+  operand of 2 GiB and more (short lines or k rows far apart), all four
+  forms: within the bound, no NaN. The small tiles, which skip padding by
+  clamping and masking, on 4001 x 3999 x 501 and config 2 (3001 x 2047 x 4099).
+
+Each test asserts that its launch takes that route (kernels::route).
 
 Tolerance: |C - C_ref| <= 4*K*2^-24*(|alpha||A||B| + |beta C0| + |bias|)_ij."""
 import ctypes
@@ -39,6 +44,7 @@ import pytest
 import xvram_amd as xv
 from xvram_amd import abi
 
+from gemm_cases import route
 from test_gpu_sgemm_device import FORMS, Hip, desc_for
 from test_gpu_tail_split import pattern_stored, synth  # noqa: F401  (fixture)
 
@@ -61,24 +67,25 @@ def hip(lib):
     h.close()
 
 
-def nan_padded(mat):
-    """Column-major storage (flat, ld) with ld rounded up to 4 floats and the
-    padding rows set to NaN."""
+def nan_padded(mat, ld=None):
+    """Column-major storage (flat, ld) with ld rounded up to 4 floats, unless
+    given, and the padding rows set to NaN."""
     rows, cols = mat.shape
-    ld = (rows + 3) // 4 * 4
+    ld = ld or (rows + 3) // 4 * 4
     buf = np.full((cols, ld), np.nan, dtype=np.float32)
     buf[:, :rows] = mat.T
     return buf.reshape(-1), ld
 
 
-def run_gemm(lib, hip, oracle_mod, m, n, k, form, seed, alpha, beta, axis, relu, repeat=2):
+def run_gemm(lib, hip, oracle_mod, m, n, k, form, seed, alpha, beta, axis, relu, repeat=2,
+             lda=None):
     ops = FORMS[form]
     a_op = np.asfortranarray(oracle_mod.fill_uniform(m * k, seed).reshape(k, m).T)
     b_op = np.asfortranarray(oracle_mod.fill_uniform(k * n, seed + 1).reshape(n, k).T)
     c0 = np.asfortranarray(oracle_mod.fill_uniform(m * n, seed + 2).reshape(n, m).T)
     length = m if axis == abi.BIAS_PER_ROW else n
     bias = (oracle_mod.fill_uniform(length, seed + 3) * 0.5).astype(np.float32)
-    a_flat, lda = nan_padded(a_op if ops[0] == abi.OP_N else a_op.T)
+    a_flat, lda = nan_padded(a_op if ops[0] == abi.OP_N else a_op.T, lda)
     b_flat, ldb = nan_padded(b_op if ops[1] == abi.OP_N else b_op.T)
     c_flat, ldc = nan_padded(c0)
     pa, pb, pc = hip.alloc(a_flat.nbytes), hip.alloc(b_flat.nbytes), hip.alloc(c_flat.nbytes)
@@ -119,6 +126,7 @@ def check(oracle_mod, outs, k, ref, absab, what):
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_edge_ring_within_bound(lib, hip, oracle_mod, form, axis):
     m, n, k = 4001, 3999, 1024
+    assert route(m, n, k, form) == "edge ring"
     outs, ref, absab = run_gemm(lib, hip, oracle_mod, m, n, k, form, 901, 1.25, -0.5, axis, True)
     check(oracle_mod, outs, k, ref, absab,
           f"{m}x{n}x{k} {form} bias {'row' if axis == abi.BIAS_PER_ROW else 'col'} + ReLU")
@@ -127,6 +135,7 @@ def test_edge_ring_within_bound(lib, hip, oracle_mod, form, axis):
 @pytest.mark.parametrize("m,n,k", [(4001, 4093, 2048), (3900, 4096, 1000)], ids=["mn", "m"])
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_edge_ring_pattern(lib, hip, synth, oracle_mod, form, m, n, k):
+    assert route(m, n, k, form) == "edge ring"
     ops = FORMS[form]
     a_st = pattern_stored(synth, "a", *((m, k) if ops[0] == abi.OP_N else (k, m)),
                           ops[0] == abi.OP_T)
@@ -156,7 +165,9 @@ def test_edge_ring_pattern(lib, hip, synth, oracle_mod, form, m, n, k):
 
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_k_remainder_onto_whole_launch(lib, hip, oracle_mod, form):
-    m, n, k = 4001, 3999, 1030
+    m, n, k = 4001, 3999, 4102 if form == "NT" else 2051
+    assert route(m, n, k, form) == \
+        f"k remainder[{m}x{n}x{k - k % 4 if form == 'NT' else k - k % 8} edge ring; {m}x{n}x{k % (4 if form == 'NT' else 8)} thin]"
     outs, ref, absab = run_gemm(lib, hip, oracle_mod, m, n, k, form, 911, 0.75, 1.5,
                                 abi.BIAS_PER_ROW, True)
     check(oracle_mod, outs, k, ref, absab, f"{m}x{n}x{k} {form} (K remainder) bias row + ReLU")
@@ -166,15 +177,34 @@ def test_k_remainder_onto_whole_launch(lib, hip, oracle_mod, form):
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_thin_k_within_bound(lib, hip, oracle_mod, form, k):
     m, n = 1001, 515
+    assert route(m, n, k, form) == "thin"
     outs, ref, absab = run_gemm(lib, hip, oracle_mod, m, n, k, form, 921 + k, -1.5, 0.25,
                                 abi.BIAS_PER_COLUMN, True)
     check(oracle_mod, outs, k, ref, absab, f"thin {m}x{n}x{k} {form} bias col + ReLU")
 
 
-@pytest.mark.parametrize("m,n,k", [(4001, 3999, 501), (4096, 4096, 1001), (3001, 2047, 4099)],
-                         ids=["wide-edge", "wide-ktail", "narrow-split"])
+@pytest.mark.parametrize("m,n,k,how", [(4096, 4096, 1403, "general"), (4001, 3999, 501, "small"),
+                                       (3001, 2047, 4099, "small")],
+                         ids=["general-ktail", "small-edge", "small-config2"])
 @pytest.mark.parametrize("form", sorted(FORMS))
-def test_other_kernels_ignore_nan_padding(lib, hip, oracle_mod, form, m, n, k):
+def test_other_kernels_ignore_nan_padding(lib, hip, oracle_mod, form, m, n, k, how):
+    assert route(m, n, k, form).startswith(how)
     outs, ref, absab = run_gemm(lib, hip, oracle_mod, m, n, k, form, 931, 1.5, 0.5,
                                 abi.BIAS_PER_COLUMN, False, repeat=1)
     check(oracle_mod, outs, k, ref, absab, f"{m}x{n}x{k} {form} under NaN padding")
+
+
+@pytest.mark.parametrize("split", [True, False], ids=["split", "unsplit"])
+@pytest.mark.parametrize("form", sorted(FORMS))
+def test_narrow_kernel_ignores_nan_padding(lib, hip, oracle_mod, form, split):
+    """The 256 x 128 kernel: an A of 2 GiB of mostly padding, edge tiles on both
+    sides and a K tail (unsplit: K = 101)."""
+    if form[0] == "T":
+        m, n, k, lda = 4104, 259, 517 if split else 101, 131076
+    else:
+        m, n, k, lda = (517, 259, 4101, 131076) if split else (517, 259, 101, 5400000)
+    how = route(m, n, k, form, lda=lda)
+    assert how.startswith("narrow split ") if split else how == "narrow"
+    outs, ref, absab = run_gemm(lib, hip, oracle_mod, m, n, k, form, 941, 1.5, 0.5,
+                                abi.BIAS_PER_ROW, True, repeat=1, lda=lda)
+    check(oracle_mod, outs, k, ref, absab, f"{m}x{n}x{k} {form} lda {lda} under NaN padding")

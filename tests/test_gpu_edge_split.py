@@ -4,15 +4,18 @@ A launch of at least 256 tiles of 256 x 256 whose m or n is not a multiple of
 256 may run as its interior tiles (ring kernels, or their tail split) and two
 edge strips, each a launch of its own (kernels::edge_parts):
 
-* 4100 x 4100 x 1024 (17 x 17 tiles: the 16 x 16 interior, a 4096 x 4 right
-  strip and a 4 x 4100 bottom strip), all four forms, seeded U[-1,1) operands
-  with alpha, beta and ReLU and a per-row or per-column bias (offset into each
-  strip's rows or columns): every element within the FP64 bound, and two
-  executions bit-identical.
-* 5000 x 5000 x 2048 (the interior of 19 x 19 tiles takes a tail split), N/N
-  and N/T: the analytic pattern, every element bit-exact.
-* 4100 x 4100 x 1024 in a session (resident, 128 MiB frames: the strips'
-  partials in one frame of the pool), N/N and T/T: the pattern, bit-exact.
+* 4251 x 4188 x 432 (the 16 x 16 interior on the ring kernels, a 4096 x 92 right
+  strip and a 155 x 4188 bottom strip on small tiles), all four forms, seeded
+  U[-1,1) operands with alpha, beta and ReLU and a per-row or per-column bias
+  (offset into each strip's rows or columns): every element within the FP64
+  bound, and two executions bit-identical.
+* 5600 x 4256 x 768 N/N and 5287 x 4287 x 1976 N/T (the interior takes a tail
+  split): the analytic pattern, every element bit-exact.
+* 5172 x 4749 x 2832 in a session (resident, 128 MiB frames: a strip's partials
+  in one frame of the pool), and 4100 x 4100 x 1024, a rectangle of 16 x 16 tiles
+  whose right strip splits, N/N and T/T: the pattern, bit-exact.
+
+Each test asserts that its launch takes that route (kernels::route).
 
 Tolerance: |C - C_ref| <= 4*K*2^-24*(|alpha||A||B| + |beta C0| + |bias|)_ij."""
 import ctypes
@@ -23,6 +26,7 @@ import pytest
 import xvram_amd as xv
 from xvram_amd import abi
 
+from gemm_cases import route
 from test_gpu_sgemm_device import FORMS, Hip, desc_for, padded, stored
 from test_gpu_tail_split import pattern_stored, synth  # noqa: F401  (fixture)
 
@@ -50,7 +54,8 @@ def hip(lib):
 @pytest.mark.parametrize("axis", [abi.BIAS_PER_ROW, abi.BIAS_PER_COLUMN], ids=["row", "col"])
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_edge_split_within_bound_and_deterministic(lib, hip, oracle_mod, form, axis):
-    m, n, k = 4100, 4100, 1024
+    m, n, k = 4251, 4188, 432
+    assert route(m, n, k, form).startswith("edge split[4096x4096x432 ring; 4096x92x432 small")
     alpha, beta = 1.25, -0.5
     ops = FORMS[form]
     seed = 801
@@ -90,9 +95,10 @@ def test_edge_split_within_bound_and_deterministic(lib, hip, oracle_mod, form, a
     assert bad == 0
 
 
-@pytest.mark.parametrize("form", ["NN", "NT"])
-def test_edge_split_with_tail_pattern(lib, hip, synth, oracle_mod, form):
-    m, n, k = 5000, 5000, 2048
+@pytest.mark.parametrize("m,n,k,form", [(5600, 4256, 768, "NN"), (5287, 4287, 1976, "NT")],
+                         ids=["NN", "NT"])
+def test_edge_split_with_tail_pattern(lib, hip, synth, oracle_mod, m, n, k, form):
+    assert route(m, n, k, form).startswith(f"edge split[{m // 256 * 256}x4096x{k} tail split 4096 ")
     ops = FORMS[form]
     a_st = pattern_stored(synth, "a", *((m, k) if ops[0] == abi.OP_N else (k, m)),
                           ops[0] == abi.OP_T)
@@ -120,9 +126,12 @@ def test_edge_split_with_tail_pattern(lib, hip, synth, oracle_mod, form):
     assert bad == 0
 
 
+@pytest.mark.parametrize("m,n,k,how", [(5172, 4749, 2832, "edge split[5120x4608x2832 rectangle"),
+                                       (4100, 4100, 1024, "rectangle[4096x4096x1024 ring;")],
+                         ids=["edge-split", "rectangle"])
 @pytest.mark.parametrize("form", ["NN", "TT"])
-def test_edge_split_in_a_session(lib, synth, oracle_mod, form):
-    m, n, k = 4100, 4100, 1024
+def test_edge_split_in_a_session(lib, synth, oracle_mod, form, m, n, k, how):
+    assert route(m, n, k, form, 128 * MiB).startswith(how)
     ops = FORMS[form]
     a_shape = (m, k) if ops[0] == abi.OP_N else (k, m)
     b_shape = (k, n) if ops[1] == abi.OP_N else (n, k)
@@ -155,16 +164,29 @@ def test_edge_split_in_a_session(lib, synth, oracle_mod, form):
     assert bad == 0
 
 
-@pytest.mark.parametrize("m,n,k,form", [(4100, 4100, 1028, "NN"), (4352, 4096, 1027, "TT"),
-                                        (4100, 4100, 1030, "NT")],
-                         ids=["edge-NN", "tail-TT", "edge-NT"])
-def test_k_remainder_within_bound(lib, hip, oracle_mod, m, n, k, form):
-    """K not a multiple of 8 (N/N, T/T) or 4 (N/T): the launch runs over the
-    rounded K (an edge or tail split, no epilogue) and then over the last 2-4
-    K rows onto that result (beta 1, the epilogue): alpha, beta, a per-row
-    bias and ReLU, every element within the FP64 bound, repeats bit-identical."""
+# The first part on a rectangle and strips, split into head and tail, as an edge split.
+K_REMAINDERS = [(4134, 4225, 1835, form, "rectangle[4096x4096x1832 ring;" if form != "NT" else "rectangle[")
+                for form in sorted(FORMS)] + [
+    (5120, 4352, 1892, "NN", "tail split 3840 3x640"),
+    (3584, 5376, 2447, "NT", "tail split 3072 6x416"),
+    (5120, 4352, 1719, "TN", "tail split 3840 3x576"),
+    (5120, 4352, 1634, "TT", "tail split 3840 3x544"),
+    (6400, 2571, 1029, "TN", "edge split["),
+]
+
+
+@pytest.mark.parametrize("m,n,k,form,first", K_REMAINDERS,
+                         ids=[f"{c[4].split('[')[0].split()[0]}-{c[3]}" for c in K_REMAINDERS])
+def test_k_remainder_within_bound(lib, hip, oracle_mod, m, n, k, form, first):
+    """K not a multiple of 8 or (N/T) 4: the launch runs over the rounded K (a
+    rectangle, a tail or an edge split, no epilogue) and then over the last 1 to 7
+    K rows onto that result (beta 1, the epilogue): alpha, beta, a per-row bias
+    and ReLU, every element within the FP64 bound, repeats bit-identical."""
     from test_gpu_sgemm_device import run_device_gemm
 
+    how = route(m, n, k, form)
+    assert how.startswith("k remainder[") and how.split(" ", 3)[2].startswith(first.split()[0]) and \
+        first in how and how.endswith(" thin]")
     outs, ref, absab = run_device_gemm(lib, hip, oracle_mod, m, n, k, FORMS[form], 811,
                                        alpha=0.75, beta=-1.25, bias_rows=True, relu=True,
                                        repeat=2)

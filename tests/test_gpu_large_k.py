@@ -4,7 +4,7 @@ the C ABI: 2049 x 2049 x 32769 with every matrix row-major, 64 MiB frames, a
 265-300). The panel planner runs it as 2049 x 2049 C tiles over nine K panels
 of 4096 (the last one 1 deep), out of core: A and B (256 MiB each) stream
 through five frames, one of which holds the split-K partials of the ragged
-2049 x 2049 x 4096 launches (256 x 128 kernel, 3 ranges). Seeded U[-1,1)
+2049 x 2049 x 4096 launches (small tiles, 2 ranges). Seeded U[-1,1)
 operands; C checked against the FP64 oracle on one full column per 256
 columns, one full row per 256 rows and 1024 random elements, every one with
 its full K, within |C - C_ref| <= 4*K*2^-24*(|A||B|)_ij."""

@@ -2,16 +2,17 @@
 memory the caller owns, enqueued on the caller's HIP stream, through the C ABI
 (extension table), against the FP64 oracle.
 
-* Config 1's shape (1024^3 N/N: 32 tiles of 256 x 128, K in 8 ranges) with the
-  library's stream-ordered workspace and with a workspace of the caller's:
-  the same bits both ways, within the FP64 bound.
-* The config-5 launch shape in every form (4096 x 256 x 4096, 16 ranges) with
-  alpha, beta and a per-row bias + ReLU: within the bound.
+* Config 1's shape (1024^3 N/N, unsplit on small tiles) without and with a
+  workspace of the caller's: the same bits both ways, within the FP64 bound.
+* The config-5 launch shape in every form (4096 x 256 x 4096) with alpha, beta
+  and a per-row bias + ReLU: within the bound.
 * Shapes that do not split (256 tiles; K too shallow for two ranges).
-* Config 2's ragged shape (3001 x 2047 x 4099, alpha 1.5, beta 0.5): 12 x 16
-  tiles of 256 x 128 split into 5 ranges (960 workgroups: two rounds of the
-  kernel's workgroup slots), with the library's workspace and with the
-  caller's: the same bits both ways, within the bound.
+* Config 2's ragged shape (3001 x 2047 x 4099, alpha 1.5, beta 0.5; unsplit on
+  small tiles), without and with a workspace of the caller's: the same bits both
+  ways, within the bound.
+* A split launch (1024 x 500 x 8192 N/T, four ranges) with the library's
+  stream-ordered workspace and with a workspace of the caller's, large enough or
+  not: the same bits.
 * Interior 256 x 256 tiles whose operand panel the ring kernels cannot
   address: op-T A with a leading dimension of 2^20 floats (a 2 GiB panel,
   beyond their 32-bit buffer offsets), 512 x 512 x 2048 in 32 ranges on the
@@ -31,6 +32,8 @@ import pytest
 
 import xvram_amd as xv
 from xvram_amd import abi
+
+from gemm_cases import route
 
 pytestmark = pytest.mark.gpu
 
@@ -176,11 +179,26 @@ def test_config1_shape_library_and_caller_workspace(lib, hip, oracle_mod):
     bad, _, ratio = oracle_mod.check_bound(np.asfortranarray(outs[0]), k, ref, absab)
     log(f"1024^3 NN, library workspace: violations {bad}, err/bound {ratio:.3e}")
     assert bad == 0
-    # Eight 4 MiB partials in a workspace of the caller's, exactly their size: the same
-    # split, the same bits.
+    # A workspace of the caller's that it does not need.
     mine, _, _ = run_device_gemm(lib, hip, oracle_mod, m, n, k, FORMS["NN"], 501,
                                  workspace_bytes=32 * MiB)
     assert np.array_equal(mine[0].view(np.uint32), outs[0].view(np.uint32))
+
+
+def test_split_library_and_caller_workspace(lib, hip, oracle_mod):
+    """1024 x 500 x 8192 N/T: four ranges on small tiles. Their four partials of
+    1024 x 500 floats in the library's workspace, in one of the caller's of exactly
+    their size and in one too small (the library's serves): the same bits."""
+    m, n, k = 1024, 500, 8192
+    assert route(m, n, k, "NT").startswith("small 64x64 ranges 4 ")
+    outs, ref, absab = run_device_gemm(lib, hip, oracle_mod, m, n, k, FORMS["NT"], 505)
+    bad, _, ratio = oracle_mod.check_bound(np.asfortranarray(outs[0]), k, ref, absab)
+    log(f"{m}x{n}x{k} NT, library workspace: violations {bad}, err/bound {ratio:.3e}")
+    assert bad == 0
+    for size in (4 * m * n * 4, 4 * m * n * 4 - 16):
+        mine, _, _ = run_device_gemm(lib, hip, oracle_mod, m, n, k, FORMS["NT"], 505,
+                                     workspace_bytes=size)
+        assert np.array_equal(mine[0].view(np.uint32), outs[0].view(np.uint32))
 
 
 @pytest.mark.parametrize("form", sorted(FORMS))
@@ -211,7 +229,7 @@ def test_config2_ragged_split(lib, hip, oracle_mod, form):
     log(f"config 2 {m}x{n}x{k} {form}, library workspace: violations {bad}, "
         f"err/bound {ratio:.3e}")
     assert bad == 0
-    # Five partials of 3004 x 2047 floats in a workspace of the caller's.
+    # A workspace of the caller's that it does not need.
     mine, _, _ = run_device_gemm(lib, hip, oracle_mod, m, n, k, FORMS[form], 541, alpha=1.5,
                                  beta=0.5, workspace_bytes=5 * 3004 * 2047 * 4)
     assert np.array_equal(mine[0].view(np.uint32), outs[0].view(np.uint32))

@@ -1,31 +1,29 @@
 """Split-K launches on the MI355X, through the C ABI, against the oracle.
 
-Launches that would leave workgroup slots idle split K (kernels::split_k_plan):
-each K range of each tile is one workgroup (of the ring kernels for interior
-256 x 256 tiles, else of the 256 x 128 kernel), writing raw partial sums into
-one frame of the pool, and a second kernel adds the partials in range order
-and applies alpha, beta and the epilogue.
+Launches that would leave CUs idle run on small tiles, whose K the waves of a
+workgroup share and which may split it over workgroups too (kernels::route):
+each K range of each tile is one workgroup, writing raw partial sums into one
+frame of the pool, and a second kernel adds the partials in range order and
+applies alpha, beta and the epilogue. Deep interior launches split on the ring
+kernels. Each test asserts its route.
 
-* The config-5 launch shape (4096 x 256 x 4096 under 64 MiB frames: 16 tiles,
-  16 ranges of 256, the partials filling the frame exactly), all four forms:
-  the analytic pattern, every element bit-exact.
-* A K tail (4096 x 256 x 4000: 16 ranges of 256, the last 160) with alpha,
-  beta and a per-column bias + ReLU, seeded U[-1,1) operands: every element
-  within the FP64 bound, and two executions bit-identical (the reduction
-  order is fixed).
+* The config-5 launch shape (4096 x 256 x 4096 under 64 MiB frames: 256 tiles of
+  64 x 64, unsplit), all four forms: the analytic pattern, every element
+  bit-exact.
+* The same with a K tail (4096 x 256 x 4000), alpha, beta and a per-column bias +
+  ReLU, seeded U[-1,1) operands: every element within the FP64 bound, and two
+  executions bit-identical.
 * A resident config-5 layer with the weights resident (16384 x 256 x 16384
-  T/N under 1 GiB frames: 64 tiles, 4 ranges of 4096): pattern bit-exact.
-* Config 1's shape (1024^3 N/N: its ring split would take 64-deep ranges, so
-  32 tiles of 256 x 128 in 8 ranges of 128): every element within the
+  T/N under 1 GiB frames: 64 tiles of 256 x 256 in 4 ranges of 4096 on the ring
+  kernels): pattern bit-exact.
+* Config 1's shape (1024^3 N/N: 256 tiles of 64 x 64): every element within the
   FP64 bound.
-* Launches that are not whole 256 x 256 tiles split on the 256 x 128 kernel:
-  501 x 200 x 2048 (2 x 2 tiles, 32 ranges; partials of leading dimension 504)
-  bit-exact on the pattern in all four forms; 501 x 200 x 1000 (eleven ranges,
-  a K tail) with alpha, beta and a per-row or per-column bias + ReLU within the
-  bound, two executions bit-identical; config 2's shape (3001 x 2047 x 4099)
-  in all four forms with alpha 1.5, beta 0.5 within the bound, under 64 MiB
-  frames (the partials' frame holds 2 ranges) and 128 MiB frames (5 ranges,
-  two rounds of the kernel's workgroup slots).
+* Small launches whose K splits: 501 x 200 x 2048 (tiles of 32 x 32 in 4 ranges;
+  partials of leading dimension 504) bit-exact on the pattern in all four forms;
+  501 x 200 x 1000 (a K tail) with alpha, beta and a per-row or per-column bias +
+  ReLU within the bound, two executions bit-identical; config 2's shape (3001 x
+  2047 x 4099, 64 x 64 tiles, unsplit) in all four forms with alpha 1.5, beta 0.5
+  within the bound, under 64 and 128 MiB frames.
 
 Tolerance: |C - C_ref| <= 4*K*2^-24*(|alpha||A||B| + |beta C0| + |bias|)_ij."""
 import ctypes
@@ -36,6 +34,8 @@ import pytest
 
 import xvram_amd as xv
 from xvram_amd import abi
+
+from gemm_cases import route
 
 pytestmark = pytest.mark.gpu
 
@@ -126,6 +126,7 @@ class Gemm:
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_split_c5_launch_pattern(lib, synth, oracle_mod, form):
     m, n, k = 4096, 256, 4096
+    assert route(m, n, k, form, 64 * MiB).startswith("small 64x64 ranges 1 ")
     s = xv.Session(lib, chunk_size_bytes=64 * MiB, cache_target_bytes=2 * GiB)
     try:
         g = Gemm(s, m, n, k, FORMS[form])
@@ -146,6 +147,7 @@ def test_split_c5_launch_pattern(lib, synth, oracle_mod, form):
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_split_k_tail_beta_epilogue_deterministic(lib, synth, oracle_mod, form):
     m, n, k = 4096, 256, 4000
+    assert route(m, n, k, form, 64 * MiB).startswith("small 64x64 ranges 1 ")
     alpha, beta = 1.5, 0.5
     bias = (oracle_mod.fill_uniform(n, 94) * 0.5).astype(np.float32)
     s = xv.Session(lib, chunk_size_bytes=64 * MiB, cache_target_bytes=2 * GiB)
@@ -177,6 +179,7 @@ def test_split_k_tail_beta_epilogue_deterministic(lib, synth, oracle_mod, form):
 
 def test_split_resident_c5_layer_pattern(lib, synth, oracle_mod):
     m, n, k = 16384, 256, 16384
+    assert route(m, n, k, "TN", GiB) == "ring split 4x4096"
     s = xv.Session(lib, chunk_size_bytes=GiB)
     try:
         g = Gemm(s, m, n, k, FORMS["TN"])
@@ -195,6 +198,7 @@ def test_split_resident_c5_layer_pattern(lib, synth, oracle_mod):
 
 def test_split_config1_shape(lib, synth, oracle_mod):
     m = n = k = 1024
+    assert route(m, n, k, "NN").startswith("small 64x64 ranges 1 ")
     s = xv.Session(lib)
     try:
         g = Gemm(s, m, n, k, FORMS["NN"])
@@ -212,6 +216,7 @@ def test_split_config1_shape(lib, synth, oracle_mod):
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_ragged_split_pattern(lib, synth, oracle_mod, form):
     m, n, k = 501, 200, 2048
+    assert route(m, n, k, form, 64 * MiB).startswith("small 32x32 ranges 4 ")
     s = xv.Session(lib, chunk_size_bytes=64 * MiB, cache_target_bytes=2 * GiB)
     try:
         g = Gemm(s, m, n, k, FORMS[form])
@@ -231,6 +236,7 @@ def test_ragged_split_pattern(lib, synth, oracle_mod, form):
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_ragged_split_k_tail_beta_epilogue(lib, synth, oracle_mod, form, axis):
     m, n, k = 501, 200, 1000
+    assert route(m, n, k, form, 64 * MiB).startswith("small 32x32 ranges 4 ")
     alpha, beta = 1.25, -0.5
     length = m if axis == abi.BIAS_PER_ROW else n
     bias = (oracle_mod.fill_uniform(length, 97) * 0.5).astype(np.float32)
@@ -266,10 +272,9 @@ def test_ragged_split_k_tail_beta_epilogue(lib, synth, oracle_mod, form, axis):
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_config2_shape_split(lib, synth, oracle_mod, form, frame_mib):
     """Config 2 (3001 x 2047 x 4099, alpha 1.5, beta 0.5) resident: one launch of
-    12 x 16 tiles of 256 x 128 that splits K into as many ranges as the
-    partials' frame holds up to the rule's 5: 2 under 64 MiB frames, 5 under
-    128 MiB."""
+    64 x 64 tiles, unsplit whatever the frames hold."""
     m, n, k = 3001, 2047, 4099
+    assert route(m, n, k, form, frame_mib * MiB).startswith("small 64x64 ranges 1 ")
     alpha, beta = 1.5, 0.5
     s = xv.Session(lib, chunk_size_bytes=frame_mib * MiB, cache_target_bytes=2 * GiB)
     try:

@@ -5,17 +5,19 @@ workgroup per CU; when its last round would fill few CUs, it runs instead as a
 head (whole tile rows, unsplit, in full rounds) and a tail (the remaining tile
 rows, K split on the ring kernels; kernels::tail_split_shape):
 
-* 4352 x 4096 x 1024 (17 x 16 tiles: a head of 16 rows, one round, and a tail
-  of one row of 16 tiles in 5 ranges of 224), all four forms, seeded U[-1,1)
-  operands with alpha, beta, a per-row bias (offset into the tail's rows) and
-  ReLU: every element within the FP64 bound, and two executions
+* 4864 x 4352 x 1000 (19 x 17 tiles: a head of 15 rows, one round, and a tail
+  of four rows of 17 tiles in 3 ranges of 352, the last 296), all four forms,
+  seeded U[-1,1) operands with alpha, beta, a per-row bias (offset into the
+  tail's rows) and ReLU: every element within the FP64 bound, and two executions
   bit-identical; with a workspace of the caller's exactly the size the tail
   wants: the same bits.
-* 4608 x 4608 x 2048 (18 x 18 tiles: a head of 14 rows, a tail of 4 rows in 7
-  ranges of 320, two rounds of the CUs, 126 MiB of partials) N/N and T/N: the
-  analytic pattern, every element bit-exact.
-* The 4352 x 4096 x 1024 launch in a session (resident, 256 MiB frames: the
-  partials in one frame of the pool), N/N and N/T: the pattern, bit-exact.
+* 5888 x 4608 x 2016 (23 x 18 tiles: a head of 14 rows, a tail of 9 rows in 3
+  ranges of 672, two rounds of the CUs) N/N and T/N: the analytic pattern, every
+  element bit-exact.
+* 5120 x 4352 x 1632 in a session (resident, 256 MiB frames: the partials in one
+  frame of the pool), N/N and N/T: the pattern, bit-exact.
+
+Each test asserts that its launch takes the tail split (kernels::route).
 
 Tolerance: |C - C_ref| <= 4*K*2^-24*(|alpha||A||B| + |beta C0| + |bias|)_ij."""
 import ctypes
@@ -27,6 +29,7 @@ import pytest
 import xvram_amd as xv
 from xvram_amd import abi
 
+from gemm_cases import route
 from test_gpu_sgemm_device import FORMS, Hip, desc_for, padded, run_device_gemm
 
 pytestmark = pytest.mark.gpu
@@ -71,7 +74,8 @@ def pattern_stored(synth, which, rows, cols, transposed):
 
 @pytest.mark.parametrize("form", sorted(FORMS))
 def test_tail_split_within_bound_and_deterministic(lib, hip, oracle_mod, form):
-    m, n, k = 4352, 4096, 1024
+    m, n, k = 4864, 4352, 1000
+    assert route(m, n, k, form) == "tail split 3840 3x352"
     outs, ref, absab = run_device_gemm(lib, hip, oracle_mod, m, n, k, FORMS[form], 701,
                                        alpha=-0.5, beta=0.75, bias_rows=True, relu=True,
                                        repeat=2)
@@ -80,16 +84,17 @@ def test_tail_split_within_bound_and_deterministic(lib, hip, oracle_mod, form):
     log(f"{m}x{n}x{k} {form} + bias/ReLU: violations {bad}, err/bound {ratio:.3e}")
     assert bad == 0
     if form == "NT":
-        # Five partials of the tail's 256 x 4096 floats in a workspace of the caller's.
+        # Three partials of the tail's 1024 x 4352 floats in a workspace of the caller's.
         mine, _, _ = run_device_gemm(lib, hip, oracle_mod, m, n, k, FORMS[form], 701,
                                      alpha=-0.5, beta=0.75, bias_rows=True, relu=True,
-                                     workspace_bytes=5 * 256 * 4096 * 4)
+                                     workspace_bytes=3 * 1024 * 4352 * 4)
         assert np.array_equal(mine[0].view(np.uint32), outs[0].view(np.uint32))
 
 
 @pytest.mark.parametrize("form", ["NN", "TN"])
 def test_two_round_tail_pattern(lib, hip, synth, oracle_mod, form):
-    m, n, k = 4608, 4608, 2048
+    m, n, k = 5888, 4608, 2016
+    assert route(m, n, k, form) == "tail split 3584 3x672"
     ops = FORMS[form]
     a_st = pattern_stored(synth, "a", *((m, k) if ops[0] == abi.OP_N else (k, m)),
                           ops[0] == abi.OP_T)
@@ -119,7 +124,8 @@ def test_two_round_tail_pattern(lib, hip, synth, oracle_mod, form):
 
 @pytest.mark.parametrize("form", ["NN", "NT"])
 def test_tail_split_in_a_session(lib, synth, oracle_mod, form):
-    m, n, k = 4352, 4096, 1024
+    m, n, k = 5120, 4352, 1632
+    assert route(m, n, k, form, 256 * MiB) == "tail split 3840 3x544"
     ops = FORMS[form]
     a_shape = (m, k) if ops[0] == abi.OP_N else (k, m)
     b_shape = (k, n) if ops[1] == abi.OP_N else (n, k)

@@ -1,11 +1,12 @@
 """GPU parity of the 256 x 256 tile kernel (sgemm_wide.hip).
 
-A launch with at least 256 such tiles (C of 4096 x 4096 or more) and operand
-panels under 2^31 bytes runs the wide kernel; these cases cover its four
+A launch of interior 256 x 256 tiles (C of 4096 x 4096 or more) whose K is no
+multiple of the ring kernels' step and which neither a K remainder nor small
+tiles would speed up runs the wide kernel, and so does a ragged one whose K
+remainder would want partials and has no workspace; these cases cover its four
 operation forms (direct-to-LDS and register-staged operands), interior and edge
-tiles, the K tail after its three-stage unrolled loop, alpha/beta, the fused
-bias/ReLU epilogue, and one out-of-core case whose 4096 x 4096 C tiles
-accumulate over several K panels.
+tiles, the K tail after its three-stage unrolled loop and alpha/beta. Every test
+asserts the route of its launches (kernels::route).
 
 N/T launches whose tiles are all interior (m, n multiples of 256) and whose K
 is a multiple of 4 run the barrier-free variant (sgemm_ring_kernel: each wave
@@ -15,16 +16,14 @@ out-of-core panels) run it, and the ring cases below add K tails around its
 8-pair unrolled loop and 7-pair prefetch distance, alpha/beta and the epilogue.
 Launches of the other forms with such tiles and K a multiple of 8 run
 sgemm_ring8_kernel (the same scheme with k-contiguous halves loaded straight
-into LDS in 8-deep slots): the NN, TN and TT interior and pattern cases above
-run it, and the ring8 cases add its slot tails, alpha/beta and the shapes
-that fall back to sgemm_wide_kernel.
+into LDS in 8-deep slots): the NN, TN and TT interior cases above run it, and
+the ring8 cases add its slot tails, alpha/beta and the shapes that fall back to
+sgemm_wide_kernel.
 
 Ragged launches whose K is a multiple of 4 (N/T) or 8 run whole on the ring
-kernels' edge instances (tests/test_gpu_edge_ring.py) or take an edge split
-(interior on the ring kernels, strips apart; tests/test_gpu_edge_split.py),
-and those whose K is not, with K rounded down at least 512, a K remainder; the
-ragged random case here has K = 501 and stays whole on sgemm_wide_kernel, and
-the ragged pattern cases of the ring tests below run the edge instances.
+kernels' edge instances (tests/test_gpu_edge_ring.py and the ragged pattern
+cases below), take an edge split or a rectangle and strips
+(tests/test_gpu_edge_split.py), or small tiles (tests/test_gpu_kwave.py).
 
 Random cases are checked element by element against the FP64 oracle on three
 column ranges (first, middle and last tile columns, every row) with the bound
@@ -37,13 +36,17 @@ import pytest
 import xvram_amd as xv
 from xvram_amd import abi
 
-from gemm_cases import Problem, logical_from_storage, pattern_operands, storage, uniform
+from gemm_cases import Problem, logical_from_storage, pattern_operands, route, storage, uniform
 
 pytestmark = pytest.mark.gpu
 
 MiB = 1 << 20
 OPS = [(abi.OP_N, abi.OP_N), (abi.OP_N, abi.OP_T), (abi.OP_T, abi.OP_N), (abi.OP_T, abi.OP_T)]
 OP_IDS = ["NN", "NT", "TN", "TT"]
+
+
+def form(ops):
+    return OP_IDS[OPS.index(tuple(ops))]
 
 
 @pytest.fixture(scope="module")
@@ -83,8 +86,10 @@ def sampled_check(oracle, prob, out, label):
 
 @pytest.mark.parametrize("ops", OPS, ids=OP_IDS)
 def test_wide_interior(resident, oracle_mod, ops):
-    """4096 x 4096 x 1040: 256 interior tiles, 65 K stages (unrolled loop + tail)."""
+    """4096 x 4096 x 1040: 256 interior tiles on the ring kernels, 65 K stages
+    (unrolled loop + tail)."""
     m, n, k = 4096, 4096, 1040
+    assert route(m, n, k, form(ops)) == "ring"
     prob = Problem(uniform(oracle_mod, m, k, 1101), uniform(oracle_mod, k, n, 1102),
                    op_a=ops[0], op_b=ops[1])
     out = prob.run(resident)
@@ -93,22 +98,39 @@ def test_wide_interior(resident, oracle_mod, ops):
 
 
 @pytest.mark.parametrize("ops", OPS, ids=OP_IDS)
-def test_wide_edges_alpha_beta(resident, oracle_mod, ops):
-    """4000 x 3950 x 501: edge tiles on both sides and a partial last K stage
-    (16 x 16 tiles: one round, no edge split; K rounded down to a multiple of 4
-    or 8 is below 512, so no K remainder: the launch stays whole on this
-    kernel)."""
-    m, n, k = 4000, 3950, 501
+def test_wide_edges_alpha_beta(lib, oracle_mod, ops):
+    """4134 x 4225 x 1835 under three frames, so without partials: edge tiles on
+    both sides and a partial last K stage, whole on this kernel."""
+    m, n, k = 4134, 4225, 1835
+    assert route(m, n, k, form(ops), None) == "general"
     prob = Problem(uniform(oracle_mod, m, k, 1201), uniform(oracle_mod, k, n, 1202),
                    uniform(oracle_mod, m, n, 1203), op_a=ops[0], op_b=ops[1],
                    alpha=-1.25, beta=0.75)
-    out = prob.run(resident)
+    with xv.Session(lib, chunk_size_bytes=128 * MiB, cache_target_bytes=3 * 128 * MiB,
+                    workspace_cap_bytes=0, device_headroom_bytes=0) as s:
+        out = prob.run(s)
+        assert prob.plan_info.tile_count == 1
     sampled_check(oracle_mod, prob, out, f"wide edges {ops}")
 
 
 @pytest.mark.parametrize("ops", OPS, ids=OP_IDS)
-def test_wide_pattern_bit_exact(resident, oracle_mod, ops):
+def test_wide_interior_alpha_beta(resident, oracle_mod, ops):
+    """4096 x 4096 x 1501: interior tiles and a partial last K stage."""
+    m, n, k = 4096, 4096, 1501
+    assert route(m, n, k, form(ops)) == "general"
+    prob = Problem(uniform(oracle_mod, m, k, 1211), uniform(oracle_mod, k, n, 1212),
+                   uniform(oracle_mod, m, n, 1213), op_a=ops[0], op_b=ops[1],
+                   alpha=1.5, beta=-0.5)
+    out = prob.run(resident)
+    sampled_check(oracle_mod, prob, out, f"wide K tail {ops}")
+
+
+@pytest.mark.parametrize("ops", OPS, ids=OP_IDS)
+def test_rectangle_pattern_bit_exact(resident, oracle_mod, ops):
+    """17 x 16 interior tiles: one round on the ring kernels, the last tile row on
+    small tiles."""
     m, n, k = 4352, 4096, 1104
+    assert route(m, n, k, form(ops)).startswith("rectangle[4096x4096x1104 ring; 256x4096x1104 small")
     a_op, b_op = pattern_operands(m, n, k)
     prob = Problem(a_op, b_op, op_a=ops[0], op_b=ops[1])
     out = prob.run(resident)
@@ -118,6 +140,7 @@ def test_wide_pattern_bit_exact(resident, oracle_mod, ops):
 
 def test_wide_beta_zero_over_nan(resident, oracle_mod):
     m, n, k = 4096, 4096, 528
+    assert route(m, n, k, "NT") == "ring"
     prob = Problem(uniform(oracle_mod, m, k, 1301), uniform(oracle_mod, k, n, 1302),
                    op_b=abi.OP_T)
     out = prob.run(resident, c_fill=np.float32(np.nan))
@@ -125,28 +148,31 @@ def test_wide_beta_zero_over_nan(resident, oracle_mod):
     sampled_check(oracle_mod, prob, out, "wide beta=0 over NaN C")
 
 
-@pytest.mark.parametrize("k", [4, 28, 32, 36, 60, 64, 1036])
+@pytest.mark.parametrize("k", [8, 28, 32, 36, 60, 64, 1036])
 def test_ring_k_tails_pattern(resident, oracle_mod, k):
     """Barrier-free N/T kernel, bit-exact pattern: fewer pairs than the
-    prefetch distance (k = 4, 28), exactly one unrolled block plus tail
+    prefetch distance (k = 8, 28), exactly one unrolled block plus tail
     (32 .. 64) and a long loop with a 3-pair tail (1036)."""
     m, n = 4096, 4096
     a_op, b_op = pattern_operands(m, n, k)
     prob = Problem(a_op, b_op, op_b=abi.OP_T)
     out = prob.run(resident)
     assert prob.plan_info.tile_count == 1
+    assert route(m, n, k, "NT") == "ring"
     expected = oracle_mod.pattern_expected_matrix(m, n, k)
     assert np.array_equal(out.astype(np.float64), expected)
 
 
-@pytest.mark.parametrize("m,n,k", [(4096, 4096, 1001), (4000, 4096, 1040), (4096, 4000, 1040)],
+@pytest.mark.parametrize("m,n,k,how", [(4096, 4096, 1501, "general"), (4000, 4096, 1040, "edge ring"),
+                                       (4096, 4000, 1040, "edge ring")],
                          ids=["k%4-wide", "m%256-edge", "n%256-edge"])
-def test_ring_fallback_shapes_pattern(resident, oracle_mod, m, n, k):
+def test_ring_fallback_shapes_pattern(resident, oracle_mod, m, n, k, how):
     """N/T launches just outside the interior barrier-free kernel's conditions:
     K not a multiple of 4 (one round of interior tiles, which neither a tail
-    split nor a K remainder would speed up: sgemm_wide_kernel), or m or n not a
-    multiple of 256 (one round of 16 x 16 tiles, which no edge split would
-    speed up: the ring kernel's edge instance). Bit-exact pattern."""
+    split, a K remainder nor small tiles would speed up: sgemm_wide_kernel), or m
+    or n not a multiple of 256 (one round of 16 x 16 tiles, which no edge split
+    would speed up: the ring kernel's edge instance). Bit-exact pattern."""
+    assert route(m, n, k, "NT") == how
     a_op, b_op = pattern_operands(m, n, k)
     prob = Problem(a_op, b_op, op_b=abi.OP_T)
     out = prob.run(resident)
@@ -167,6 +193,7 @@ def test_ring8_k_tails_pattern(resident, oracle_mod, ops, k):
     unrolled block (32), a block plus a tail (40, 56) and a long loop with a
     3-slot tail (1048)."""
     m, n = 4096, 4096
+    assert route(m, n, k, form(ops)) == "ring"
     a_op, b_op = pattern_operands(m, n, k)
     prob = Problem(a_op, b_op, op_a=ops[0], op_b=ops[1])
     out = prob.run(resident)
@@ -177,7 +204,8 @@ def test_ring8_k_tails_pattern(resident, oracle_mod, ops, k):
 
 @pytest.mark.parametrize("ops", KC_OPS, ids=KC_IDS)
 def test_ring8_alpha_beta(resident, oracle_mod, ops):
-    m, n, k = 4608, 4096, 1000
+    m, n, k = 4096, 4096, 1000
+    assert route(m, n, k, form(ops)) == "ring"
     prob = Problem(uniform(oracle_mod, m, k, 1701), uniform(oracle_mod, k, n, 1702),
                    uniform(oracle_mod, m, n, 1703), op_a=ops[0], op_b=ops[1], alpha=-1.25,
                    beta=0.75)
@@ -185,13 +213,14 @@ def test_ring8_alpha_beta(resident, oracle_mod, ops):
     sampled_check(oracle_mod, prob, out, f"ring8 alpha/beta {ops}")
 
 
-@pytest.mark.parametrize("ops,m,k", [(OPS[0], 4096, 1004), (OPS[2], 4000, 1040), (OPS[3], 4096, 1020)],
+@pytest.mark.parametrize("ops,m,k", [(OPS[0], 4096, 1404), (OPS[2], 4000, 1040), (OPS[3], 4096, 1420)],
                          ids=["NN-k%8-wide", "TN-m%256-edge", "TT-k%8-wide"])
 def test_ring8_fallback_shapes_pattern(resident, oracle_mod, ops, m, k):
     """Launches just outside that kernel's interior conditions in one round of
     16 x 16 tiles: K not a multiple of 8 (sgemm_wide_kernel) or m not a
     multiple of 256 (its edge instance). Bit-exact pattern."""
     n = 4096
+    assert route(m, n, k, form(ops)) == ("general" if m == 4096 else "edge ring")
     a_op, b_op = pattern_operands(m, n, k)
     prob = Problem(a_op, b_op, op_a=ops[0], op_b=ops[1])
     out = prob.run(resident)
@@ -200,17 +229,19 @@ def test_ring8_fallback_shapes_pattern(resident, oracle_mod, ops, m, k):
 
 
 def test_ring_alpha_beta(resident, oracle_mod):
-    m, n, k = 4608, 4096, 1000
+    m, n, k = 4096, 4096, 1000
+    assert route(m, n, k, "NT") == "ring"
     prob = Problem(uniform(oracle_mod, m, k, 1601), uniform(oracle_mod, k, n, 1602),
                    uniform(oracle_mod, m, n, 1603), op_b=abi.OP_T, alpha=-1.25, beta=0.75)
     out = prob.run(resident)
     sampled_check(oracle_mod, prob, out, "ring alpha/beta")
 
 
-@pytest.mark.parametrize("n", [4000, 4096], ids=["wide", "ring"])
+@pytest.mark.parametrize("n", [4000, 4096], ids=["edge", "ring"])
 @pytest.mark.parametrize("axis", [abi.BIAS_PER_ROW, abi.BIAS_PER_COLUMN], ids=["row", "col"])
 def test_wide_epilogue(lib, oracle_mod, axis, n):
     m, k = 4096, 800
+    assert route(m, n, k, "NT") == ("ring" if n == 4096 else "edge ring")
     a = uniform(oracle_mod, m, k, 1401)
     b = uniform(oracle_mod, k, n, 1402)
     c0 = uniform(oracle_mod, m, n, 1403)
@@ -281,5 +312,6 @@ def test_mixed_kernels_out_of_core_pattern(lib, oracle_mod):
         out = prob.run(s)
         info = prob.plan_info
     assert (info.tile_m, info.tile_n, info.tile_k) == (4096, 4096, 4096) and info.tile_count == 8
+    assert route(4096, 4096, 4096, "NT") == "ring" and route(4096, 4096, 1906, "NT") == "general"
     expected = oracle_mod.pattern_expected_matrix(m, n, k)
     assert np.array_equal(out.astype(np.float64), expected)

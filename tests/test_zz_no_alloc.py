@@ -15,6 +15,7 @@ import pytest
 import xvram_amd as xv
 from xvram_amd import abi
 
+from gemm_cases import route
 from test_gpu_sgemm_device import FORMS, Hip, desc_for, padded, stored
 
 pytestmark = pytest.mark.gpu
@@ -39,20 +40,19 @@ def test_no_alloc_matches_sgemm_device(lib, oracle_mod):
     hip = Hip()
     s = hip.stream()
     try:
-        # 16 tiles x 16 ranges on the ring kernels (64 MiB of partials), then
-        # 16 tiles of 256 x 128 x 16 ranges (32 MiB) over what the first call
-        # left there, then a ragged launch
-        # (2 x 2 tiles of 256 x 128, 32 ranges, partials of leading dimension
-        # 504), then config 2's shape (192 tiles of 256 x 128, 5 ranges: 117
-        # MiB of partials, most of the 128 MiB scratch), then a tail split
-        # (17 x 16 tiles: 16 rows unsplit, the last row in 5 ranges), then an
-        # edge split (4100 x 4100: the 16 x 16 interior and two split strips).
-        for call, (m, n, k, form, seed) in enumerate([(4096, 256, 4096, "NN", 601),
-                                                      (1024, 512, 2048, "NT", 602),
-                                                      (501, 200, 2048, "TN", 603),
-                                                      (3001, 2047, 4099, "NN", 604),
-                                                      (4352, 4096, 1024, "TT", 605),
-                                                      (4100, 4100, 1024, "NT", 606)]):
+        # A launch that wants none, then 128 tiles of 64 x 64 in 4 ranges (8 MiB of
+        # partials), a ragged launch over what that call left there (32 x 32
+        # tiles in 4 ranges, partials of leading dimension 504), a ring split (4
+        # ranges, 32 MiB), a tail split (9 of 23 tile rows in 3 ranges: 121 MiB, most
+        # of the 128 MiB scratch) and a rectangle with a strip that splits.
+        for call, (m, n, k, form, seed, how) in enumerate([
+                (4096, 256, 4096, "NN", 601, "small 64x64 ranges 1 "),
+                (1024, 512, 8192, "NT", 602, "small 64x64 ranges 4 "),
+                (501, 200, 2048, "TN", 603, "small 32x32 ranges 4 "),
+                (8192, 512, 16384, "NN", 604, "ring split 4x4096"),
+                (5888, 4608, 2016, "TT", 605, "tail split 3584 3x672"),
+                (4100, 4100, 1024, "NT", 606, "rectangle[4096x4096x1024 ring; 4096x4x1024 small 32x32 ranges 4 ")]):
+            assert route(m, n, k, form).startswith(how)
             ops = FORMS[form]
             a_op = np.asfortranarray(oracle_mod.fill_uniform(m * k, seed).reshape(k, m).T)
             b_op = np.asfortranarray(oracle_mod.fill_uniform(k * n, seed + 1).reshape(n, k).T)
