@@ -341,7 +341,7 @@ Error device_gemm_failure(int rc, const char* entry) {
                       "this build has no GPU (host simulation)");
   if (rc == kScratchTooSmall)
     return make_error(XVRAM_STATUS_INVALID_ARGUMENT, kStage, entry,
-                      "the split's partials exceed the 64 MiB static scratch; pass a workspace");
+                      "the split's partials exceed the 128 MiB static scratch; pass a workspace");
   Error e = make_error(rc == 2 /* hipErrorOutOfMemory */ ? XVRAM_STATUS_DEVICE_OUT_OF_MEMORY
                                                           : XVRAM_STATUS_CUDA_ERROR,
                        kStage, entry, "the HIP runtime refused the launch or its workspace");

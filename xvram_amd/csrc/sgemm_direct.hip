@@ -3,6 +3,7 @@
 // split-K workspace is settled and the launch enqueued on the caller's stream.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <mutex>
 #include <vector>
@@ -18,13 +19,15 @@ namespace {
 // GPU in this file's code object, held until the process ends and shared by
 // every call on that GPU (calls that overlap on one GPU race on it). A split
 // never wants more: at most one 256 x 256 partial tile per CU (ring kernels;
-// two per CU for a tail split) or one 256 x 128 tile per workgroup of two
-// rounds of two per CU (the 256 x 128 kernel). Every partial element the reduction uses is written before it
-// is read (the padding rows of a ragged partial are read but not used), so
-// nothing in the array needs clearing between calls.
+// two per CU for a tail split), one 256 x 128 tile per workgroup of two rounds
+// of two per CU (the 256 x 128 kernel) or kKwaveMaxPartialBytes (small tiles).
+// Every partial element the reduction uses is written before it is read (the
+// padding rows of a ragged partial are read but not used), so nothing in the
+// array needs clearing between calls.
 constexpr uint64_t kScratchBytes = 128ull << 20;
 static_assert(kScratchBytes >= uint64_t(2 * kernels::kComputeUnits) * 256 * 256 * 4 &&
-                  kScratchBytes >= kernels::kSplitMaxPartialBytes,
+                  kScratchBytes >= kernels::kSplitMaxPartialBytes &&
+                  kScratchBytes >= kernels::kKwaveMaxPartialBytes,
               "the scratch holds the largest split");
 static __device__ __align__(256) float scratch[kScratchBytes / 4];
 
@@ -32,6 +35,10 @@ static __device__ __align__(256) float scratch[kScratchBytes / 4];
 // GPU current (in host code the array's name is only a stand-in).
 std::mutex g_scratch_mutex;
 std::vector<void*> g_scratch_address;
+int g_scratch_known = 0; // GPUs whose address is in g_scratch_address
+// It is known on every GPU of the process: a call that needs no scratch then
+// neither asks for its stream's GPU nor takes the lock.
+std::atomic<bool> g_scratch_everywhere{false};
 
 int scratch_address(hipStream_t stream, void** out) {
   int device = -1;
@@ -52,6 +59,9 @@ int scratch_address(hipStream_t stream, void** out) {
       return static_cast<int>(e);
     }
     g_scratch_address[device] = p;
+    int count = 0;
+    if (hipGetDeviceCount(&count) == hipSuccess && ++g_scratch_known == count)
+      g_scratch_everywhere.store(true, std::memory_order_relaxed);
   }
   *out = g_scratch_address[device];
   return 0;
@@ -63,6 +73,8 @@ int direct_sgemm_no_alloc(const kernels::SgemmLaunch& launch, void* stream) {
   kernels::SgemmLaunch l = launch;
   l.padded = true;
   const uint64_t wanted = kernels::launch_bytes_wanted(l);
+  if (wanted == 0 && g_scratch_everywhere.load(std::memory_order_relaxed))
+    return kernels::launch_sgemm(l, stream);
   // Looked up on the first call on a GPU whether or not it splits: the array
   // becomes resident with its code object then, and no later call takes memory.
   void* p = nullptr;
