@@ -62,7 +62,7 @@ constexpr int kThreads = 256;
 constexpr int kWaves = 4;
 
 // k values of one wave between folds, of tiles inside rows [0, rows) x columns
-// [0, cols) and of the others (a tile cut by m or n among them).
+// [0, cols) and of the others.
 struct Folds {
   int inside, edge, rows, cols;
 };
@@ -113,7 +113,9 @@ __device__ __forceinline__ int piece_place(int lrow, int g) {
 }
 
 // Tile 32*MB x 32*NB; slots of 8*KP k values, R of them in each wave's ring;
-// kPerCu workgroups share a CU (their LDS and registers fit).
+// kPerCu workgroups share a CU (their LDS and registers fit); kRegions: tiles past
+// folds.rows or folds.cols fold at another depth (instances of their own: the
+// choice costs the others 1 to 2 %, 500 x 500 x 60000 T/N 227.4 -> 231.6 us).
 //
 // A slot's halves in its ring place: an extent-contiguous half (op-N A, op-T
 // B) row-major 8*KP x extent as loaded, a k-contiguous one as piece_place says.
@@ -123,7 +125,7 @@ __device__ __forceinline__ int piece_place(int lrow, int g) {
 // half it issues the next kGroup loads of the slot R ahead, into the ring place
 // of the slot whose last fragments are in registers, and in its middle it reads
 // the next step's fragments (after waiting for their slot when it is a new one).
-template <bool kAKC, bool kBKC, int MB, int NB, int KP, int R, int kPerCu, bool kFold>
+template <bool kAKC, bool kBKC, int MB, int NB, int KP, int R, int kPerCu, bool kFold, bool kRegions>
 __global__ __launch_bounds__(kThreads, kPerCu) void sgemm_kwave_kernel(Params p, Folds folds) {
   constexpr int TM = 32 * MB, TN = 32 * NB;
   constexpr int kGroup = MB + NB;         // wave loads of 1 KiB per 8 k values
@@ -351,7 +353,8 @@ __global__ __launch_bounds__(kThreads, kPerCu) void sgemm_kwave_kernel(Params p,
       }
     };
     // Slots per run: a multiple of kUnroll.
-    const int run = (m0 + TM <= folds.rows && n0 + TN <= folds.cols ? folds.inside : folds.edge) / kSlotK;
+    const bool inside = !kRegions || (m0 + TM <= folds.rows && n0 + TN <= folds.cols);
+    const int run = (inside ? folds.inside : folds.edge) / kSlotK;
     int from = 0;                  // first slot of the current run
     if constexpr (kFold) {
       for (int to = run - kUnroll; ; to += run) {
@@ -447,22 +450,28 @@ template <bool AK, bool BK>
 hipError_t launch_form(const Params& p, int tile, const Folds& folds, hipStream_t s, hipEvent_t e0,
                        hipEvent_t e1) {
   const dim3 grid(static_cast<unsigned>(p.tiles_m * p.tiles_n * p.splits)), block(kThreads);
+  const bool regions = folds.edge != folds.inside;
   const auto go = [&](auto kernel) {
     hipExtLaunchKernelGGL(kernel, grid, block, 0, s, e0, e1, 0, p, folds);
     return hipGetLastError();
   };
   // kKwaveTiles (sgemm_launch.hpp) in its order.
   switch (tile) {
-  case 0: return go(sgemm_kwave_kernel<AK, BK, 1, 1, 2, 2, 4, true>);
-  case 1: return go(sgemm_kwave_kernel<AK, BK, 2, 1, 2, 2, 3, true>);
-  case 2: return go(sgemm_kwave_kernel<AK, BK, 2, 2, 2, 2, 2, true>);
-  case 3: return go(sgemm_kwave_kernel<AK, BK, 4, 1, 2, 2, 2, true>);
-  case 4: return go(sgemm_kwave_kernel<AK, BK, 1, 1, 4, 4, 1, true>);
+  case 0: return regions ? go(sgemm_kwave_kernel<AK, BK, 1, 1, 2, 2, 4, true, true>)
+                         : go(sgemm_kwave_kernel<AK, BK, 1, 1, 2, 2, 4, true, false>);
+  case 1: return regions ? go(sgemm_kwave_kernel<AK, BK, 2, 1, 2, 2, 3, true, true>)
+                         : go(sgemm_kwave_kernel<AK, BK, 2, 1, 2, 2, 3, true, false>);
+  case 2: return regions ? go(sgemm_kwave_kernel<AK, BK, 2, 2, 2, 2, 2, true, true>)
+                         : go(sgemm_kwave_kernel<AK, BK, 2, 2, 2, 2, 2, true, false>);
+  case 3: return regions ? go(sgemm_kwave_kernel<AK, BK, 4, 1, 2, 2, 2, true, true>)
+                         : go(sgemm_kwave_kernel<AK, BK, 4, 1, 2, 2, 2, true, false>);
+  case 4: return regions ? go(sgemm_kwave_kernel<AK, BK, 1, 1, 4, 4, 1, true, true>)
+                         : go(sgemm_kwave_kernel<AK, BK, 1, 1, 4, 4, 1, true, false>);
   case 5:
-    if constexpr (!AK && !BK) return go(sgemm_kwave_kernel<AK, BK, 4, 2, 1, 3, 2, false>);
+    if constexpr (!AK && !BK) return go(sgemm_kwave_kernel<AK, BK, 4, 2, 1, 3, 2, false, false>);
     break;
   case 6:
-    if constexpr (!AK && !BK) return go(sgemm_kwave_kernel<AK, BK, 2, 2, 1, 2, 4, false>);
+    if constexpr (!AK && !BK) return go(sgemm_kwave_kernel<AK, BK, 2, 2, 1, 2, 4, false, false>);
   }
   return hipErrorInvalidValue;
 }
@@ -481,7 +490,6 @@ hipError_t launch_kwave(const Params& p0, const KwavePlan& plan, bool a_kcontig,
   p.tiles_n = (p.n + 32 * t.nb - 1) / (32 * t.nb);
   p.splits = plan.splits;
   p.split_depth = plan.depth;
-  // Where all fold alike, tiles cut by m or n do too.
   const Folds folds{plan.fold, plan.edge_fold, static_cast<int>(plan.rows), static_cast<int>(plan.cols)};
   hipEvent_t last = p.splits > 1 ? nullptr : stop;
   hipError_t e;
