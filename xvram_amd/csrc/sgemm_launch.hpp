@@ -570,11 +570,12 @@ inline int64_t k_remainder_shape(int64_t m, int64_t n, int64_t k, bool nt) {
 // split's partials at 1.2 us per million elements and 8, strips at what
 // kwave_fastest says, a K remainder at 2.3 us per million elements of C and 4;
 // the small tiles at 7 % over kwave_fastest's time from K = 1500 on (their
-// operands no longer stay in the L2), proportionally less below. On 48 shapes
-// from 4096^2 x 256 to 6499^3 the choice was within 0.4 % of the better of the
-// two on average (6 % at worst): 3712 x 4590 x 503 N/T 313 -> 140 us, 5994 x
-// 3000 x 146 N/T 125 -> 62, 6379 x 2968 x 32 N/T 67 -> 34, 1504 x 15840 x 1728
-// N/T 785 -> 607, 5280^3 N/N 2344 -> 2127.
+// operands no longer stay in the L2), proportionally less below. 3712 x 4590 x 503
+// N/T 313 -> 139 us, 5994 x 3000 x 146 N/T 123 -> 61, 6379 x 2968 x 32 N/T 67 -> 34,
+// 1504 x 15840 x 1728 N/T 782 -> 601, 5280^3 N/N 2331 -> 2095. Over 128 launches of
+// 51 shapes, each timed on every plan, what this and the next rule choose is 5.4 %
+// faster than the rules above and 1.5 % slower than the fastest (whose chains no
+// rule bounds; 64 % at worst, 6379 x 2968 x 32 N/N, 69 us).
 inline double ring_time(int64_t tiles, int64_t k) {
   return double(cu_rounds(tiles)) * (0.2155 * double(k) + 14.0);
 }
@@ -616,18 +617,18 @@ inline double ring_rules_time(int64_t m, int64_t n, int64_t k, bool nt) {
 // interior 256 x 256 tiles that fills whole rounds of the CUs best, on the ring
 // kernels, and the rest of C, a right and a bottom strip, on small tiles: no
 // round is mostly empty, no tile is padded to 256 and nothing is split and
-// reduced. 5000^3 T/T, 16 x 16 tiles and strips 904 wide: 1867 -> 1770 us; 4500^3
-// N/N 1380 -> 1307, 4576^3 N/T 1406 -> 1317, 11378 x 2374 x 7040 T/T 2870 -> 2705.
-// Modelled like the rest, the strips at 131 TFLOP/s and 8 us each, for K from
-// 1024 on, and taken where that is 3 % faster than the rules above and than
-// small tiles alone (53 shapes: none more than 1.1 % slower than before). Its tiles
-// run unsplit on the ring kernels, as modelled, also where the chains (below)
+// reduced. 5000^3 T/T, 16 x 16 tiles in two passes and strips 904 wide: 1832 -> 1794
+// us; 4352 x 4096 x 1024 N/N 302 -> 258, 4500^3 N/N 1354 -> 1325, 11378 x 2374 x 7040
+// T/T 2837 -> 2687. Modelled like the rest, the strips at 131 TFLOP/s and 8 us each,
+// for K from 1024 on, and taken where that is 3 % faster than the rules above and
+// than small tiles alone (4576^3, level by the clock, loses 1 %). Its tiles run
+// unsplit on the ring kernels, as modelled, also where the chains (below)
 // leave it a few less than a round. Where the best rectangle of all is one round
 // of 244 to 255 tiles, so that the rules above leave most of a round idle too,
 // the small tiles are taken up to 7 % above those rules' modelled time (none of
 // 1086 such launches models above; their chains are at most 1024 instead of K):
-// 5586 x 3566 x 3344 N/T 954 us (those rules 986, the rectangle with its 252 tiles
-// on small ones 967), 1792 x 11520 x 4496 N/T 1315 (1442, 1335).
+// 1792 x 11520 x 4496 N/T 1309 us (those rules 1439, the rectangle with its 252 tiles
+// on small ones 1335), 5586 x 3566 x 3344 N/N 1003 (986, 994).
 struct ManyPlan {
   KwavePlan small;        // on small tiles (tile >= 0), or
   int64_t mi = 0, ni = 0; // the rectangle's rows and columns; neither: the rules above
