@@ -2,7 +2,7 @@
 
 A launch of at least 256 tiles of 256 x 256 whose m or n is not a multiple of
 256 may run as its interior tiles (ring kernels, or their tail split) and two
-edge strips, each a launch of its own (kernels::edge_parts):
+edge strips, each a launch of its own (kernels::edge_parts_shape):
 
 * 4251 x 4188 x 432 (the 16 x 16 interior on the ring kernels, a 4096 x 92 right
   strip and a 155 x 4188 bottom strip on small tiles), all four forms, seeded

@@ -26,6 +26,8 @@ def fns():
     dll.xvram_hostsim_split_shape.argtypes = [i64] * 3 + [ctypes.c_int] * 2 + [ctypes.c_uint64, pint, pint]
     dll.xvram_hostsim_launch_bytes_wanted.argtypes = [ctypes.c_int] * 5 + [i64] * 2
     dll.xvram_hostsim_launch_bytes_wanted.restype = ctypes.c_uint64
+    dll.xvram_hostsim_k_remainder_shape.argtypes = [i64] * 3 + [ctypes.c_int]
+    dll.xvram_hostsim_k_remainder_shape.restype = i64
     return dll
 
 
@@ -168,6 +170,34 @@ def test_no_chain_is_longer_than_the_large_kernels_make_it():
     assert route(5000, 5000, 2048, "NN").startswith("rectangle[4096x4096x1024 ring; 4096x4096x1024 ring;")
     # Rows that lie in a tail of 320-deep ranges.
     assert fn(2304, 8512, 2080, 0, 0, 2304, 2080, 1800, 0, 0) <= 320
+
+
+def test_odd_k_runs_on_the_kernel_rated_faster():
+    """Interior launches of an odd K: without a K remainder they run on the general
+    kernel or on small tiles, whichever models faster (up to K = 1200 the small
+    tiles up to 4 % behind), and never on neither because a rectangle that no K
+    remainder will run modelled faster still."""
+    dll = fns()
+    dll.xvram_hostsim_odd_k_times.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int] + \
+        [ctypes.POINTER(ctypes.c_double)] * 2
+    small, general = ctypes.c_double(), ctypes.c_double()
+    rng = np.random.default_rng(59)
+    seen = {"general": 0, "small": 0, "k remainder": 0}
+    for _ in range(1500):
+        m, n = (256 * int(2 ** v) for v in rng.uniform(3, 6.2, 2))
+        k, form = int(rng.integers(520, 12000)) | 1, ("NN", "NT")[int(rng.integers(0, 2))]
+        if m // 256 * (n // 256) < 256:
+            continue
+        how = route(m, n, k, form)
+        kind = next(r for r in seen if how.startswith(r))
+        seen[kind] += 1
+        dll.xvram_hostsim_odd_k_times(m, n, k, form == "NT", ctypes.byref(small), ctypes.byref(general))
+        limit = 1.04 if k < 1200 else 1.0
+        if kind == "general":
+            assert small.value >= limit * general.value, (m, n, k, form)
+        elif dll.xvram_hostsim_k_remainder_shape(m, n, k, form == "NT") == 0:
+            assert small.value < limit * general.value, (m, n, k, form)
+    assert min(seen.values()) > 20, seen
 
 
 def test_rule_is_quick_for_many_tiles():

@@ -627,6 +627,14 @@ extern "C" __attribute__((visibility("default"))) int xvram_hostsim_kwave_many(
   return p.small.tile;
 }
 
+// The model's times (us) of a launch of many interior tiles on small ones and on
+// the general kernel (kernels::small_time, general_time).
+extern "C" __attribute__((visibility("default"))) void xvram_hostsim_odd_k_times(
+    int64_t m, int64_t n, int64_t k, int nt, double* small, double* general) {
+  *small = xvram::kernels::small_time(m, n, k, nt != 0);
+  *general = xvram::kernels::general_time(m / 256 * (n / 256), k, nt != 0);
+}
+
 // Launches and parts of launches whose route had that number in kernels::Run
 // since the last reset.
 extern "C" __attribute__((visibility("default"))) uint64_t xvram_hostsim_runs(int run) {

@@ -587,6 +587,13 @@ inline double general_time(int64_t tiles, int64_t k, bool nt) {
   return double(cu_rounds(tiles)) * ((nt ? 0.2195 : 0.2241) * double(k) + 28.0);
 }
 
+// The same of many tiles on small ones.
+inline double small_time(int64_t m, int64_t n, int64_t k, bool nt) {
+  double time = 0;
+  kwave_fastest(m, n, k, nt, 0, &time);
+  return time * (1.0 + 0.07 * std::min(1.0, double(k) / 1500.0));
+}
+
 // The model's time of an interior launch with its tail split.
 inline double interior_time(int64_t m, int64_t n, int64_t k) {
   const TailSplit ts = (m / 256) * (n / 256) >= kComputeUnits
@@ -689,10 +696,8 @@ inline ManyPlan many_shape(int64_t m, int64_t n, int64_t k, bool nt, const Chain
   const Chains chains = general ? Chains{m, k, k} : ring_rules_chains(m, n, k1, nt);
   const ChainBound rules{chains.tail, chains.shortest, m / 256 * 256, n / 256 * 256};
   // Rated as if no chain were bounded: the folds cost little (kwave_fastest).
-  double small = 0;
-  kwave_fastest(m, n, k, nt, 0, &small);
+  const double small = small_time(m, n, k, nt);
   const KwavePlan kw = kwave_fastest(m, n, k, nt, 0, nullptr, rules);
-  small *= 1.0 + 0.07 * std::min(1.0, double(k) / 1500.0);
   const double rest = k1 == k ? 0.0 : 2.3e-6 * double(m) * double(n) + 4.0;
   const double ring =
       general ? general_time(m / 256 * (n / 256), k, nt) : ring_rules_time(m, n, k1, nt) + rest;
