@@ -628,7 +628,7 @@ inline double ring_rules_time(int64_t m, int64_t n, int64_t k, bool nt) {
 // us; 4352 x 4096 x 1024 N/N 302 -> 258, 4500^3 N/N 1354 -> 1325, 11378 x 2374 x 7040
 // T/T 2837 -> 2687. Modelled like the rest, the strips at 131 TFLOP/s and 8 us each,
 // for K from 1024 on, and taken where that is 3 % faster than the rules above and
-// than small tiles alone (4576^3, level by the clock, loses 1 %). Its tiles run
+// than small tiles alone (4576^3, so rated, runs 1 % slower). Its tiles run
 // unsplit on the ring kernels, as modelled, also where the chains (below)
 // leave it a few less than a round. Where the best rectangle of all is one round
 // of 244 to 255 tiles, so that the rules above leave most of a round idle too,
